@@ -1,0 +1,416 @@
+// cell_step: one time step of a grid in one launch, one cell per lane and no
+// z-march, for grids whose state fits the 256 MB Infinity Cache (or nearly).
+// A tiled launch (fused_step) of such a grid is bound by the latency of its
+// blocks' marches, not by bytes: at 64^3 it runs 256 blocks for 16 us.
+//
+// A lane computes its cell's H^{n+1/2}, D^{n+1} (with the source) and
+// E^{n+1} from loads that depend on nothing but the cell's index: the six
+// halo H values that curl H needs (at i-1, j-1, k-1) are recomputed from
+// H^{n-1/2} and E^n, operation for operation as fused_tile does, so the two
+// kernels give identical results.  All loads of a wave go out together;
+// there is no LDS and no barrier.  Loads and stores are cached ones: the next
+// step reads what this one wrote, and streaming stores would send it to HBM
+// (128^3 fp32: 45 us with them, 32 us without).
+//
+// The first-order Mur faces and the probe row are part of the same launch:
+//   * a face cell's new E needs E^{n+1} of its inward neighbour, E^n of both
+//     and nothing else, all of which the lane of that neighbour holds.  So
+//     the lanes at i = 1, i = nx-2, j = 1, ... store the face cells beside
+//     them, and a face cell's own lane does not store the components that a
+//     face segment covers (the segments are disjoint per component, and no
+//     segment writes a cell that another one reads at n+1);
+//   * a probe is one wave that evaluates the cell again (for an E cell on a
+//     face: its neighbour) and, instead of storing, writes the value asked
+//     for, so it waits for no other wave.
+//
+// Measured on MI355X, whole steps, against fused_step and the Mur launch
+// (us): fp32 24^3 5.7 (15.1), 64^3 7.4 (16.6), 100^3 20.6 (31.2), 128^3 31
+// (47), 160x160x100 35 (60); fp16 64^3 6.7 (18.0), 96x121x77 13.0 (27.6),
+// 151x138x188 45 (78).  The kernel itself takes 27.4 us at 128^3 (5.3 TB/s at
+// the L2's far side, where a stream of the same arrays reaches 8.0): it is
+// held by instruction issue and resident waves (7 of 8 a SIMD), with 55
+// memory instructions and 216 vector ones a wave.
+#include <hip/hip_ext.h>
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "fdtd_device.h"
+#include "fdtd_internal.h"
+
+namespace {
+
+constexpr int kCellBlock = 256;
+
+// The Mur segment (numbered as in mur_segments) that writes E component c at
+// (i, j, k), and the step towards the cell whose lane evaluates it; -1: none.
+__device__ __forceinline__ int face_of(int c, int i, int j, int k, int nx, int ny, int nz, int &di, int &dj, int &dk)
+{
+    const bool ii = i >= 1 && i < nx - 1, ji = j >= 1 && j < ny - 1, ki = k >= 1 && k < nz - 1;
+    const bool il = i < nx - 1, jl = j < ny - 1, kl = k < nz - 1;
+    di = dj = dk = 0;
+    const int ex = i == 0 ? 0 : (i == nx - 1 ? 1 : -1), ey = j == 0 ? 0 : (j == ny - 1 ? 1 : -1),
+              ez = k == 0 ? 0 : (k == nz - 1 ? 1 : -1);
+    if (c == 0 && il) {
+        if (ey >= 0 && ki) { dj = 1 - 2 * ey; return ey; }
+        if (ez >= 0 && ji) { dk = 1 - 2 * ez; return 2 + ez; }
+    } else if (c == 1 && jl) {
+        if (ex >= 0 && ki) { di = 1 - 2 * ex; return 4 + ex; }
+        if (ez >= 0 && ii) { dk = 1 - 2 * ez; return 6 + ez; }
+    } else if (c == 2 && kl) {
+        if (ex >= 0 && ji) { di = 1 - 2 * ex; return 8 + ex; }
+        if (ey >= 0 && ii) { dj = 1 - 2 * ey; return 10 + ey; }
+    }
+    return -1;
+}
+
+// One load per value, never merged with its neighbours' (a wavefront-scope
+// relaxed load is an ordinary cached load that the compiler does not widen):
+// a dword, byte or short load of a wave takes 4.8 cycles of the CU's address
+// unit, an 8- or 12-byte one 16.5, so two or three dword loads are cheaper.
+template <typename T>
+__device__ __forceinline__ float at(const char *p, uint32_t b, int d = 0)
+{
+    if constexpr (sizeof(T) == 4)
+        return __hip_atomic_load((const float *)(p + b) + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    else
+        return Elem<T>::cvt(__hip_atomic_load((const unsigned short *)(p + b) + d, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WAVEFRONT));
+}
+
+// A Mur face's new value q * x as storage type T holds it.  The compiler
+// rounds the Mur kernel's fp16 product once, to fp16 (v_fma_mixlo_f16), and
+// the x faces that the tiled step updates twice, by way of fp32; `once` says
+// which of the two the tiled step gives this face.
+template <typename T>
+__device__ __forceinline__ float mur_round(float q, float x, bool once)
+{
+    float v = q * x;
+    if constexpr (std::is_same<T, __half>::value) {
+        if (once) {
+            uint32_t r = 0;
+            asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "+v"(r) : "v"(q), "v"(x));
+            return Elem<T>::cvt((unsigned short)r);
+        }
+        asm("" : "+v"(v));
+    }
+    return Elem<T>::rnd(v);
+}
+
+// What a lane loads: the cell's operands and its neighbours'.  Suffixes: im,
+// ip at i-1, i+1 and so on; no suffix: the cell.
+struct Ops {
+    float ex, ey, ez, ex_im, ey_im, ez_im, ey_ip, ez_ip, ex_jp, ez_jp, ex_jp_im, ex_jm, ey_jm, ez_jm, ey_jm_ip;
+    float ex_kp, ey_kp, ex_kp_im, ey_kp_jm, ex_km, ey_km, ez_km, ez_km_ip, ez_km_jp;
+    float hx, hy, hz, hy_im, hz_im, hx_jm, hz_jm, hx_km, hy_km;
+    float dx, dy, dz;                        // D^n
+    float exm, eym, ezm, dxm, dym, dzm;      // E^{n-1}, D^{n-1}
+    float a, c, d, k1, k2, k3, k5;
+    double g1, g2, g3;
+    bool src;
+};
+
+// BXL: log2 of the lanes of a block along x (32 or 64); the other lanes are
+// rows.  Exact form: cells whose material has a = g3 = +0 (C.zmask) do not
+// load E^{n-1} and D^{n-1}, as fused_tile's zero-term rows, decided per lane;
+// a context that always loads them passes zmask = 0 to the same kernel.
+template <typename T, bool EXACT, int BXL>
+__global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
+{
+    using X = Elem<T>;
+    constexpr uint32_t ES = sizeof(T);
+    constexpr int BX = 1 << BXL, BY = kCellBlock / BX, WY = 64 / BX;
+    const int nx = C.nx, ny = C.ny, nz = C.nz;
+
+    // Blocks (x, k) of plane k in 8 runs of C.run tiles, one run per XCD
+    // (workgroups go to the XCDs round-robin by id and gridDim.x is a
+    // multiple of 8), so a tile's neighbours in the plane and the same tiles
+    // of the planes around it share its L2.  Rows past nz hold the probes.
+    int i, j, k;
+    bool own = true, deep = false, edge = false;
+    int probe = -1, pf = -1, pseg = -1;      // probe: its index, field and face segment
+    const int bz = (int)blockIdx.y;
+    if (bz < nz) {
+        const int t = ((int)blockIdx.x & 7) * C.run + ((int)blockIdx.x >> 3);
+        if (t >= C.tiles) return;
+        const int ty = C.tiles_x == 1 ? t : (int)__umulhi((unsigned)t, C.tx_mul), tx = t - ty * C.tiles_x;
+        const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = (int)threadIdx.x & 63;
+        const int jw = ty * BY + w * WY;     // the wave's first row
+        if (jw >= ny) return;
+        i = tx * BX + (l & (BX - 1));
+        j = BX >= 64 ? jw : jw + (l >> BXL);
+        k = bz;
+        own = i < nx && j < ny;
+        j = min(j, ny - 1);
+        deep = jw >= 2 && jw + WY <= ny - 2 && k >= 2 && k < nz - 2 && nx > 3;
+        edge = tx == 0 || (nx - 2 >= tx * BX && nx - 2 < tx * BX + BX);
+    } else {
+        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * (int)gridDim.x + (int)blockIdx.x) * (kCellBlock / 64) +
+                                               ((int)threadIdx.x >> 6));
+        if (probe >= C.p.nprobe) return;
+        const int *q = C.p.probes + 4 * probe;
+        pf = q[0]; i = q[1]; j = q[2]; k = q[3];
+        if (pf >= 6) {
+            int di, dj, dk;
+            pseg = face_of(pf - 6, i, j, k, nx, ny, nz, di, dj, dk);
+            i += di; j += dj; k += dk;
+        }
+    }
+
+    // deep: the wave's rows and plane are at least two cells inside the y and z faces, so that of the faces only
+    // those along x are near (edge: its tile holds i = 1 or nx-2)
+    // Byte offset of the cell from bases that lie `guard` elements before the arrays' origins.
+    const uint32_t syb = C.sy, szb = C.sz;
+    const uint32_t o = C.o0 + (uint32_t)k * szb + (uint32_t)j * syb + (uint32_t)i * ES;
+    const uint32_t ojp = o + syb, ojm = o - syb, okp = o + szb, okm = o - szb;
+    const uint32_t id = C.ids[o / ES];
+    Ops v;
+    const char *px = C.e0[0], *py = C.e0[1], *pz = C.e0[2], *qx = C.h0[0], *qy = C.h0[1], *qz = C.h0[2];
+    v.ex = at<T>(px, o); v.ey = at<T>(py, o); v.ez = at<T>(pz, o);
+    v.ex_im = at<T>(px, o, -1); v.ey_im = at<T>(py, o, -1); v.ez_im = at<T>(pz, o, -1);
+    v.ey_ip = at<T>(py, o, 1); v.ez_ip = at<T>(pz, o, 1);
+    v.ex_jp = at<T>(px, ojp); v.ez_jp = at<T>(pz, ojp); v.ex_jp_im = at<T>(px, ojp, -1);
+    v.ex_jm = at<T>(px, ojm); v.ey_jm = at<T>(py, ojm); v.ez_jm = at<T>(pz, ojm); v.ey_jm_ip = at<T>(py, ojm, 1);
+    v.ex_kp = at<T>(px, okp); v.ey_kp = at<T>(py, okp); v.ex_kp_im = at<T>(px, okp, -1);
+    v.ey_kp_jm = at<T>(py, okp - syb);
+    v.ex_km = at<T>(px, okm); v.ey_km = at<T>(py, okm); v.ez_km = at<T>(pz, okm); v.ez_km_ip = at<T>(pz, okm, 1);
+    v.ez_km_jp = at<T>(pz, okm + syb);
+    v.hx = at<T>(qx, o); v.hy = at<T>(qy, o); v.hz = at<T>(qz, o);
+    v.hy_im = at<T>(qy, o, -1); v.hz_im = at<T>(qz, o, -1);
+    v.hx_jm = at<T>(qx, ojm); v.hz_jm = at<T>(qz, ojm);
+    v.hx_km = at<T>(qx, okm); v.hy_km = at<T>(qy, okm);
+    v.dx = at<T>(C.d0[0], o); v.dy = at<T>(C.d0[1], o); v.dz = at<T>(C.d0[2], o);
+    float4 mc = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (deep && edge && (i == 1 || i == nx - 2)) mc = (i == 1 ? C.mur[0] : C.mur[1])[k * ny + j];
+    const uint32_t m = id & kMaterialMask;
+    v.src = (id & kSourceBit) != 0;
+    const char *lut = (const char *)C.lut + m * (uint32_t)sizeof(MatCoef);
+    if constexpr (EXACT) {
+        const MatCoef *q = (const MatCoef *)lut;
+        v.a = q->a; v.c = q->c; v.d = q->d;
+        v.g1 = q->g1; v.g2 = q->g2; v.g3 = q->g3;
+    } else {
+        const MatCoef *q = (const MatCoef *)lut;
+        v.k1 = q->k1; v.k2 = q->k2; v.k3 = q->k3; v.k5 = q->k5;
+    }
+    bool need = true;
+    if constexpr (EXACT) need = own && !(m < 32 && (C.zmask >> m & 1u));
+    v.exm = v.eym = v.ezm = v.dxm = v.dym = v.dzm = 0.0f;
+    if (need) {
+        v.exm = at<T>(C.e1[0], o); v.eym = at<T>(C.e1[1], o); v.ezm = at<T>(C.e1[2], o);
+        v.dxm = at<T>(C.d1[0], o); v.dym = at<T>(C.d1[1], o); v.dzm = at<T>(C.d1[2], o);
+    }
+
+    const float chx = C.ch[0], chy = C.ch[1], chz = C.ch[2];
+    const float cdx = C.cd[0], cdy = C.cd[1], cdz = C.cd[2];
+    auto up_x = [&](float h, float z, float zjp, float y, float ykp) { return h - chy * (zjp - z) + chy * (ykp - y); };
+    auto up_y = [&](float h, float x, float xkp, float z, float zip) { return h - chz * (xkp - x) + chx * (zip - z); };
+    auto up_z = [&](float h, float y, float yip, float x, float xjp) { return h - chx * (yip - y) + chy * (xjp - x); };
+    auto st = [&](char *p, uint32_t b, float x) { X::st((T *)p, b, x); };
+    auto ld = [&](const char *p, uint32_t b) { return X::ld((const T *)p, b); };
+
+    const bool kh = k < nz - 1, kz = k >= 1 && kh;
+    const bool jl = j < ny - 1, ji = j >= 1 && jl;
+    const bool il = i < nx - 1, ii = i >= 1 && il;
+    const float hx = (ii && jl && kh) ? up_x(v.hx, v.ez, v.ez_jp, v.ey, v.ey_kp) : v.hx;
+    const float hy = (il && ji && kh) ? up_y(v.hy, v.ex, v.ex_kp, v.ez, v.ez_ip) : v.hy;
+    const float hz = (il && jl && kz) ? up_z(v.hz, v.ey, v.ey_ip, v.ex, v.ex_jp) : v.hz;
+    // H^{n+1/2} at j-1, i-1 and k-1 (used only where that cell exists)
+    const float hx_jm = (ii && kh) ? up_x(v.hx_jm, v.ez_jm, v.ez, v.ey_jm, v.ey_kp_jm) : v.hx_jm;
+    const float hz_jm = (il && kz) ? up_z(v.hz_jm, v.ey_jm, v.ey_jm_ip, v.ex_jm, v.ex) : v.hz_jm;
+    const float hy_im = (ji && kh) ? up_y(v.hy_im, v.ex_im, v.ex_kp_im, v.ez_im, v.ez) : v.hy_im;
+    const float hz_im = (jl && kz) ? up_z(v.hz_im, v.ey_im, v.ey, v.ex_im, v.ex_jp_im) : v.hz_im;
+    const float hx_km = (ii && jl) ? up_x(v.hx_km, v.ez_km, v.ez_km_jp, v.ey_km, v.ey) : v.hx_km;
+    const float hy_km = (il && ji) ? up_y(v.hy_km, v.ex_km, v.ex, v.ez_km, v.ez_km_ip) : v.hy_km;
+
+    // A source cell's Dz is written even outside the Dz update range (as in fused_tile).
+    const bool rdx = il && ji && kz, rdy = ii && jl && kz, rdz = (ii && ji && kh) || v.src;
+    const bool reyz = i >= 1 && k >= 1;
+    const float dxu = v.dx + cdy * (hz - hz_jm) - cdz * (hy - hy_km);
+    const float dyu = v.dy + cdz * (hx - hx_km) - cdx * (hz - hz_im);
+    float dzu = v.dz + cdx * (hy - hy_im) - cdy * (hx - hx_jm);
+    dzu = v.src ? dzu - C.jz : dzu;
+    float dyp = dyu, dzp = dzu;
+    // E cells whose D is not updated read the target slot's value (in deep rows those are the cells of the high x
+    // face, whose E the face takes over).
+    if (!deep && own && reyz && !(rdy && rdz)) {
+        if (!rdy) dyp = ld(C.dT[1], o);
+        if (!rdz) dzp = ld(C.dT[2], o);
+    }
+
+    float exn, eyn, ezn;
+    if constexpr (EXACT) {
+        {
+            // see fused_tile: where d*E^n is -0 or E^n or D^n is not finite, the
+            // dropped terms could show, and the operands are loaded after all.
+            // -0 is the least integer; a sum of magnitudes is not finite if one
+            // of them is not (or, harmlessly, if it overflows).
+            const int z = min(min(__float_as_int(v.d * v.ex), __float_as_int(v.d * v.ey)), __float_as_int(v.d * v.ez));
+            const float mag = __builtin_fabsf(v.ex) + __builtin_fabsf(v.ey) + __builtin_fabsf(v.ez) +
+                              __builtin_fabsf(v.dx) + __builtin_fabsf(v.dy) + __builtin_fabsf(v.dz);
+            if (!need && own && (z == (int)0x80000000 || !__builtin_isfinite(mag))) {
+                v.exm = at<T>(C.e1[0], o); v.eym = at<T>(C.e1[1], o); v.ezm = at<T>(C.e1[2], o);
+                v.dxm = at<T>(C.d1[0], o); v.dym = at<T>(C.d1[1], o); v.dzm = at<T>(C.d1[2], o);
+            }
+        }
+        exn = e_update(v.c, v.d, v.a, v.g1, v.g2, v.g3, v.ex, v.exm, dxu, v.dx, v.dxm);
+        eyn = e_update(v.c, v.d, v.a, v.g1, v.g2, v.g3, v.ey, v.eym, dyp, v.dy, v.dym);
+        ezn = e_update(v.c, v.d, v.a, v.g1, v.g2, v.g3, v.ez, v.ezm, dzp, v.dz, v.dzm);
+    } else {
+        exn = e_update_scaled(v.k1, v.k2, v.k3, v.k5, v.ex, v.exm, dxu, v.dx, v.dxm);
+        eyn = e_update_scaled(v.k1, v.k2, v.k3, v.k5, v.ey, v.eym, dyp, v.dy, v.dym);
+        ezn = e_update_scaled(v.k1, v.k2, v.k3, v.k5, v.ez, v.ezm, dzp, v.dz, v.dzm);
+    }
+
+    // Mur faces beside this cell (fdtd_calculations.cu:237-427): c = {q, A, B, C} of
+    // the face cell, tn, sn the neighbour (this cell) at n+1 and n, sf the face at n.
+    auto mur = [](const float4 c, float tn, float sn, float sf, bool once) {
+        return mur_round<T>(c.x, (c.y * tn + c.z * sn) - c.w * sf, once);
+    };
+    const bool hi = C.hi_once != 0;
+    if (deep) {   // only the x faces are near
+        if (own) {
+            st(C.h1[0], o, hx); st(C.h1[1], o, hy); st(C.h1[2], o, hz);
+            if (il) { st(C.dT[0], o, dxu); st(C.eT[0], o, exn); }
+            if (ii) { st(C.dT[1], o, dyu); st(C.eT[1], o, eyn); st(C.eT[2], o, ezn); }
+            if (rdz) st(C.dT[2], o, dzu);
+            if (i == 1) {
+                st(C.eT[1], o - ES, mur(mc, X::rnd(eyn), v.ey, v.ey_im, false));
+                st(C.eT[2], o - ES, mur(mc, X::rnd(ezn), v.ez, v.ez_im, false));
+            }
+            if (i == nx - 2) {
+                // the x-high Ey face reads the source neighbour twice (fdtd_calculations.cu:323-325)
+                st(C.eT[1], o + ES, mur(mc, v.ey, v.ey, v.ey_ip, hi));
+                st(C.eT[2], o + ES, mur(mc, X::rnd(ezn), v.ez, v.ez_ip, hi));
+            }
+        }
+        return;
+    }
+    float pv = 0.0f;
+    auto face = [&](int seg, char *dst, uint32_t b, const float4 *coef, long long cell, float tn, float sn, float sf,
+                    bool once) {
+        const float x = mur(coef[cell], tn, sn, sf, once);
+        if (probe < 0) st(dst, b, x);
+        else if (seg == pseg) pv = x;
+    };
+    const bool fx0 = i == 1, fx1 = i == nx - 2, fy0 = j == 1, fy1 = j == ny - 2, fz0 = k == 1, fz1 = k == nz - 2;
+    if (own && (fx0 || fx1 || fy0 || fy1 || fz0 || fz1)) {
+        const float rx = X::rnd(exn), ry = X::rnd(eyn);
+        // Ez at k = 0 is outside the E update: a face there reads the target slot (not written in this step)
+        float rz = X::rnd(ezn);
+        if (k == 0) rz = ld(C.eT[2], o);
+        const long long cx = (long long)k * ny + j, cy = (long long)k * nx + i, cz = (long long)j * nx + i;
+        if (fx0) {
+            if (jl && kz) face(4, C.eT[1], o - ES, C.mur[0], cx, ry, v.ey, v.ey_im, false);
+            if (ji && kh) face(8, C.eT[2], o - ES, C.mur[0], cx, rz, v.ez, v.ez_im, false);
+        }
+        if (fx1) {
+            if (jl && kz) face(5, C.eT[1], o + ES, C.mur[1], cx, v.ey, v.ey, v.ey_ip, hi);
+            if (ji && kh) face(9, C.eT[2], o + ES, C.mur[1], cx, rz, v.ez, v.ez_ip, hi);
+        }
+        if (fy0) {
+            if (il && kz) face(0, C.eT[0], o - syb, C.mur[2], cy, rx, v.ex, v.ex_jm, true);
+            if (ii && kh) face(10, C.eT[2], o - syb, C.mur[2], cy, rz, v.ez, v.ez_jm, true);
+        }
+        if (fy1) {
+            if (il && kz) face(1, C.eT[0], o + syb, C.mur[3], cy, rx, v.ex, v.ex_jp, true);
+            if (ii && kh) face(11, C.eT[2], o + syb, C.mur[3], cy, rz, v.ez, v.ez_jp, true);
+        }
+        if (fz0) {
+            if (il && ji) face(2, C.eT[0], o - szb, C.mur[4], cz, rx, v.ex, v.ex_km, true);
+            if (ii && jl) face(6, C.eT[1], o - szb, C.mur[4], cz, ry, v.ey, v.ey_km, true);
+        }
+        if (fz1) {
+            if (il && ji) face(3, C.eT[0], o + szb, C.mur[5], cz, rx, v.ex, v.ex_kp, true);
+            if (ii && jl) face(7, C.eT[1], o + szb, C.mur[5], cz, ry, v.ey, v.ey_kp, true);
+        }
+    }
+    if (probe < 0) {
+        if (own) {
+            st(C.h1[0], o, hx); st(C.h1[1], o, hy); st(C.h1[2], o, hz);
+            if (rdx) { st(C.dT[0], o, dxu); st(C.eT[0], o, exn); }
+            if (rdy) st(C.dT[1], o, dyu);
+            if (rdz) st(C.dT[2], o, dzu);
+            // face cells that a segment covers are stored by their neighbour's lane
+            const bool fy = (i == nx - 1 && jl && kz) || (k == nz - 1 && ii && jl);
+            const bool fz = (i == nx - 1 && ji && kh) || ((j == 0 || j == ny - 1) && ii && kh);
+            if (reyz && !fy) st(C.eT[1], o, eyn);
+            if (reyz && !fz) st(C.eT[2], o, ezn);
+        }
+        return;
+    }
+    // the value probe pf records: what this step stores, or what the target slot keeps
+    switch (pf) {
+    case 0: pv = rdx ? X::rnd(dxu) : ld(C.dT[0], o); break;
+    case 1: pv = rdy ? X::rnd(dyu) : ld(C.dT[1], o); break;
+    case 2: pv = rdz ? X::rnd(dzu) : ld(C.dT[2], o); break;
+    case 3: pv = X::rnd(hx); break;
+    case 4: pv = X::rnd(hy); break;
+    case 5: pv = X::rnd(hz); break;
+    default:
+        if (pseg < 0) {
+            if (pf == 6) pv = rdx ? X::rnd(exn) : ld(C.eT[0], o);
+            else if (pf == 7) pv = reyz ? X::rnd(eyn) : ld(C.eT[1], o);
+            else pv = reyz ? X::rnd(ezn) : ld(C.eT[2], o);
+        }
+        break;
+    }
+    if ((threadIdx.x & 63) == 0) C.p.out[(long long)C.p.row * C.p.nprobe + probe] = (double)pv * C.p.factor[pf];
+}
+
+template <typename T, bool EXACT>
+hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
+{
+    const void *k = c.bxl == 6 ? (const void *)cell_step<T, EXACT, 6> : (const void *)cell_step<T, EXACT, 5>;
+    const unsigned gx = 8u * (unsigned)c.run;
+    const unsigned waves = kCellBlock / 64, pb = ((unsigned)c.p.nprobe + waves - 1) / waves;
+    const dim3 grid(gx, (unsigned)c.nz + (pb + gx - 1) / gx);
+    CellArgs arg = c;
+    void *args[] = {&arg};
+    return hipExtLaunchKernel(k, grid, dim3(kCellBlock), args, 0, s, t0, t1, 0);
+}
+
+// One coefficient per thread; blockIdx.y: the face.
+__global__ __launch_bounds__(kCellBlock) void mur_coefs(const MurCoefArgs a)
+{
+    const int f = (int)blockIdx.y, axis = f >> 1, end = f & 1;
+    const long long n = axis == 0 ? (long long)a.ny * a.nz : axis == 1 ? (long long)a.nx * a.nz : (long long)a.nx * a.ny;
+    const long long q = (long long)blockIdx.x * kCellBlock + threadIdx.x;
+    if (q >= n) return;
+    // the two cells of the pair in the reference's plane: x (k, j, 2), y (k, 2, i), z (2, j, i)
+    const long long k = q / a.nx, at = axis == 0 ? 2 * q : axis == 1 ? 2 * k * a.nx + (q - k * a.nx) : q;
+    const long long step = axis == 0 ? 1 : axis == 1 ? a.nx : n;
+    const float *rp = axis == 0 ? a.rp[end ? 3 : 0] : axis == 1 ? a.rp[end ? 4 : 1] : a.rp[end ? 5 : 2];
+    const float rpf = rp[at + (end ? step : 0)], rpn = rp[at + (end ? 0 : step)];
+    const float h = axis == 0 ? a.h[0] : axis == 1 ? a.h[1] : a.h[2];
+    const float sf = sqrtf(a.mu0 * a.eps0 * rpf), sn = sqrtf(a.mu0 * a.eps0 * rpn);
+    float4 c;
+    c.x = 1 / (a.dt + h * sf);
+    c.y = a.dt - h * sn;
+    c.z = a.dt + h * sn;
+    c.w = a.dt - h * sf;
+    const long long nyz = (long long)a.ny * a.nz, nxz = (long long)a.nx * a.nz;
+    const long long base = axis == 0 ? 0 : axis == 1 ? 2 * nyz : 2 * (nyz + nxz);
+    a.out[base + end * n + q] = c;
+}
+
+}  // namespace
+
+hipError_t launch_mur_coefs(const MurCoefArgs &a, hipStream_t s)
+{
+    const long long m = std::max({(long long)a.ny * a.nz, (long long)a.nx * a.nz, (long long)a.nx * a.ny});
+    mur_coefs<<<dim3((unsigned)((m + kCellBlock - 1) / kCellBlock), 6), kCellBlock, 0, s>>>(a);
+    return hipGetLastError();
+}
+
+hipError_t launch_cell_step(const CellArgs &c, int storage, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
+{
+    switch (storage) {
+    case kStoreF32: return launch_cell_t<float, true>(c, s, t0, t1);
+    case kStoreF32Fast: return launch_cell_t<float, false>(c, s, t0, t1);
+    case kStoreF16: return launch_cell_t<__half, false>(c, s, t0, t1);
+    case kStoreBF16: return launch_cell_t<__hip_bfloat16, false>(c, s, t0, t1);
+    default: return hipErrorInvalidValue;
+    }
+}

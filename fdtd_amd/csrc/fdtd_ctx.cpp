@@ -40,6 +40,7 @@ struct fdtd_ctx {
     int ty, kchunk, tiles_x, tiles_y, tiles_z;
     int cpl = 1;                         // cells per lane of the fused kernel
     int txw = 64;                        // threads per tile row (one cell per lane)
+    bool cell = false;                   // steps run as cell_step, not in tiles
     bool fields_set = false;             // set_field or load gave non-zero state
 
     long long guard = 0;                 // elements before/after the field arrays and the ids
@@ -56,10 +57,11 @@ struct fdtd_ctx {
     unsigned char *ids = nullptr;
     MatCoef *lut = nullptr;
     int nmat = 0;
+    uint32_t zmask = 0;                  // bit m < 32: material m has a = g3 = +0 (CellArgs)
     std::vector<float> table;             // nmat x {sigma, eps_s, eps_inf, tau}
     bool lut_dirty = true;
     float *rp[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    float4 *murx = nullptr;              // x-face Mur coefficients: 2 planes of ny*nz
+    float4 *mur = nullptr;               // Mur coefficients of the six faces (launch_mur_coefs)
     std::vector<unsigned char> ids_host;  // material ids without source bits
     std::vector<int> src;                 // 3 per source
     std::vector<int> probe_field;         // field of each probe
@@ -144,6 +146,13 @@ int upload_lut(fdtd_ctx *c)
     HIP_TRY(hipDeviceSynchronize());
     HIP_TRY(hipMemcpy(c->lut, lut.data(), sizeof(MatCoef) * c->nmat, hipMemcpyHostToDevice));
     c->lut_dirty = false;
+    c->zmask = 0;
+    for (int m = 0; m < std::min(c->nmat, 32); m++) {
+        uint32_t a, g[2];
+        memcpy(&a, &lut[m].a, 4);
+        memcpy(g, &lut[m].g3, 8);
+        if (a == 0 && g[0] == 0 && g[1] == 0) c->zmask |= 1u << m;
+    }
     return 0;
 }
 
@@ -158,6 +167,18 @@ void set_shape(fdtd_ctx *c, int ty, int kchunk, int cpl, int txw = 64)
     c->tiles_y = (c->ny + ty - 1) / ty;
     c->tiles_z = (c->nz + c->kchunk - 1) / c->kchunk;
     c->kchunk2 = c->kchunk;
+}
+
+// Whether a context steps one cell per lane (cell_step): nothing of the tiled
+// launch is asked for, and the padded state is small enough (cell_state_limit).
+bool default_cell(const fdtd_ctx *c)
+{
+    const FdtdExt &e = c->ext;
+    if (e.tile_y || e.kchunk || e.tile_x || e.lane_cells || e.time_steps == 2) return false;
+    FdtdExt d;
+    fdtd_ext_defaults(&d);
+    if (e.xcd_remap != d.xcd_remap) return false;
+    return c->nz <= kCellMaxPlanes && 24 * c->Np * c->esz <= cell_state_limit(c->esz);
 }
 
 // Launch shape a context takes for a grid, from launch-shape sweeps on
@@ -182,12 +203,18 @@ void default_shape(int nx, int ny, int nz, const FdtdExt &e, int cus, int *ty, i
     *txw = *cpl == 2 ? 64 : (e.tile_x ? e.tile_x : 64);
 }
 
-hipError_t upload_murx(fdtd_ctx *c, const float *rpx0, const float *rpxEnd)
+// The Mur coefficients of the six faces, from the rp planes on the device;
+// waits for them (steps may follow on any stream).
+hipError_t set_mur(fdtd_ctx *c)
 {
-    const size_t n = (size_t)c->ny * c->nz;
-    std::vector<float4> h(2 * n);
-    mur_x_coefs(c->ny, c->nz, c->dt, c->dx, c->mu0, c->eps0, rpx0, rpxEnd, h.data(), h.data() + n);
-    return hipMemcpy(c->murx, h.data(), sizeof(float4) * 2 * n, hipMemcpyHostToDevice);
+    MurCoefArgs a;
+    for (int r = 0; r < 6; r++) a.rp[r] = c->rp[r];
+    a.out = c->mur;
+    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
+    a.dt = c->dt; a.mu0 = c->mu0; a.eps0 = c->eps0;
+    a.h[0] = c->dx; a.h[1] = c->dy; a.h[2] = c->dz;
+    const hipError_t e = launch_mur_coefs(a, nullptr);
+    return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
 }
 
 }  // namespace
@@ -261,6 +288,7 @@ extern "C" int fdtd_ctx_create(const FdtdParams *p, const FdtdExt *ext, fdtd_ctx
     int txw = 64;
     default_shape(c->nx, c->ny, c->nz, e, 0, &c->ty, &c->kchunk, &c->cpl, &txw);
     set_shape(c, c->ty, c->kchunk, c->cpl, txw);
+    c->cell = default_cell(c);
 
     const size_t nf = 24;  // 9 E + 9 D + 6 H
     c->guard = fused_guard(c->pitch, c->plane);
@@ -284,16 +312,10 @@ extern "C" int fdtd_ctx_create(const FdtdParams *p, const FdtdExt *ext, fdtd_ctx
                            (size_t)2 * c->ny * c->nz, (size_t)c->nx * 2 * c->nz, (size_t)c->nx * c->ny * 2};
     for (int r = 0; r < 6 && he == hipSuccess; r++) {
         he = hipMalloc(&c->rp[r], rps[r] * sizeof(float));
-        if (he == hipSuccess) {
-            std::vector<float> ones(rps[r], 1.0f);
-            he = hipMemcpy(c->rp[r], ones.data(), rps[r] * sizeof(float), hipMemcpyHostToDevice);
-        }
+        if (he == hipSuccess) he = hipMemsetD32((hipDeviceptr_t)c->rp[r], 0x3f800000, rps[r]);   // 1.0f
     }
-    if (he == hipSuccess) he = hipMalloc(&c->murx, sizeof(float4) * 2 * (size_t)c->ny * c->nz);
-    if (he == hipSuccess) {
-        std::vector<float> o0((size_t)2 * c->ny * c->nz, 1.0f);
-        he = upload_murx(c, o0.data(), o0.data());
-    }
+    if (he == hipSuccess) he = hipMalloc(&c->mur, sizeof(float4) * mur_coef_count(c->nx, c->ny, c->nz));
+    if (he == hipSuccess) he = set_mur(c);
     if (he != hipSuccess) {
         int rc = fdtd_hip_fail(he, "fdtd_ctx_create");
         fdtd_ctx_destroy(c);
@@ -316,7 +338,7 @@ extern "C" int fdtd_ctx_destroy(fdtd_ctx *c)
     (void)hipFree(c->ids_base);
     (void)hipFree(c->lut);
     for (int r = 0; r < 6; r++) (void)hipFree(c->rp[r]);
-    (void)hipFree(c->murx);
+    (void)hipFree(c->mur);
     (void)hipFree(c->probes);
     (void)hipFree(c->probe_out);
     (void)hipFree(c->slice_stage);
@@ -388,7 +410,7 @@ extern "C" int fdtd_ctx_set_rp(fdtd_ctx *c, const float *rpx0, const float *rpy0
     HIP_TRY(hipDeviceSynchronize());
     for (int r = 0; r < 6; r++)
         HIP_TRY(hipMemcpy(c->rp[r], src[r], rps[r] * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(upload_murx(c, rpx0, rpxEnd));
+    HIP_TRY(set_mur(c));
     return 0;
 }
 
@@ -520,8 +542,8 @@ void fill_step_args(fdtd_ctx *c, int n, StepArgs &a)
     a.mur_x = fused_mur_x(c->nx, c->kchunk, 64 * c->cpl);
     a.cpl = c->cpl;
     a.txw = c->txw;
-    a.murx0 = c->murx;
-    a.murx1 = c->murx + (size_t)c->ny * c->nz;
+    a.murx0 = c->mur;
+    a.murx1 = c->mur + (size_t)c->ny * c->nz;
     // zero-term rows rely on E^{n-1}, D^{n-1} being finite wherever E^n, D^n are, which stepping from
     // zero (or from any state the steps made) keeps; a state set from outside may not
     a.zskip = (c->storage == FDTD_STORE_F32 && c->ext.load_zero_terms == 0 && !c->fields_set) ? 1 : 0;
@@ -558,6 +580,49 @@ ProbeArgs probe_row(fdtd_ctx *c, char *const *fields)
         p.row = c->probe_rows++;
     }
     return p;
+}
+
+// One launch of cell_step for the step of `a` (c->n and c->hcur already
+// advanced, so that the probe row names the newest fields).
+void fill_cell_args(fdtd_ctx *c, const StepArgs &a, CellArgs &q)
+{
+    const size_t gb = (size_t)c->guard * c->esz;
+    auto in = [&](const char **d, const void *x, const void *y, const void *z) {
+        d[0] = (const char *)x - gb; d[1] = (const char *)y - gb; d[2] = (const char *)z - gb;
+    };
+    auto out = [&](char **d, void *x, void *y, void *z) { d[0] = (char *)x - gb; d[1] = (char *)y - gb; d[2] = (char *)z - gb; };
+    in(q.e0, a.ex0, a.ey0, a.ez0);
+    in(q.e1, a.ex1, a.ey1, a.ez1);
+    in(q.d0, a.dx0, a.dy0, a.dz0);
+    in(q.d1, a.dx1, a.dy1, a.dz1);
+    in(q.h0, a.hxo, a.hyo, a.hzo);
+    out(q.eT, a.exT, a.eyT, a.ezT);
+    out(q.dT, a.dxT, a.dyT, a.dzT);
+    out(q.h1, a.hxn, a.hyn, a.hzn);
+    q.ids = a.ids - c->guard;
+    q.lut = a.lut;
+    q.nx = c->nx; q.ny = c->ny; q.nz = c->nz;
+    q.o0 = (uint32_t)gb;
+    q.sy = (uint32_t)(c->pitch * c->esz);
+    q.sz = (uint32_t)(c->plane * c->esz);
+    q.ch[0] = a.chx; q.ch[1] = a.chy; q.ch[2] = a.chz;
+    q.cd[0] = a.cdx; q.cd[1] = a.cdy; q.cd[2] = a.cdz;
+    q.jz = a.jz;
+    q.zmask = a.zskip ? c->zmask : 0;
+    q.bxl = cell_lanes_log2(c->nx);
+    q.hi_once = a.mur_x == 2;
+    const int bx = 1 << q.bxl, by = 256 / bx;
+    q.tiles_x = (c->nx + bx - 1) / bx;
+    q.tx_mul = (uint32_t)(((1ull << 32) + q.tiles_x - 1) / q.tiles_x);
+    q.tiles = q.tiles_x * ((c->ny + by - 1) / by);
+    q.run = (q.tiles + 7) / 8;
+    const size_t nyz = (size_t)c->ny * c->nz, nxz = (size_t)c->nx * c->nz, nxy = (size_t)c->nx * c->ny;
+    const float4 *m = c->mur;
+    const size_t step[6] = {nyz, nyz, nxz, nxz, nxy, nxy};
+    for (int f = 0; f < 6; f++) { q.mur[f] = m; m += step[f]; }
+    char *fields[9];
+    for (int f = 0; f < 9; f++) fields[f] = field_dev(c, f, 0);
+    q.p = probe_row(c, fields);
 }
 
 // Energy sum and z-slice capture of step c->n, when due.
@@ -709,6 +774,17 @@ extern "C" int fdtd_step_fused(fdtd_ctx *c, hipStream_t stream)
     StepArgs a;
     fill_step_args(c, n, a);
     const bool timed = timed_launch(c, 1);
+    hipEvent_t t0 = timed ? c->tev[2 * c->tused] : nullptr, t1 = timed ? c->tev[2 * c->tused + 1] : nullptr;
+    if (c->cell) {
+        c->n = n + 1;
+        c->hcur ^= 1;
+        CellArgs q;
+        fill_cell_args(c, a, q);
+        const hipError_t e = launch_cell_step(q, c->storage, stream, t0, t1);
+        if (e != hipSuccess) return fdtd_hip_fail(e, "cell_step");
+        if (timed) c->tused++;
+        return after_step(c, stream);
+    }
     hipError_t e = timed ? launch_fused_step(a, c->ty, c->storage, stream, c->tev[2 * c->tused], c->tev[2 * c->tused + 1])
                          : launch_fused_step(a, c->ty, c->storage, stream);
     if (e != hipSuccess) return fdtd_hip_fail(e, "fused_step");
@@ -1089,20 +1165,26 @@ extern "C" int fdtd_ctx_autotune(fdtd_ctx *c, int trial_steps, hipStream_t strea
     const int nform = c->esz == 2 ? 3 : 2;
     float best = 0.0f;
     int bty = c->ty, bkc = c->kchunk, bcpl = c->cpl, btxw = c->txw;
+    bool bcell = false;
+    auto trial = [&]() -> float {   // ms of the trial steps as the context is set up now
+        rc = fdtd_run(c, 2, stream);
+        if (rc) return 0.0f;
+        e = hipEventRecord(t0, stream);
+        if (e == hipSuccess) rc = fdtd_run(c, trial_steps, stream);
+        if (!rc && e == hipSuccess) e = hipEventRecord(t1, stream);
+        if (!rc && e == hipSuccess) e = hipEventSynchronize(t1);
+        float ms = 0.0f;
+        if (!rc && e == hipSuccess) e = hipEventElapsedTime(&ms, t0, t1);
+        if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune timing");
+        return ms;
+    };
+    c->cell = false;
     for (int a = 0; a < 3 && !rc; a++)
         for (int b = 0; b < 5 && !rc; b++)
             for (int f = 0; f < nform && !rc; f++) {
                 const int q = forms[f][0], w = forms[f][1];
                 set_shape(c, tys[a], kcs[b], q, w);
-                rc = fdtd_run(c, 2, stream);
-                if (rc) break;
-                e = hipEventRecord(t0, stream);
-                if (e == hipSuccess) rc = fdtd_run(c, trial_steps, stream);
-                if (!rc && e == hipSuccess) e = hipEventRecord(t1, stream);
-                if (!rc && e == hipSuccess) e = hipEventSynchronize(t1);
-                float ms = 0.0f;
-                if (!rc && e == hipSuccess) e = hipEventElapsedTime(&ms, t0, t1);
-                if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune timing");
+                const float ms = trial();
                 if (!rc && (best == 0.0f || ms < best)) {
                     best = ms;
                     bty = tys[a];
@@ -1111,6 +1193,11 @@ extern "C" int fdtd_ctx_autotune(fdtd_ctx *c, int trial_steps, hipStream_t strea
                     btxw = w;
                 }
             }
+    if (!rc && c->ext.time_steps != 2 && c->nz <= kCellMaxPlanes) {
+        c->cell = true;
+        const float ms = trial();
+        bcell = !rc && ms < best;
+    }
     if (t0) (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);
     // back to the zero state at step 0
@@ -1129,6 +1216,7 @@ extern "C" int fdtd_ctx_autotune(fdtd_ctx *c, int trial_steps, hipStream_t strea
     c->tseen = 0;
     c->tkind = 0;
     set_shape(c, bty, bkc, bcpl, btxw);
+    c->cell = bcell;
     if (rc) return rc;
     if (tile_y) *tile_y = bty;
     if (kchunk) *kchunk = bkc;

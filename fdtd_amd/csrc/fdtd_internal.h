@@ -73,15 +73,30 @@ struct StepArgs {
     int zskip;
 };
 
-// Coefficients {q, A, B, C} of the first-order Mur update of one x-face
+// Coefficients {q, A, B, C} of the first-order Mur update of one face
 // cell, E' = q*((A*tn + B*sn) - C*sf), evaluated in float exactly as the
-// reference's expression (fdtd_calculations.cu:303-329, 369-395) rounds
+// reference's expression (fdtd_calculations.cu:216-428) rounds
 // them: q = 1/(dt + h sqrt(mu0 eps0 rp_face)), A = dt - h sqrt(mu0 eps0
 // rp_nb), B = dt + h sqrt(mu0 eps0 rp_nb), C = dt - h sqrt(mu0 eps0
-// rp_face).  Planes of ny*nz entries, (k, j) order: out0 from rpx0 (face
-// index 0), out1 from rpxEnd (face index 1).
+// rp_face).  mur_x_coefs: planes of ny*nz entries, (k, j) order: out0 from
+// rpx0 (face index 0), out1 from rpxEnd (face index 1).
 void mur_x_coefs(int ny, int nz, float dt, float hx, float mu0, float eps0, const float *rpx0, const float *rpxEnd,
                  float4 *out0, float4 *out1);
+
+// The same on the device for the six faces of a grid, from its rp planes in
+// fdtd_ctx_set_rp's order: out holds x low, x high in (k, j) order, y low, y
+// high in (k, i) order, z low, z high in (j, i) order, one after the other.
+struct MurCoefArgs {
+    const float *rp[6];
+    float4 *out;
+    int nx, ny, nz;
+    float dt, h[3], mu0, eps0;
+};
+inline size_t mur_coef_count(int nx, int ny, int nz)
+{
+    return 2 * ((size_t)ny * nz + (size_t)nx * nz + (size_t)nx * ny);
+}
+hipError_t launch_mur_coefs(const MurCoefArgs &a, hipStream_t s);
 
 // Which Mur x faces the fused kernel takes over.  The x-high faces need the
 // cell at i = nx-2 from the face's wave: E^{n+1}_z from the previous lane
@@ -166,6 +181,45 @@ struct EnergyArgs {
 };
 constexpr int kEnergyBlocks = 1024;
 hipError_t launch_energy(const EnergyArgs &a, int storage, hipStream_t s);
+
+// One step of a grid in one launch, one cell per lane, with its Mur faces and
+// probe row (fdtd_cell.hip).  The field and id pointers lie fused_guard
+// elements before the arrays' origins; o0 = the guard in bytes.
+struct CellArgs {
+    const char *e0[3], *e1[3], *d0[3], *d1[3], *h0[3];   // E, D at levels n and n-1, H^{n-1/2}
+    char *eT[3], *dT[3], *h1[3];                         // E, D at level n+1, H^{n+1/2}
+    const uint8_t *ids;
+    const MatCoef *lut;
+    int nx, ny, nz;
+    uint32_t o0, sy, sz;           // bytes: guard, row, plane
+    int tiles_x, tiles, run;       // tiles per row and per plane, ceil(tiles / 8)
+    uint32_t tx_mul;               // ceil(2^32 / tiles_x)
+    float ch[3], cd[3], jz;
+    uint32_t zmask;                // bit m: material m < 32 has a = g3 = +0 and its cells do not load levels n-1
+    int bxl;                       // 5 or 6: 32 or 64 lanes of a 256-lane tile along x
+    int hi_once;                   // the tiled step leaves the x-high faces to the Mur kernel (fused_mur_x 2)
+    const float4 *mur[6];          // launch_mur_coefs: x low, x high, y low, ...
+    ProbeArgs p;                   // p.nprobe = 0: no probe row; p.field is not read
+};
+// Padded state (bytes of the 24 field arrays) up to which a context steps
+// with cell_step.  fp32 crosses the tiled launch where the Infinity Cache
+// (256 MB) no longer holds most of the state: 54 against 69 us at 285 MB
+// (160x160x116), 57.6 against 64.4 at 283 MB (128x128x180), even at 344 MB
+// (160x160x140, 79.5 against 78.7), 98 against 83 at 398 MB.  The 16-bit tiled
+// kernels are held by instructions: even at 566 MB (fp16 256x256x180, 155
+// against 153.5), 173 against 181 at 629 MB, 215 against 205 at 805 MB.
+constexpr int kCellMaxPlanes = 60000;   // planes and probe rows are blockIdx.y
+inline size_t cell_state_limit(size_t esz) { return esz == 2 ? 640000000 : 320000000; }
+// log2 of the lanes of its tiles along x: 64, or 32 where those leave clearly
+// fewer lanes idle (96 wide: 16.1 against 16.8 us in fp32, 13.0 against 13.8
+// in fp16; 160 wide, where 32 lanes would fill 20 % more: 35.2 against 37.5).
+inline int cell_lanes_log2(int nx)
+{
+    const double e6 = (double)nx / (64 * ((nx + 63) / 64)), e5 = (double)nx / (32 * ((nx + 31) / 32));
+    return e6 < 0.8 * e5 ? 5 : 6;
+}
+hipError_t launch_cell_step(const CellArgs &c, int storage, hipStream_t s, hipEvent_t t0 = nullptr,
+                            hipEvent_t t1 = nullptr);
 
 // Streaming probe (fdtd_stream_probe): 15 read and 9 written arrays of n floats.
 struct StreamMix {

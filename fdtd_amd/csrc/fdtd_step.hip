@@ -17,14 +17,13 @@
 //     a uint8 id per cell (top bit = source cell), staged in LDS.
 // mur_faces: the 12 (component, face) first-order Mur updates
 // (fdtd_calculations.cu:216-428) over face cells only.
-#include <hip/hip_bf16.h>
-#include <hip/hip_fp16.h>
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <type_traits>
 
+#include "fdtd_device.h"
 #include "fdtd_internal.h"
 
 namespace {
@@ -64,93 +63,6 @@ __device__ inline int xcd_logical(int b, int nblk, int mode, int unit)
 __device__ inline int xcd_unit(int mode, int tiles_x, int tiles_y)
 {
     return mode == 3 ? tiles_x : mode == 4 ? (tiles_y + 7) / 8 * tiles_x : tiles_x * tiles_y;
-}
-
-__device__ inline float e_update(float c, float d, float a, double g1, double g2, double g3, float e0, float e1,
-                                 float dn1, float dn, float dm1)
-{
-    const float fe = d * e0 - a * e1;
-    double s = (double)fe + g1 * (double)dn1;
-    s = s - g2 * (double)dn;
-    s = s + g3 * (double)dm1;
-    return (float)((double)c * s);
-}
-
-// Element access at a 32-bit byte offset from a scalar base, for the three
-// storage types.  fp32 values pass through; fp16/bf16 convert to and from
-// fp32 with round-to-nearest-even.  The _nt forms are the streaming
-// (nontemporal) variants for data a launch touches once: the ring levels n
-// and n-1 of D, level n-1 of E and every store.
-template <typename T> struct Elem;
-
-template <> struct Elem<float> {
-    static __device__ __forceinline__ float rnd(float v) { return v; }
-    static __device__ __forceinline__ float ld(const float *p, uint32_t b) { return *(const float *)((const char *)p + b); }
-    static __device__ __forceinline__ float ld_nt(const float *p, uint32_t b)
-    {
-        return __builtin_nontemporal_load((const float *)((const char *)p + b));
-    }
-    static __device__ __forceinline__ void st(float *p, uint32_t b, float v) { *(float *)((char *)p + b) = v; }
-    static __device__ __forceinline__ void st_nt(float *p, uint32_t b, float v)
-    {
-        __builtin_nontemporal_store(v, (float *)((char *)p + b));
-    }
-};
-
-template <> struct Elem<__half> {
-    static __device__ __forceinline__ float cvt(unsigned short u) { return __half2float(__ushort_as_half(u)); }
-    static __device__ __forceinline__ unsigned short enc(float v) { return __half_as_ushort(__float2half_rn(v)); }
-    static __device__ __forceinline__ float rnd(float v) { return cvt(enc(v)); }
-    static __device__ __forceinline__ float ld(const __half *p, uint32_t b)
-    {
-        return cvt(*(const unsigned short *)((const char *)p + b));
-    }
-    static __device__ __forceinline__ float ld_nt(const __half *p, uint32_t b)
-    {
-        return cvt(__builtin_nontemporal_load((const unsigned short *)((const char *)p + b)));
-    }
-    static __device__ __forceinline__ void st(__half *p, uint32_t b, float v) { *(unsigned short *)((char *)p + b) = enc(v); }
-    static __device__ __forceinline__ void st_nt(__half *p, uint32_t b, float v)
-    {
-        __builtin_nontemporal_store(enc(v), (unsigned short *)((char *)p + b));
-    }
-};
-
-template <> struct Elem<__hip_bfloat16> {
-    static __device__ __forceinline__ float cvt(unsigned short u) { return __uint_as_float((uint32_t)u << 16); }
-    static __device__ __forceinline__ unsigned short enc(float v)
-    {
-        // round to nearest even; NaN stays NaN
-        const uint32_t x = __float_as_uint(v);
-        if ((x & 0x7fffffffu) > 0x7f800000u) return (unsigned short)((x >> 16) | 0x40u);
-        return (unsigned short)((x + 0x7fffu + ((x >> 16) & 1u)) >> 16);
-    }
-    static __device__ __forceinline__ float rnd(float v) { return cvt(enc(v)); }
-    static __device__ __forceinline__ float ld(const __hip_bfloat16 *p, uint32_t b)
-    {
-        return cvt(*(const unsigned short *)((const char *)p + b));
-    }
-    static __device__ __forceinline__ float ld_nt(const __hip_bfloat16 *p, uint32_t b)
-    {
-        return cvt(__builtin_nontemporal_load((const unsigned short *)((const char *)p + b)));
-    }
-    static __device__ __forceinline__ void st(__hip_bfloat16 *p, uint32_t b, float v)
-    {
-        *(unsigned short *)((char *)p + b) = enc(v);
-    }
-    static __device__ __forceinline__ void st_nt(__hip_bfloat16 *p, uint32_t b, float v)
-    {
-        __builtin_nontemporal_store(enc(v), (unsigned short *)((char *)p + b));
-    }
-};
-
-// E^{n+1} in scaled units (16-bit storage): fp32 throughout.
-__device__ inline float e_update_scaled(float k1, float k2, float k3, float k5, float e0, float e1, float dn1,
-                                        float dn, float dm1)
-{
-    const float d1 = dn1 - dn;
-    const float d2 = d1 - (dn - dm1);
-    return k1 * e0 - k2 * e1 + k3 * d1 + k5 * d2;
 }
 
 // First-order Mur update of one face cell (fdtd_calculations.cu:237-427):

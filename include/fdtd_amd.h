@@ -183,7 +183,7 @@ int fdtd_ctx_load(fdtd_ctx *ctx, const char *path);
  * the five launches of one step of the reference's loop (fdtd.cu:129-214,
  * updateHField ... updateMurBoundary, with the ring rotation of
  * fdtd.cu:115-530) as two launches, the fused H/D/source/E kernel and the
- * Mur faces with the step's probe row. */
+ * Mur faces with the step's probe row, or for a small grid as one. */
 int fdtd_step_fused(fdtd_ctx *ctx, hipStream_t stream);
 /* `steps` steps; enqueues only (no host synchronisation). */
 int fdtd_run(fdtd_ctx *ctx, int steps, hipStream_t stream);
@@ -219,13 +219,16 @@ int fdtd_slices_read(fdtd_ctx *ctx, int *steps, float *data, int max_slices);
 
 /* Autotuner: times every launch shape (tile rows {2,4,8} x z planes per
  * block {3,4,6,8,16} x tile rows of 64 or 128 threads, and two cells per lane
- * under 16-bit storage) on this
- * grid for trial_steps steps each, keeps the fastest and returns the
+ * under 16-bit storage, and one lane per cell without tiles) on this
+ * grid for trial_steps steps each, keeps the fastest (tile_y, kchunk and
+ * lane_cells: the fastest of the shapes) and returns the
  * context to its zero state at step 0 (probe rows and captures restart).
  * Needs a context that has not stepped and whose fields were not set. */
 int fdtd_ctx_autotune(fdtd_ctx *ctx, int trial_steps, hipStream_t stream, int *tile_y, int *kchunk, int *lane_cells);
 
-/* The launch shape chosen for the context's fused kernel. */
+/* The launch shape chosen for the context's fused kernel.  A context whose
+ * state fits the Infinity Cache, and whose FdtdExt fixes no part of the shape,
+ * steps with one lane per cell instead (same results) and does not use it. */
 int fdtd_ctx_launch_shape(fdtd_ctx *ctx, int *tile_x, int *tile_y, int *kchunk, int *blocks);
 /* The launch shape fdtd_ctx_create would take for this grid and extension
  * (no counterpart in the reference, whose launch geometry is fixed at

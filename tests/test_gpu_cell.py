@@ -1,0 +1,102 @@
+"""The one-lane-per-cell step (small grids) against the tiled step and the
+oracle: widths at and around the tile edges, the smallest grids, faces seen
+by probes, sources on the upper faces, every storage form."""
+import numpy as np
+import pytest
+
+import fdtd_amd as F
+from tests.helpers import bits_equal, first_diff
+
+pytestmark = pytest.mark.gpu
+
+DT, DX = 3.8105118e-12, 2.0e-3
+MU0, EPS0 = 1.2566371e-06, 8.841941e-12
+
+SHAPES = [(3, 3, 3), (4, 9, 5), (33, 5, 4), (64, 6, 5), (65, 9, 6), (97, 12, 7), (31, 66, 12), (130, 17, 9)]
+
+
+def _probes(shape):
+    """Every field inside, at the corners of the box and on each face."""
+    nx, ny, nz = shape
+    at = [(nx // 2, ny // 2, nz // 2), (0, 0, 0), (nx - 1, ny - 1, nz - 1), (0, ny // 2, nz // 2),
+          (nx - 1, ny // 2, nz // 2), (nx // 2, 0, nz // 2), (nx // 2, ny - 1, nz // 2), (nx // 2, ny // 2, 0),
+          (nx // 2, ny // 2, nz - 1), (1, 1, 1), (nx - 2, ny - 2, nz - 2), (0, 1, 0)]
+    return np.asarray([(f, *c) for c in at for f in range(9)], np.int32)
+
+
+def _run(shape, storage, steps, tiled):
+    rng = np.random.default_rng([*shape, storage])
+    nx, ny, nz = shape
+    table = np.asarray([(0.0, 1.0, 1.0, 0.0), (0.8, 55.0, 40.0, 8e-12), (0.1, 4.0, 3.0, 0.0)], np.float32)
+    ids = rng.integers(0, 3, (nz, ny, nx)).astype(np.uint8)
+    rps = [rng.uniform(1.0, 3.0, n).astype(np.float32) for n in (2 * ny * nz, nx * 2 * nz, nx * ny * 2) * 2]
+    src = np.asarray([(nx - 1, 1, nz // 2), (1, ny - 1, nz - 1), (nx // 2 or 1, ny // 2 or 1, nz // 2)], np.int32)
+    jz = rng.uniform(-1.0, 1.0, steps).astype(np.float32)
+    probes = _probes(shape)
+    with F.Context(F.make_params(shape, DT, DX, 1.1 * DX, 0.9 * DX, MU0, EPS0), storage=storage,
+                   tile_y=4 if tiled else 0) as ctx:
+        ctx.set_materials(ids, table)
+        ctx.set_rp(rps)
+        ctx.set_sources(src, jz)
+        ctx.set_probes(probes, steps)
+        ctx.step()
+        ctx.run(steps - 1)
+        fields = {(f, lv): ctx.get(f, lv) for f in range(9) for lv in ([0] if 3 <= f < 6 else [0, 1, 2])}
+        series = ctx.probes()
+    for p, (f, i, j, k) in enumerate(probes):   # a probe's last row is the field's value
+        assert np.float32(series[-1, p]) == fields[(f, 0)][k, j, i], f"probe {F.FIELDS[f]} at {(i, j, k)}"
+    return fields, series
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("storage", [F.STORE_F32, F.STORE_F16, F.STORE_BF16, F.STORE_F32_FAST])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_cells_equal_tiles(shape, storage):
+    a, pa = _run(shape, storage, 7, False)
+    b, pb = _run(shape, storage, 7, True)
+    for key in a:
+        assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
+    assert np.array_equal(pa.view(np.uint64), pb.view(np.uint64))
+    assert np.isfinite(pa).all() and np.abs(pa).max() > 0
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("shape", [(96, 37, 30), (65, 40, 33)])   # x-high faces in the tile, and left to the Mur kernel
+def test_cells_equal_tiles_f16_faces(shape):
+    """fp16 faces round once or twice as the tiled step does; it takes many
+    face updates to tell."""
+    a, pa = _run(shape, F.STORE_F16, 90, False)
+    b, pb = _run(shape, F.STORE_F16, 90, True)
+    for key in a:
+        assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
+
+
+@pytest.mark.parametrize("shape", [(3, 9, 5), (33, 20, 11), (64, 24, 9)])
+def test_cells_equal_the_oracle(shape):
+    from oracle import oracle as O
+    rng = np.random.default_rng(list(shape))
+    nx, ny, nz = shape
+    table = np.asarray([(0.0, 1.0, 1.0, 0.0), (0.8, 55.0, 40.0, 8e-12)], np.float32)
+    ids = rng.integers(0, 2, (nz, ny, nx)).astype(np.uint8)
+    src, jz = np.asarray([(1, 2, 1), (nx - 1, ny - 1, nz - 1)], np.int32), rng.uniform(-1, 1, 9).astype(np.float32)
+    probes = _probes(shape)
+    ctx = F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0))
+    ctx.set_materials(ids, table)
+    ctx.set_sources(src, jz)
+    ctx.set_probes(probes, 9)
+    sim = O.Sim(shape, DT, DX, DX, DX, MU0, EPS0, prec=32)
+    t = table[ids.astype(np.int64)]
+    sim.set_materials(t[..., 0], t[..., 1], t[..., 2], t[..., 3])
+    sim.set_sources(src, jz, jz_mode=1)
+    for f in range(9):                          # random start: every operand non-zero
+        for lv in ([0] if 3 <= f < 6 else [0, 1, 2]):
+            v = rng.uniform(-1, 1, (nz, ny, nx)).astype(np.float32)
+            ctx.set(f, lv, v)
+            sim.set(f, lv, v)
+    ctx.run(9)
+    ref = sim.run(9, probes)
+    for f in range(9):
+        for lv in ([0] if 3 <= f < 6 else [0, 1, 2]):
+            a, b = ctx.get(f, lv), sim.get(f, lv)
+            assert bits_equal(a, b), f"{F.FIELDS[f]} level {lv}: {first_diff(a, b)}"
+    assert np.array_equal(ctx.probes().astype(np.float32).view(np.uint32), ref.astype(np.float32).view(np.uint32))
