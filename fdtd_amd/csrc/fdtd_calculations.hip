@@ -7,8 +7,8 @@
 // division).  Built with -ffp-contract=off, they are bit-identical to a
 // straight C evaluation of the reference's equations.
 //
-// Launch geometry is the library's: one lane per cell over the flattened
-// grid, 256 lanes per block, so every lane of a wave64 is busy whatever nx is
+// Launch geometry is the library's: lanes over the flattened planes or grid,
+// 256 lanes per block, so every lane of a wave64 is busy whatever nx is
 // (the reference's (128,1,1) blocks leave half the lanes idle at nx = 64).
 #include <hip/hip_runtime.h>
 
@@ -26,62 +26,139 @@ struct LegacyParams {
     int nsrc;
     int njz;
     int debye_mode;
+    // from the host: dt/(mu0*d), dt/d per axis, rounded as the reference's
+    // float expressions, and the multiplies that divide by nx and nx*ny
+    float chx, chy, chz, cdx, cdy, cdz;
+    uint32_t nx_mul, nx_shift, nxy_mul, nxy_shift;
 };
 
 __constant__ LegacyParams c_p;
 __constant__ int c_sources[D_MAX_SOURCES * 3];
 __constant__ float c_jz[D_MAX_JZ];
 
-LegacyParams h_p = {0, 0, 0, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0, 0, FDTD_DEBYE_FIXED};
+LegacyParams h_p = {0, 0, 0, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0, 0, FDTD_DEBYE_FIXED, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0, 0, 0, 0};
 bool h_params_set = false;
 
 constexpr int kBlock = 256;
 
-__device__ inline bool cell_of(long long q, const LegacyParams &p, int &i, int &j, int &k)
+// A cell number (Q: uint32_t, or size_t for grids of 2^32 cells and more) is
+// divided by nx and nx*ny with a multiply each (exact for every 32-bit number:
+// m = floor(2^32 (2^s - d) / d) + 1, s = ceil(log2 d)); two 64-bit divisions
+// cost more instructions than the whole H update.
+__device__ __forceinline__ uint32_t div_by(uint32_t q, uint32_t mul, uint32_t shift)
 {
-    const long long nxy = (long long)p.nx * p.ny;
-    if (q >= nxy * p.nz) return false;
-    k = (int)(q / nxy);
-    const long long r = q - (long long)k * nxy;
-    j = (int)(r / p.nx);
-    i = (int)(r - (long long)j * p.nx);
-    return true;
+    const uint32_t t = __umulhi(mul, q);
+    return (t + ((q - t) >> 1)) >> shift;
 }
 
+template <typename Q>
+__device__ __forceinline__ int row_of(const LegacyParams &p, Q q)   // q / nx
+{
+    if constexpr (sizeof(Q) == 4) return (int)div_by(q, p.nx_mul, p.nx_shift);
+    else return (int)(q / (Q)p.nx);
+}
+
+// Plane pairs over blockIdx.y, in groups of kPairs over blockIdx.z (H and D).
+constexpr int kPairs = 32768;
+
+// A load that the compiler does not merge with its neighbour's (a wave's
+// 8-byte load takes three times the address unit's cycles of a 4-byte one).
+template <typename Q>
+__device__ __forceinline__ float ld(const float *p, Q q)
+{
+    return __hip_atomic_load(p + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// Own-cell operands and results: streaming ones (ST) where the grid's arrays
+// exceed the Infinity Cache.
+template <bool ST, typename Q>
+__device__ __forceinline__ float ld_own(const float *p, Q q)
+{
+    if (ST) return __builtin_nontemporal_load(p + q);
+    return ld(p, q);
+}
+template <bool ST, typename Q>
+__device__ __forceinline__ void st_own(float *p, Q q, float v)
+{
+    if (ST) __builtin_nontemporal_store(v, p + q);
+    else p[q] = v;
+}
+
+// H and D: one lane per pair of cells one above the other, so that a plane's
+// values serve as the next one's neighbours, and every load of the two ahead
+// of the first use, with neighbours outside the grid clamped to the cell
+// (those updates are masked).  100^3 in the Infinity Cache on MI355X (us): H
+// 7.7 -> 5.8, D 8.8 -> 6.4 against one component after another's loads; with
+// one cell per lane 6.8 and 9.0.
+
 // fdtd_calculations.cu:32-77
+template <typename Q, bool ST>
 __global__ __launch_bounds__(kBlock) void legacy_h(float *hx, float *hy, float *hz, const float *ex, const float *ey,
                                                    const float *ez)
 {
-    const LegacyParams p = c_p;
-    int i, j, k;
-    const long long o = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (!cell_of(o, p, i, j, k)) return;
-    const long long sy = p.nx, sz = (long long)p.nx * p.ny;
-    if (i >= 1 && i < p.nx - 1 && j < p.ny - 1 && k < p.nz - 1)
-        hx[o] = hx[o] - p.dt / (p.mu0 * p.dy) * (ez[o + sy] - ez[o]) + p.dt / (p.mu0 * p.dy) * (ey[o + sz] - ey[o]);
-    if (i < p.nx - 1 && j >= 1 && j < p.ny - 1 && k < p.nz - 1)
-        hy[o] = hy[o] - p.dt / (p.mu0 * p.dz) * (ex[o + sz] - ex[o]) + p.dt / (p.mu0 * p.dx) * (ez[o + 1] - ez[o]);
-    if (i < p.nx - 1 && j < p.ny - 1 && k >= 1 && k < p.nz - 1)
-        hz[o] = hz[o] - p.dt / (p.mu0 * p.dx) * (ey[o + 1] - ey[o]) + p.dt / (p.mu0 * p.dy) * (ex[o + sy] - ex[o]);
+    const LegacyParams &p = c_p;
+    const Q nxy = (Q)p.nx * (Q)p.ny, q = blockIdx.x * (Q)kBlock + threadIdx.x;
+    const int k0 = (int)(blockIdx.z * kPairs + blockIdx.y) * 2;
+    if (q >= nxy || k0 >= p.nz) return;
+    const int j = row_of(p, q), i = (int)(q - (Q)j * (Q)p.nx);
+    const bool ip = i < p.nx - 1, jp = j < p.ny - 1;
+    const Q qi = ip ? q + 1 : q, qj = jp ? q + (Q)p.nx : q;
+    float hx0[2], hy0[2], hz0[2], x[3], y[3], z[2], xj[2], yi[2], zi[2], zj[2];
+#pragma unroll
+    for (int h = 0; h < 3; h++) {
+        const size_t o = (size_t)min(k0 + h, p.nz - 1) * nxy;
+        x[h] = ld(ex + o, q); y[h] = ld(ey + o, q);
+        if (h < 2) {
+            z[h] = ld(ez + o, q);
+            hx0[h] = ld_own<ST>(hx + o, q); hy0[h] = ld_own<ST>(hy + o, q); hz0[h] = ld_own<ST>(hz + o, q);
+            xj[h] = ld(ex + o, qj); yi[h] = ld(ey + o, qi); zi[h] = ld(ez + o, qi); zj[h] = ld(ez + o, qj);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int k = k0 + h;
+        if (k >= p.nz - 1) break;   // no component of the last plane is updated
+        const size_t o = (size_t)k * nxy;
+        if (i >= 1 && ip && jp) st_own<ST>(hx + o, q, hx0[h] - p.chy * (zj[h] - z[h]) + p.chy * (y[h + 1] - y[h]));
+        if (ip && j >= 1 && jp) st_own<ST>(hy + o, q, hy0[h] - p.chz * (x[h + 1] - x[h]) + p.chx * (zi[h] - z[h]));
+        if (ip && jp && k >= 1) st_own<ST>(hz + o, q, hz0[h] - p.chx * (yi[h] - y[h]) + p.chy * (xj[h] - x[h]));
+    }
 }
 
 // fdtd_calculations.cu:80-122
+template <typename Q, bool ST>
 __global__ __launch_bounds__(kBlock) void legacy_d(float *dxT, float *dyT, float *dzT, const float *dxS,
                                                    const float *dyS, const float *dzS, const float *hx,
                                                    const float *hy, const float *hz)
 {
-    const LegacyParams p = c_p;
-    int i, j, k;
-    const long long o = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (!cell_of(o, p, i, j, k)) return;
-    const long long sy = p.nx, sz = (long long)p.nx * p.ny;
-    const float x = p.dt / p.dx, y = p.dt / p.dy, z = p.dt / p.dz;
-    if (i < p.nx - 1 && j >= 1 && j < p.ny - 1 && k >= 1 && k < p.nz - 1)
-        dxT[o] = dxS[o] + y * (hz[o] - hz[o - sy]) - z * (hy[o] - hy[o - sz]);
-    if (i >= 1 && i < p.nx - 1 && j < p.ny - 1 && k >= 1 && k < p.nz - 1)
-        dyT[o] = dyS[o] + z * (hx[o] - hx[o - sz]) - x * (hz[o] - hz[o - 1]);
-    if (i >= 1 && i < p.nx - 1 && j >= 1 && j < p.ny - 1 && k < p.nz - 1)
-        dzT[o] = dzS[o] + x * (hy[o] - hy[o - 1]) - y * (hx[o] - hx[o - sy]);
+    const LegacyParams &p = c_p;
+    const Q nxy = (Q)p.nx * (Q)p.ny, q = blockIdx.x * (Q)kBlock + threadIdx.x;
+    const int k0 = (int)(blockIdx.z * kPairs + blockIdx.y) * 2;
+    if (q >= nxy || k0 >= p.nz) return;
+    const int j = row_of(p, q), i = (int)(q - (Q)j * (Q)p.nx);
+    const bool ip = i < p.nx - 1, jp = j < p.ny - 1, i1 = i >= 1, j1 = j >= 1;
+    const Q qi = i1 ? q - 1 : q, qj = j1 ? q - (Q)p.nx : q;
+    float dx[2], dy[2], dz[2], x[3], y[3], z[2], xj[2], yi[2], zi[2], zj[2];   // x[h], y[h]: plane k0 + h - 1
+#pragma unroll
+    for (int h = -1; h < 2; h++) {
+        const size_t o = (size_t)max(min(k0 + h, p.nz - 1), 0) * nxy;
+        x[h + 1] = ld(hx + o, q); y[h + 1] = ld(hy + o, q);
+        if (h >= 0) {
+            z[h] = ld(hz + o, q);
+            dx[h] = ld_own<ST>(dxS + o, q); dy[h] = ld_own<ST>(dyS + o, q); dz[h] = ld_own<ST>(dzS + o, q);
+            xj[h] = ld(hx + o, qj); yi[h] = ld(hy + o, qi); zi[h] = ld(hz + o, qi); zj[h] = ld(hz + o, qj);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int k = k0 + h;
+        if (k >= p.nz - 1) break;   // no component of the last plane is updated
+        const bool k1 = k >= 1;
+        const size_t o = (size_t)k * nxy;
+        if (ip && j1 && jp && k1) st_own<ST>(dxT + o, q, dx[h] + p.cdy * (z[h] - zj[h]) - p.cdz * (y[h + 1] - y[h]));
+        if (i1 && ip && jp && k1) st_own<ST>(dyT + o, q, dy[h] + p.cdz * (x[h + 1] - x[h]) - p.cdx * (z[h] - zi[h]));
+        if (i1 && ip && j1 && jp) st_own<ST>(dzT + o, q, dz[h] + p.cdx * (y[h + 1] - yi[h]) - p.cdy * (x[h + 1] - xj[h]));
+    }
 }
 
 // fdtd_calculations.cu:187-213: one lane per listed source.
@@ -110,6 +187,7 @@ __device__ inline float e_update(float c, float d, float a, double g1, double g2
 }
 
 // fdtd_calculations.cu:125-184
+template <typename Q, bool ST>
 __global__ __launch_bounds__(kBlock) void legacy_e(float *exT, float *eyT, float *ezT, const float *ex0,
                                                    const float *ey0, const float *ez0, const float *ex1,
                                                    const float *ey1, const float *ez1, const float *dx0,
@@ -118,33 +196,46 @@ __global__ __launch_bounds__(kBlock) void legacy_e(float *exT, float *eyT, float
                                                    const float *dy2, const float *dz2, const float *sigma,
                                                    const float *epsI, const float *epsS, const float *tauD)
 {
-    const LegacyParams p = c_p;
-    int i, j, k;
-    const long long o = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (!cell_of(o, p, i, j, k)) return;
-    const bool ux = (i < p.nx - 1 && j >= 1 && j < p.ny - 1 && k >= 1 && k < p.nz - 1);
-    const bool uyz = (i >= 1 && k >= 1);
+    // one lane per cell of the flattened grid: every wave's 19 streams move whole lines whatever nx*ny is (14.6 us
+    // at 100^3 with the lanes numbered from each plane's start, 13.6 so)
+    const LegacyParams &p = c_p;
+    const Q nxy = (Q)p.nx * (Q)p.ny, o = blockIdx.x * (Q)kBlock + threadIdx.x;
+    if (o >= nxy * (Q)p.nz) return;
+    int k;
+    if constexpr (sizeof(Q) == 4) k = (int)div_by(o, p.nxy_mul, p.nxy_shift);
+    else k = (int)(o / nxy);
+    const Q r = o - (Q)k * nxy;
+    const int j = row_of(p, r), i = (int)(r - (Q)j * (Q)p.nx);
+    const bool ux = i < p.nx - 1 && j >= 1 && j < p.ny - 1 && k >= 1 && k < p.nz - 1;
+    const bool uyz = i >= 1 && k >= 1;
     if (!ux && !uyz) return;
-    const float sg = sigma[o], ei = epsI[o], es = epsS[o], tau = tauD[o];
+    auto v = [&](const float *a) { return ST ? __builtin_nontemporal_load(a + o) : a[o]; };
+    const float sg = v(sigma), ei = v(epsI), es = v(epsS), tau = v(tauD);
     const float dt = p.dt, e0 = p.eps0;
     const float a = 2.0 * e0 * ei * tau;
     const float b = a + 2.0 * dt * (e0 * es + sg * tau);
-    const float c = 1.0 / (b + sg * dt * dt);
+    const float cc = 1.0 / (b + sg * dt * dt);
     const float d = (p.debye_mode == FDTD_DEBYE_REF) ? (float)(2.0 * b - sg * dt * dt)
                                                       : (float)((double)a + (double)b - (double)(sg * dt * dt));
     const double g1 = 2.0 * (dt + tau);
     const double g2 = 2.0 * dt + 4.0 * tau;
     const double g3 = 2.0 * tau;
-    if (ux) exT[o] = e_update(c, d, a, g1, g2, g3, ex0[o], ex1[o], dx0[o], dx1[o], dx2[o]);
+    if (ux) st_own<ST>(exT, o, e_update(cc, d, a, g1, g2, g3, v(ex0), v(ex1), v(dx0), v(dx1), v(dx2)));
     if (uyz) {
-        eyT[o] = e_update(c, d, a, g1, g2, g3, ey0[o], ey1[o], dy0[o], dy1[o], dy2[o]);
-        ezT[o] = e_update(c, d, a, g1, g2, g3, ez0[o], ez1[o], dz0[o], dz1[o], dz2[o]);
+        st_own<ST>(eyT, o, e_update(cc, d, a, g1, g2, g3, v(ey0), v(ey1), v(dy0), v(dy1), v(dy2)));
+        st_own<ST>(ezT, o, e_update(cc, d, a, g1, g2, g3, v(ez0), v(ez1), v(dz0), v(dz1), v(dz2)));
     }
 }
 
 inline int set_err(hipError_t e) { return (int)e; }
 
 }  // namespace
+
+// Streaming operands where the 25 arrays of the reference's FdtdField exceed
+// the Infinity Cache (us per call, cached -> streaming): 160^3 (410 MB) E 63.7
+// -> 57.6; 256^3 H 122.9 -> 95.2, D 132 -> 99, E 276 -> 248.
+static inline bool streaming() { return 100LL * h_p.nx * h_p.ny * h_p.nz > (256LL << 20); }
+static inline bool wide() { return (long long)h_p.nx * h_p.ny * h_p.nz >= (1LL << 32); }
 
 extern "C" int fdtdSetDebyeMode(int mode)
 {
@@ -162,6 +253,16 @@ extern "C" int copySymbolsToDevice(FdtdParams *params)
     h_p.nx = params->nx; h_p.ny = params->ny; h_p.nz = params->nz;
     h_p.dt = params->dt; h_p.dx = params->dx; h_p.dy = params->dy; h_p.dz = params->dz;
     h_p.mu0 = params->mu0; h_p.eps0 = params->eps0;
+    h_p.chx = h_p.dt / (h_p.mu0 * h_p.dx); h_p.chy = h_p.dt / (h_p.mu0 * h_p.dy); h_p.chz = h_p.dt / (h_p.mu0 * h_p.dz);
+    h_p.cdx = h_p.dt / h_p.dx; h_p.cdy = h_p.dt / h_p.dy; h_p.cdz = h_p.dt / h_p.dz;
+    auto divisor = [](unsigned long long d, uint32_t &mul, uint32_t &shift) {   // 2 <= d < 2^32 (div_by)
+        uint32_t s = 0;
+        while ((1ull << s) < d) s++;
+        mul = (uint32_t)((((1ull << s) - d) << 32) / d + 1);
+        shift = s - 1;
+    };
+    divisor(h_p.nx, h_p.nx_mul, h_p.nx_shift);
+    if (!wide()) divisor((unsigned long long)h_p.nx * h_p.ny, h_p.nxy_mul, h_p.nxy_shift);
     const int ns = std::max(0, std::min(D_MAX_SOURCES, params->sourcesCount));
     const int nj = std::max(0, std::min(D_MAX_JZ, params->jzCount));
     for (int s = 0; s < ns; s++)
@@ -186,11 +287,20 @@ static inline dim3 flat_grid()
     return dim3((unsigned)((n + kBlock - 1) / kBlock));
 }
 
+static inline dim3 pair_grid()
+{
+    const long long n = (long long)h_p.nx * h_p.ny;
+    const int pairs = h_p.nz / 2 + h_p.nz % 2;
+    return dim3((unsigned)((n + kBlock - 1) / kBlock), (unsigned)std::min(pairs, kPairs),
+                (unsigned)((pairs + kPairs - 1) / kPairs));
+}
+
 extern "C" int updateHField(float *hx, float *hy, float *hz, float *exSource, float *eySource, float *ezSource,
                             hipStream_t stream)
 {
     if (!h_params_set) return FDTD_ESTATE;
-    legacy_h<<<flat_grid(), kBlock, 0, stream>>>(hx, hy, hz, exSource, eySource, ezSource);
+    (wide() ? legacy_h<size_t, true> : streaming() ? legacy_h<uint32_t, true> : legacy_h<uint32_t, false>)
+        <<<pair_grid(), kBlock, 0, stream>>>(hx, hy, hz, exSource, eySource, ezSource);
     return set_err(hipGetLastError());
 }
 
@@ -198,8 +308,8 @@ extern "C" int updateDField(float *dxTarget, float *dyTarget, float *dzTarget, f
                             float *dzSource, float *hx, float *hy, float *hz, hipStream_t stream)
 {
     if (!h_params_set) return FDTD_ESTATE;
-    legacy_d<<<flat_grid(), kBlock, 0, stream>>>(dxTarget, dyTarget, dzTarget, dxSource, dySource, dzSource, hx, hy,
-                                                 hz);
+    (wide() ? legacy_d<size_t, true> : streaming() ? legacy_d<uint32_t, true> : legacy_d<uint32_t, false>)
+        <<<pair_grid(), kBlock, 0, stream>>>(dxTarget, dyTarget, dzTarget, dxSource, dySource, dzSource, hx, hy, hz);
     return set_err(hipGetLastError());
 }
 
@@ -210,10 +320,8 @@ extern "C" int updateEField(float *exTarget, float *eyTarget, float *ezTarget, f
                             float *epsS, float *tauD, hipStream_t stream)
 {
     if (!h_params_set) return FDTD_ESTATE;
-    legacy_e<<<flat_grid(), kBlock, 0, stream>>>(exTarget, eyTarget, ezTarget, exSource0, eySource0, ezSource0,
-                                                 exSource1, eySource1, ezSource1, dxSource0, dySource0, dzSource0,
-                                                 dxSource1, dySource1, dzSource1, dxSource2, dySource2, dzSource2,
-                                                 sigma, epsI, epsS, tauD);
+    (wide() ? legacy_e<size_t, true> : streaming() ? legacy_e<uint32_t, true> : legacy_e<uint32_t, false>)
+        <<<flat_grid(), kBlock, 0, stream>>>(exTarget, eyTarget, ezTarget, exSource0, eySource0, ezSource0, exSource1, eySource1, ezSource1, dxSource0, dySource0, dzSource0, dxSource1, dySource1, dzSource1, dxSource2, dySource2, dzSource2, sigma, epsI, epsS, tauD);
     return set_err(hipGetLastError());
 }
 
