@@ -286,6 +286,7 @@ struct SnapArgs {
     float *out;
     int nx, ny, nz, pitch;
     long long plane;
+    uint32_t nx_mul, nx_shift;     // t / nx = (m + ((t - m) >> 1)) >> nx_shift, m = hi32(nx_mul * t); set at launch
 };
 hipError_t launch_snapshot(const SnapArgs &a, int storage, hipStream_t s);
 // Mur faces and one probe row in one launch (p.nprobe = 0: faces only).  The
