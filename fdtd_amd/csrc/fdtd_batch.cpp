@@ -1,7 +1,9 @@
 // Batches of independent grids (fdtd_amd.h, fdtd_batch_*): one device arena
-// holds every grid's state; each batch step is one persistent fused launch
-// per storage form present, one Mur launch and one probe launch over all
-// running grids.  The launches read the grids' descriptors, the per-form
+// holds every grid's state.  Small grids are stepped in groups whose state
+// fits the Infinity Cache, one launch per group and step (cell_batch), many
+// steps of a group in a row.  The others take one persistent fused launch per
+// storage form present, one Mur launch and one probe launch per step over all
+// of them.  The launches read the grids' descriptors, the per-form
 // tile lists and a step counter from device memory, so a sequence of steps
 // is captured once per (tile rows, forms present, length) as a HIP graph and
 // replayed while grids join and leave; the host re-uploads the tables
@@ -28,8 +30,19 @@ size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 struct DevTables {
     BatchInst inst[kBatchMaxInst];
     BatchClass cls[kBatchClasses];
+    CellInst cell[kBatchMaxInst];
+    CellGroups groups;
     BatchShared sh;
 };
+
+// Padded state of the grids that cell_batch steps together, and the steps it
+// takes with one group before it goes on to the next: a group's state stays
+// in the Infinity Cache (256 MB) meanwhile.  Twelve fp32 grids around 96^3
+// (1.1 GB) on MI355X, in Gcell-updates/s: 51.5 as set; 45.3 with groups of
+// 120 MB, 48.8 with 180, 42.3 with 300, 38.3 with 400; 45.6 with 8 steps at a
+// time, 52.6 with 64; 38.8 where field_step_batch steps all of them together.
+constexpr size_t kCellGroupBytes = 240000000;
+constexpr int kCellRunSteps = 32;
 
 // Byte layout of one grid's arena region.
 struct Layout {
@@ -176,6 +189,7 @@ struct fdtd_batch {
         size_t off = 0;
         Layout L;
         BatchInst d;
+        CellInst c;
         long long start = 0;
         int steps = 0;
         double sE = 1, sD = 1, sH = 1;
@@ -188,6 +202,9 @@ struct fdtd_batch {
     bool dirty = true;                 // device tables out of date
     std::vector<int> running;          // slots in the device tables
     int mask = 0;                      // kernel classes in the device tables
+    bool by_cell = true;               // small grids step by cell_batch, the others in tiles
+    struct Group { int first, count, blocks, storage; };
+    std::vector<Group> groups;         // of the device tables
     int grid[kBatchClasses] = {};
     int tiles[kBatchClasses] = {};
     long long cells[kBatchClasses] = {};
@@ -221,6 +238,52 @@ bool is_running(const fdtd_batch *b, int s)
     return I.used && b->step - I.start < I.steps;
 }
 
+// Whether cell_batch steps the grid: as a context's default_cell.
+bool cell_grid(const fdtd_batch *b, const fdtd_batch::Inst &I)
+{
+    return b->by_cell && I.d.nz <= kCellMaxPlanes && 24 * I.L.Np * I.L.esz <= cell_state_limit(I.L.esz);
+}
+
+// Groups of the grids `cell` whose state fits kCellGroupBytes together (one
+// larger grid makes a group), storage by storage, largest first; fills the
+// group tables.
+void make_groups(fdtd_batch *b, std::vector<int> cell, DevTables *T)
+{
+    b->groups.clear();
+    auto bytes = [&](int s) { return 24 * b->in[s].L.Np * b->in[s].L.esz; };
+    std::sort(cell.begin(), cell.end(), [&](int p, int q) {
+        const int sp = b->in[p].d.storage, sq = b->in[q].d.storage;
+        if (sp != sq) return sp < sq;
+        return bytes(p) != bytes(q) ? bytes(p) > bytes(q) : p < q;
+    });
+    std::vector<std::vector<int>> bins;
+    std::vector<size_t> room;
+    size_t open = 0;   // first bin of the storage at hand
+    for (size_t t = 0; t < cell.size(); t++) {
+        const int s = cell[t];
+        if (t > 0 && b->in[s].d.storage != b->in[cell[t - 1]].d.storage) open = bins.size();
+        size_t w = open;
+        while (w < bins.size() && room[w] < bytes(s)) w++;
+        if (w == bins.size()) {
+            bins.push_back({});
+            room.push_back(std::max(kCellGroupBytes, bytes(s)));
+        }
+        bins[w].push_back(s);
+        room[w] -= bytes(s);
+    }
+    int at = 0;
+    T->groups.start[0] = 0;
+    for (const auto &bin : bins) {
+        const int first = at;
+        for (int s : bin) {
+            T->groups.idx[at] = s;
+            T->groups.start[at + 1] = T->groups.start[at] + cell_blocks(b->in[s].c);
+            at++;
+        }
+        b->groups.push_back({first, at - first, T->groups.start[at] - T->groups.start[first], b->in[bin[0]].d.storage});
+    }
+}
+
 // Rebuilds the work tables for the grids running at the current step and
 // enqueues their upload on `stream` when they differ from the device's.
 int sync_tables(fdtd_batch *b, hipStream_t stream)
@@ -236,7 +299,8 @@ int sync_tables(fdtd_batch *b, hipStream_t stream)
         b->stage_pending[k] = false;
     }
     DevTables *T = b->stage[k];
-    int maxslot = -1;
+    int maxslot = -1, maxcell = -1;
+    std::vector<int> cell;
     for (int c = 0; c < kBatchClasses; c++) {
         T->cls[c].n = 0;
         T->cls[c].total = 0;
@@ -261,17 +325,26 @@ int sync_tables(fdtd_batch *b, hipStream_t stream)
         d.tiles_x = (d.nx + tw - 1) / tw;
         d.tiles_y = (d.ny + b->ty - 1) / b->ty;
         d.tiles_z = (d.nz + d.kchunk - 1) / d.kchunk;
+        const int c = batch_class(d.storage, d.cpl);
+        const int nt = d.tiles_x * d.tiles_y * d.tiles_z;
+        b->tiles[c] += nt;
+        b->cells[c] += (long long)d.nx * d.ny * d.nz;
+        if (cell_grid(b, I)) {
+            I.c.start = d.start;
+            I.c.nsteps = d.nsteps;
+            I.c.hi_once = d.mur_x == 2;
+            T->cell[s] = I.c;
+            maxcell = std::max(maxcell, s);
+            cell.push_back(s);
+            continue;
+        }
         T->inst[s] = d;
         maxslot = std::max(maxslot, s);
-        const int c = batch_class(d.storage, d.cpl);
         mask |= 1 << c;
         BatchClass &C = T->cls[c];
-        const int nt = d.tiles_x * d.tiles_y * d.tiles_z;
         C.idx[C.n] = s;
         C.total += nt;
         C.start[++C.n] = C.total;
-        b->tiles[c] += nt;
-        b->cells[c] += (long long)d.nx * d.ny * d.nz;
         const int mb = (d.mur_seg[12] + kMurBlock - 1) / kMurBlock;
         S.mur_idx[S.nmur] = s;
         S.mur_total += mb;
@@ -281,6 +354,11 @@ int sync_tables(fdtd_batch *b, hipStream_t stream)
             S.rec[S.nrec][1] = p;
             S.nrec++;
         }
+    }
+    make_groups(b, cell, T);
+    if (maxcell >= 0) {
+        HIP_TRY(hipMemcpyAsync(b->dev->cell, T->cell, sizeof(CellInst) * (maxcell + 1), hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipMemcpyAsync(&b->dev->groups, &T->groups, sizeof(T->groups), hipMemcpyHostToDevice, stream));
     }
     if (maxslot >= 0)
         HIP_TRY(hipMemcpyAsync(b->dev->inst, T->inst, sizeof(BatchInst) * (maxslot + 1), hipMemcpyHostToDevice, stream));
@@ -526,6 +604,37 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     d.murx1 = d.murx0 + (size_t)ny * nz;
     // zero-term rows: exact fp32 form; batch grids start from zero fields
     d.zskip = (e.storage == FDTD_STORE_F32 && e.load_zero_terms == 0) ? 1 : 0;
+    CellInst &c = I.c;
+    memset(&c, 0, sizeof c);
+    const size_t gb = (size_t)L.guard * L.esz;
+    for (int s = 0; s < 3; s++)
+        for (int q = 0; q < 3; q++) {
+            c.E[s][q] = (char *)d.E[s][q] - gb;
+            c.D[s][q] = (char *)d.D[s][q] - gb;
+            if (s < 2) c.H[s][q] = (char *)d.H[s][q] - gb;
+        }
+    c.ids = d.ids - L.guard;
+    c.lut = d.lut;
+    c.jz = d.jz;
+    for (int r = 0; r < 6; r++) c.rp[r] = d.rp[r];
+    c.murx0 = d.murx0;
+    c.murx1 = d.murx1;
+    c.probes = d.probes;
+    c.probe_out = d.probe_out;
+    for (int f = 0; f < 9; f++) c.factor[f] = d.factor[f];
+    c.nx = nx; c.ny = ny; c.nz = nz;
+    c.o0 = (uint32_t)gb;
+    c.sy = (uint32_t)(L.pitch * L.esz);
+    c.sz = (uint32_t)(L.plane * L.esz);
+    cell_tiles(nx, ny, c);
+    for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
+    c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : 0;
+    c.nprobe = d.nprobe;
+    c.probe_rows = d.probe_rows;
+    c.jz_len = d.jz_len;
+    c.jz_hold3 = d.jz_hold3;
+    c.dt = d.dt; c.mu0 = d.mu0; c.eps0 = d.eps0;
+    c.h[0] = d.hx; c.h[1] = d.hy; c.h[2] = d.hz;
     I.start = b->step;
     I.used = true;
     b->dirty = true;
@@ -556,8 +665,8 @@ extern "C" int fdtd_batch_run(fdtd_batch *b, int steps, hipStream_t stream)
     if (b->step + steps >= INT_MAX) return fdtd_fail(FDTD_ERANGE, "batch step counter would overflow");
     int left = steps;
     while (left > 0) {
-        const int g = std::min(left, b->graph_steps);
         if (int rc = sync_tables(b, stream)) return rc;
+        const int g = std::min(left, b->mask ? b->graph_steps : std::max(b->graph_steps, kCellRunSteps));
         if (b->running.empty()) {
             // nothing runs: the counter moves on the host; the next table
             // upload carries it to the device
@@ -565,11 +674,17 @@ extern "C" int fdtd_batch_run(fdtd_batch *b, int steps, hipStream_t stream)
             b->dirty = true;
             break;
         }
-        hipGraphExec_t exec = nullptr;
-        if (int rc = graph_for(b, b->mask, g, &exec)) return rc;
-        HIP_TRY(hipGraphLaunch(exec, stream));
         b->ran = true;
         b->last = stream;
+        if (b->mask) {
+            hipGraphExec_t exec = nullptr;
+            if (int rc = graph_for(b, b->mask, g, &exec)) return rc;
+            HIP_TRY(hipGraphLaunch(exec, stream));
+        }
+        for (const auto &G : b->groups)
+            for (int t = 0; t < g; t++)
+                HIP_TRY(launch_cell_batch(b->dev->cell, &b->dev->groups, G.first, G.count, G.blocks, (int)b->step + t,
+                                          G.storage, stream));
         b->step += g;
         left -= g;
     }
@@ -650,6 +765,7 @@ extern "C" int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int g
     if (kchunk < 0 || graph_steps < 0) return fdtd_fail(FDTD_EINVAL, "negative kchunk/graph_steps");
     if (tile_y) b->ty = tile_y;
     if (kchunk) b->kchunk = kchunk;
+    if (tile_y || kchunk) b->by_cell = false;
     if (graph_steps) b->graph_steps = graph_steps;
     b->dirty = true;
     return 0;
@@ -683,26 +799,40 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
     const int tys[3] = {2, 4, 8}, kcs[5] = {3, 4, 6, 8, 16};
     float best = 0.0f;
     int bty = b->ty, bkc = b->kchunk;
+    auto trial = [&](int n) -> float {   // ms per step over n steps as the batch is set up now
+        b->dirty = true;
+        rc = fdtd_batch_run(b, 2, stream);  // builds the graphs, uploads the tables
+        if (rc) return 0.0f;
+        e = hipEventRecord(t0, stream);
+        if (e == hipSuccess) rc = fdtd_batch_run(b, n, stream);
+        if (!rc && e == hipSuccess) e = hipEventRecord(t1, stream);
+        if (!rc && e == hipSuccess) e = hipEventSynchronize(t1);
+        float ms = 0.0f;
+        if (!rc && e == hipSuccess) e = hipEventElapsedTime(&ms, t0, t1);
+        if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune timing");
+        return ms / n;
+    };
+    b->by_cell = false;
     for (int a = 0; a < 3 && !rc; a++)
         for (int c = 0; c < 5 && !rc; c++) {
             b->ty = tys[a];
             b->kchunk = kcs[c];
-            b->dirty = true;
-            rc = fdtd_batch_run(b, 2, stream);  // builds the graphs, uploads the tables
-            if (rc) break;
-            e = hipEventRecord(t0, stream);
-            if (e == hipSuccess) rc = fdtd_batch_run(b, trial_steps, stream);
-            if (!rc && e == hipSuccess) e = hipEventRecord(t1, stream);
-            if (!rc && e == hipSuccess) e = hipEventSynchronize(t1);
-            float ms = 0.0f;
-            if (!rc && e == hipSuccess) e = hipEventElapsedTime(&ms, t0, t1);
-            if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune timing");
+            const float ms = trial(trial_steps);
             if (!rc && (best == 0.0f || ms < best)) {
                 best = ms;
                 bty = tys[a];
                 bkc = kcs[c];
             }
         }
+    bool bcells = false;
+    if (!rc) {
+        b->by_cell = true;
+        b->ty = bty;
+        b->kchunk = bkc;
+        const float ms = trial(std::max(trial_steps, kCellRunSteps));   // each group's steps in a row, as a run takes them
+        bcells = !rc && ms < best;
+    }
+    b->by_cell = bcells;
     if (t0) (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);
     // Back to the zero initial state at step0 with the fastest shape.

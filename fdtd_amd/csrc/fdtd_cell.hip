@@ -98,6 +98,116 @@ __device__ __forceinline__ float mur_round(float q, float x, bool once)
     return Elem<T>::rnd(v);
 }
 
+// The Mur coefficients of a face cell (launch_mur_coefs).
+__device__ __forceinline__ float4 mur_coef(float dt, float h, float m0, float e0, float rpf, float rpn)
+{
+    const float sf = sqrtf(m0 * e0 * rpf), sn = sqrtf(m0 * e0 * rpn);
+    float4 c;
+    c.x = 1 / (dt + h * sf);
+    c.y = dt - h * sn;
+    c.z = dt + h * sn;
+    c.w = dt - h * sf;
+    return c;
+}
+
+// The operands of one grid's step from kernel arguments.
+struct OneStep {
+    const CellArgs &a;
+    __device__ __forceinline__ int nx() const { return a.nx; }
+    __device__ __forceinline__ int ny() const { return a.ny; }
+    __device__ __forceinline__ int nz() const { return a.nz; }
+    __device__ __forceinline__ uint32_t o0() const { return a.o0; }
+    __device__ __forceinline__ uint32_t sy() const { return a.sy; }
+    __device__ __forceinline__ uint32_t sz() const { return a.sz; }
+    __device__ __forceinline__ int tiles_x() const { return a.tiles_x; }
+    __device__ __forceinline__ int tiles() const { return a.tiles; }
+    __device__ __forceinline__ int run() const { return a.run; }
+    __device__ __forceinline__ uint32_t tx_mul() const { return a.tx_mul; }
+    __device__ __forceinline__ const uint8_t * ids() const { return a.ids; }
+    __device__ __forceinline__ const MatCoef * lut() const { return a.lut; }
+    __device__ __forceinline__ float ch(int q) const { return a.ch[q]; }
+    __device__ __forceinline__ float cd(int q) const { return a.cd[q]; }
+    __device__ __forceinline__ uint32_t zmask() const { return a.zmask; }
+    __device__ __forceinline__ int hi_once() const { return a.hi_once; }
+    __device__ __forceinline__ const char * e0(int q) const { return a.e0[q]; }
+    __device__ __forceinline__ const char * e1(int q) const { return a.e1[q]; }
+    __device__ __forceinline__ const char * d0(int q) const { return a.d0[q]; }
+    __device__ __forceinline__ const char * d1(int q) const { return a.d1[q]; }
+    __device__ __forceinline__ const char * h0(int q) const { return a.h0[q]; }
+    __device__ __forceinline__ char * eT(int q) const { return a.eT[q]; }
+    __device__ __forceinline__ char * dT(int q) const { return a.dT[q]; }
+    __device__ __forceinline__ char * h1(int q) const { return a.h1[q]; }
+    __device__ __forceinline__ float jz() const { return a.jz; }
+    __device__ __forceinline__ int nprobe() const { return a.p.nprobe; }
+    __device__ __forceinline__ const int * probes() const { return a.p.probes; }
+    // coefficients of the face (0, 1: x low, high; 2, 3: y; 4, 5: z) beside cell (i, j, k)
+    __device__ __forceinline__ float4 coef(int f, int i, int j, int k) const
+    {
+        const long long c = f < 2 ? (long long)k * a.ny + j : f < 4 ? (long long)k * a.nx + i : (long long)j * a.nx + i;
+        const float4 *p = f == 0 ? a.mur[0] : f == 1 ? a.mur[1] : f == 2 ? a.mur[2] : f == 3 ? a.mur[3] : f == 4 ? a.mur[4] : a.mur[5];
+        return p[c];
+    }
+    __device__ __forceinline__ void record(int probe, int field, float v) const
+    {
+        a.p.out[(long long)a.p.row * a.p.nprobe + probe] = (double)v * a.p.factor[field];
+    }
+};
+
+// The same of a batch's grid at its step n, from its descriptor: the ring
+// slot and H buffer roles follow n as a single grid's do.  The y and z faces'
+// coefficients come from the rp planes (a batch keeps no table of them).
+template <typename V> using Const = const __attribute__((address_space(4))) V;
+struct BatchStep {
+    Const<CellInst> *d;
+    int s0, s1, sT, hb;     // slots of levels n, n-1, n+1; buffer of H^{n-1/2}
+    int n;
+    __device__ __forceinline__ int nx() const { return d->nx; }
+    __device__ __forceinline__ int ny() const { return d->ny; }
+    __device__ __forceinline__ int nz() const { return d->nz; }
+    __device__ __forceinline__ uint32_t o0() const { return d->o0; }
+    __device__ __forceinline__ uint32_t sy() const { return d->sy; }
+    __device__ __forceinline__ uint32_t sz() const { return d->sz; }
+    __device__ __forceinline__ int tiles_x() const { return d->tiles_x; }
+    __device__ __forceinline__ int tiles() const { return d->tiles; }
+    __device__ __forceinline__ int run() const { return d->run; }
+    __device__ __forceinline__ uint32_t tx_mul() const { return d->tx_mul; }
+    __device__ __forceinline__ const uint8_t * ids() const { return d->ids; }
+    __device__ __forceinline__ const MatCoef * lut() const { return d->lut; }
+    __device__ __forceinline__ float ch(int q) const { return d->ch[q]; }
+    __device__ __forceinline__ float cd(int q) const { return d->cd[q]; }
+    __device__ __forceinline__ uint32_t zmask() const { return d->zmask; }
+    __device__ __forceinline__ int hi_once() const { return d->hi_once; }
+    __device__ __forceinline__ const char * e0(int q) const { return d->E[s0][q]; }
+    __device__ __forceinline__ const char * e1(int q) const { return d->E[s1][q]; }
+    __device__ __forceinline__ const char * d0(int q) const { return d->D[s0][q]; }
+    __device__ __forceinline__ const char * d1(int q) const { return d->D[s1][q]; }
+    __device__ __forceinline__ const char * h0(int q) const { return d->H[hb][q]; }
+    __device__ __forceinline__ char * eT(int q) const { return d->E[sT][q]; }
+    __device__ __forceinline__ char * dT(int q) const { return d->D[sT][q]; }
+    __device__ __forceinline__ char * h1(int q) const { return d->H[hb ^ 1][q]; }
+    __device__ __forceinline__ int nprobe() const { return d->nprobe; }
+    __device__ __forceinline__ const int * probes() const { return d->probes; }
+    __device__ __forceinline__ float jz() const
+    {
+        const int t = d->jz_hold3 ? (n / 3) * 3 : n;
+        return t < d->jz_len ? ((Const<float> *)d->jz)[t] : 0.0f;
+    }
+    __device__ __forceinline__ float4 coef(int f, int i, int j, int k) const
+    {
+        if (f < 2) return (f == 0 ? d->murx0 : d->murx1)[(long long)k * d->ny + j];
+        // the pair of cells in the reference's planes y (k, 2, i) and z (2, j, i); low faces: the first is the face
+        const long long step = f < 4 ? d->nx : (long long)d->nx * d->ny;
+        const long long at = f < 4 ? (long long)k * 2 * d->nx + i : (long long)j * d->nx + i;
+        const float *rp = f == 2 ? d->rp[1] : f == 3 ? d->rp[4] : f == 4 ? d->rp[2] : d->rp[5];
+        const float r0 = rp[at], r1 = rp[at + step];
+        return mur_coef(d->dt, f < 4 ? d->h[1] : d->h[2], d->mu0, d->eps0, f & 1 ? r1 : r0, f & 1 ? r0 : r1);
+    }
+    __device__ __forceinline__ void record(int probe, int field, float v) const
+    {
+        if (n < d->probe_rows) d->probe_out[(long long)n * d->nprobe + probe] = (double)v * d->factor[field];
+    }
+};
+
 // What a lane loads: the cell's operands and its neighbours'.  Suffixes: im,
 // ip at i-1, i+1 and so on; no suffix: the cell.
 struct Ops {
@@ -111,30 +221,31 @@ struct Ops {
     bool src;
 };
 
+// One block's cells (or, past the planes, its probes) of a grid's step.
 // BXL: log2 of the lanes of a block along x (32 or 64); the other lanes are
-// rows.  Exact form: cells whose material has a = g3 = +0 (C.zmask) do not
+// rows.  Exact form: cells whose material has a = g3 = +0 (zmask) do not
 // load E^{n-1} and D^{n-1}, as fused_tile's zero-term rows, decided per lane;
-// a context that always loads them passes zmask = 0 to the same kernel.
-template <typename T, bool EXACT, int BXL>
-__global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
+// a grid that always loads them has zmask = 0.  C: where the step's operands
+// are (OneStep, BatchStep); block bx of the 8 * C.run() of plane bz.
+template <typename T, bool EXACT, int BXL, typename G>
+__device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
 {
     using X = Elem<T>;
     constexpr uint32_t ES = sizeof(T);
     constexpr int BX = 1 << BXL, BY = kCellBlock / BX, WY = 64 / BX;
-    const int nx = C.nx, ny = C.ny, nz = C.nz;
+    const int nx = C.nx(), ny = C.ny(), nz = C.nz();
 
-    // Blocks (x, k) of plane k in 8 runs of C.run tiles, one run per XCD
-    // (workgroups go to the XCDs round-robin by id and gridDim.x is a
-    // multiple of 8), so a tile's neighbours in the plane and the same tiles
-    // of the planes around it share its L2.  Rows past nz hold the probes.
+    // Blocks (bx, k) of plane k in 8 runs of tiles, one run per XCD (workgroups
+    // go to the XCDs round-robin by id, and a plane takes a multiple of 8), so a
+    // tile's neighbours in the plane and the same tiles of the planes around it
+    // share its L2.  Rows past nz hold the probes.
     int i, j, k;
     bool own = true, deep = false, edge = false;
     int probe = -1, pf = -1, pseg = -1;      // probe: its index, field and face segment
-    const int bz = (int)blockIdx.y;
     if (bz < nz) {
-        const int t = ((int)blockIdx.x & 7) * C.run + ((int)blockIdx.x >> 3);
-        if (t >= C.tiles) return;
-        const int ty = C.tiles_x == 1 ? t : (int)__umulhi((unsigned)t, C.tx_mul), tx = t - ty * C.tiles_x;
+        const int t = (bx & 7) * C.run() + (bx >> 3);
+        if (t >= C.tiles()) return;
+        const int ty = C.tiles_x() == 1 ? t : (int)__umulhi((unsigned)t, C.tx_mul()), tx = t - ty * C.tiles_x();
         const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = (int)threadIdx.x & 63;
         const int jw = ty * BY + w * WY;     // the wave's first row
         if (jw >= ny) return;
@@ -146,10 +257,10 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
         deep = jw >= 2 && jw + WY <= ny - 2 && k >= 2 && k < nz - 2 && nx > 3;
         edge = tx == 0 || (nx - 2 >= tx * BX && nx - 2 < tx * BX + BX);
     } else {
-        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * (int)gridDim.x + (int)blockIdx.x) * (kCellBlock / 64) +
+        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * 8 * C.run() + bx) * (kCellBlock / 64) +
                                                ((int)threadIdx.x >> 6));
-        if (probe >= C.p.nprobe) return;
-        const int *q = C.p.probes + 4 * probe;
+        if (probe >= C.nprobe()) return;
+        const int *q = C.probes() + 4 * probe;
         pf = q[0]; i = q[1]; j = q[2]; k = q[3];
         if (pf >= 6) {
             int di, dj, dk;
@@ -161,12 +272,12 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
     // deep: the wave's rows and plane are at least two cells inside the y and z faces, so that of the faces only
     // those along x are near (edge: its tile holds i = 1 or nx-2)
     // Byte offset of the cell from bases that lie `guard` elements before the arrays' origins.
-    const uint32_t syb = C.sy, szb = C.sz;
-    const uint32_t o = C.o0 + (uint32_t)k * szb + (uint32_t)j * syb + (uint32_t)i * ES;
+    const uint32_t syb = C.sy(), szb = C.sz();
+    const uint32_t o = C.o0() + (uint32_t)k * szb + (uint32_t)j * syb + (uint32_t)i * ES;
     const uint32_t ojp = o + syb, ojm = o - syb, okp = o + szb, okm = o - szb;
-    const uint32_t id = C.ids[o / ES];
+    const uint32_t id = C.ids()[o / ES];
     Ops v;
-    const char *px = C.e0[0], *py = C.e0[1], *pz = C.e0[2], *qx = C.h0[0], *qy = C.h0[1], *qz = C.h0[2];
+    const char *px = C.e0(0), *py = C.e0(1), *pz = C.e0(2), *qx = C.h0(0), *qy = C.h0(1), *qz = C.h0(2);
     v.ex = at<T>(px, o); v.ey = at<T>(py, o); v.ez = at<T>(pz, o);
     v.ex_im = at<T>(px, o, -1); v.ey_im = at<T>(py, o, -1); v.ez_im = at<T>(pz, o, -1);
     v.ey_ip = at<T>(py, o, 1); v.ez_ip = at<T>(pz, o, 1);
@@ -180,12 +291,12 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
     v.hy_im = at<T>(qy, o, -1); v.hz_im = at<T>(qz, o, -1);
     v.hx_jm = at<T>(qx, ojm); v.hz_jm = at<T>(qz, ojm);
     v.hx_km = at<T>(qx, okm); v.hy_km = at<T>(qy, okm);
-    v.dx = at<T>(C.d0[0], o); v.dy = at<T>(C.d0[1], o); v.dz = at<T>(C.d0[2], o);
+    v.dx = at<T>(C.d0(0), o); v.dy = at<T>(C.d0(1), o); v.dz = at<T>(C.d0(2), o);
     float4 mc = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (deep && edge && (i == 1 || i == nx - 2)) mc = (i == 1 ? C.mur[0] : C.mur[1])[k * ny + j];
+    if (deep && edge && (i == 1 || i == nx - 2)) mc = C.coef(i == 1 ? 0 : 1, i, j, k);
     const uint32_t m = id & kMaterialMask;
     v.src = (id & kSourceBit) != 0;
-    const char *lut = (const char *)C.lut + m * (uint32_t)sizeof(MatCoef);
+    const char *lut = (const char *)C.lut() + m * (uint32_t)sizeof(MatCoef);
     if constexpr (EXACT) {
         const MatCoef *q = (const MatCoef *)lut;
         v.a = q->a; v.c = q->c; v.d = q->d;
@@ -195,15 +306,15 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
         v.k1 = q->k1; v.k2 = q->k2; v.k3 = q->k3; v.k5 = q->k5;
     }
     bool need = true;
-    if constexpr (EXACT) need = own && !(m < 32 && (C.zmask >> m & 1u));
+    if constexpr (EXACT) need = own && !(m < 32 && (C.zmask() >> m & 1u));
     v.exm = v.eym = v.ezm = v.dxm = v.dym = v.dzm = 0.0f;
     if (need) {
-        v.exm = at<T>(C.e1[0], o); v.eym = at<T>(C.e1[1], o); v.ezm = at<T>(C.e1[2], o);
-        v.dxm = at<T>(C.d1[0], o); v.dym = at<T>(C.d1[1], o); v.dzm = at<T>(C.d1[2], o);
+        v.exm = at<T>(C.e1(0), o); v.eym = at<T>(C.e1(1), o); v.ezm = at<T>(C.e1(2), o);
+        v.dxm = at<T>(C.d1(0), o); v.dym = at<T>(C.d1(1), o); v.dzm = at<T>(C.d1(2), o);
     }
 
-    const float chx = C.ch[0], chy = C.ch[1], chz = C.ch[2];
-    const float cdx = C.cd[0], cdy = C.cd[1], cdz = C.cd[2];
+    const float chx = C.ch(0), chy = C.ch(1), chz = C.ch(2);
+    const float cdx = C.cd(0), cdy = C.cd(1), cdz = C.cd(2);
     auto up_x = [&](float h, float z, float zjp, float y, float ykp) { return h - chy * (zjp - z) + chy * (ykp - y); };
     auto up_y = [&](float h, float x, float xkp, float z, float zip) { return h - chz * (xkp - x) + chx * (zip - z); };
     auto up_z = [&](float h, float y, float yip, float x, float xjp) { return h - chx * (yip - y) + chy * (xjp - x); };
@@ -230,13 +341,13 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
     const float dxu = v.dx + cdy * (hz - hz_jm) - cdz * (hy - hy_km);
     const float dyu = v.dy + cdz * (hx - hx_km) - cdx * (hz - hz_im);
     float dzu = v.dz + cdx * (hy - hy_im) - cdy * (hx - hx_jm);
-    dzu = v.src ? dzu - C.jz : dzu;
+    dzu = v.src ? dzu - C.jz() : dzu;
     float dyp = dyu, dzp = dzu;
     // E cells whose D is not updated read the target slot's value (in deep rows those are the cells of the high x
     // face, whose E the face takes over).
     if (!deep && own && reyz && !(rdy && rdz)) {
-        if (!rdy) dyp = ld(C.dT[1], o);
-        if (!rdz) dzp = ld(C.dT[2], o);
+        if (!rdy) dyp = ld(C.dT(1), o);
+        if (!rdz) dzp = ld(C.dT(2), o);
     }
 
     float exn, eyn, ezn;
@@ -250,8 +361,8 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
             const float mag = __builtin_fabsf(v.ex) + __builtin_fabsf(v.ey) + __builtin_fabsf(v.ez) +
                               __builtin_fabsf(v.dx) + __builtin_fabsf(v.dy) + __builtin_fabsf(v.dz);
             if (!need && own && (z == (int)0x80000000 || !__builtin_isfinite(mag))) {
-                v.exm = at<T>(C.e1[0], o); v.eym = at<T>(C.e1[1], o); v.ezm = at<T>(C.e1[2], o);
-                v.dxm = at<T>(C.d1[0], o); v.dym = at<T>(C.d1[1], o); v.dzm = at<T>(C.d1[2], o);
+                v.exm = at<T>(C.e1(0), o); v.eym = at<T>(C.e1(1), o); v.ezm = at<T>(C.e1(2), o);
+                v.dxm = at<T>(C.d1(0), o); v.dym = at<T>(C.d1(1), o); v.dzm = at<T>(C.d1(2), o);
             }
         }
         exn = e_update(v.c, v.d, v.a, v.g1, v.g2, v.g3, v.ex, v.exm, dxu, v.dx, v.dxm);
@@ -268,29 +379,28 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
     auto mur = [](const float4 c, float tn, float sn, float sf, bool once) {
         return mur_round<T>(c.x, (c.y * tn + c.z * sn) - c.w * sf, once);
     };
-    const bool hi = C.hi_once != 0;
+    const bool hi = C.hi_once() != 0;
     if (deep) {   // only the x faces are near
         if (own) {
-            st(C.h1[0], o, hx); st(C.h1[1], o, hy); st(C.h1[2], o, hz);
-            if (il) { st(C.dT[0], o, dxu); st(C.eT[0], o, exn); }
-            if (ii) { st(C.dT[1], o, dyu); st(C.eT[1], o, eyn); st(C.eT[2], o, ezn); }
-            if (rdz) st(C.dT[2], o, dzu);
+            st(C.h1(0), o, hx); st(C.h1(1), o, hy); st(C.h1(2), o, hz);
+            if (il) { st(C.dT(0), o, dxu); st(C.eT(0), o, exn); }
+            if (ii) { st(C.dT(1), o, dyu); st(C.eT(1), o, eyn); st(C.eT(2), o, ezn); }
+            if (rdz) st(C.dT(2), o, dzu);
             if (i == 1) {
-                st(C.eT[1], o - ES, mur(mc, X::rnd(eyn), v.ey, v.ey_im, false));
-                st(C.eT[2], o - ES, mur(mc, X::rnd(ezn), v.ez, v.ez_im, false));
+                st(C.eT(1), o - ES, mur(mc, X::rnd(eyn), v.ey, v.ey_im, false));
+                st(C.eT(2), o - ES, mur(mc, X::rnd(ezn), v.ez, v.ez_im, false));
             }
             if (i == nx - 2) {
                 // the x-high Ey face reads the source neighbour twice (fdtd_calculations.cu:323-325)
-                st(C.eT[1], o + ES, mur(mc, v.ey, v.ey, v.ey_ip, hi));
-                st(C.eT[2], o + ES, mur(mc, X::rnd(ezn), v.ez, v.ez_ip, hi));
+                st(C.eT(1), o + ES, mur(mc, v.ey, v.ey, v.ey_ip, hi));
+                st(C.eT(2), o + ES, mur(mc, X::rnd(ezn), v.ez, v.ez_ip, hi));
             }
         }
         return;
     }
     float pv = 0.0f;
-    auto face = [&](int seg, char *dst, uint32_t b, const float4 *coef, long long cell, float tn, float sn, float sf,
-                    bool once) {
-        const float x = mur(coef[cell], tn, sn, sf, once);
+    auto face = [&](int seg, char *dst, uint32_t b, int side, float tn, float sn, float sf, bool once) {
+        const float x = mur(C.coef(side, i, j, k), tn, sn, sf, once);
         if (probe < 0) st(dst, b, x);
         else if (seg == pseg) pv = x;
     };
@@ -299,64 +409,94 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
         const float rx = X::rnd(exn), ry = X::rnd(eyn);
         // Ez at k = 0 is outside the E update: a face there reads the target slot (not written in this step)
         float rz = X::rnd(ezn);
-        if (k == 0) rz = ld(C.eT[2], o);
-        const long long cx = (long long)k * ny + j, cy = (long long)k * nx + i, cz = (long long)j * nx + i;
+        if (k == 0) rz = ld(C.eT(2), o);
         if (fx0) {
-            if (jl && kz) face(4, C.eT[1], o - ES, C.mur[0], cx, ry, v.ey, v.ey_im, false);
-            if (ji && kh) face(8, C.eT[2], o - ES, C.mur[0], cx, rz, v.ez, v.ez_im, false);
+            if (jl && kz) face(4, C.eT(1), o - ES, 0, ry, v.ey, v.ey_im, false);
+            if (ji && kh) face(8, C.eT(2), o - ES, 0, rz, v.ez, v.ez_im, false);
         }
         if (fx1) {
-            if (jl && kz) face(5, C.eT[1], o + ES, C.mur[1], cx, v.ey, v.ey, v.ey_ip, hi);
-            if (ji && kh) face(9, C.eT[2], o + ES, C.mur[1], cx, rz, v.ez, v.ez_ip, hi);
+            if (jl && kz) face(5, C.eT(1), o + ES, 1, v.ey, v.ey, v.ey_ip, hi);
+            if (ji && kh) face(9, C.eT(2), o + ES, 1, rz, v.ez, v.ez_ip, hi);
         }
         if (fy0) {
-            if (il && kz) face(0, C.eT[0], o - syb, C.mur[2], cy, rx, v.ex, v.ex_jm, true);
-            if (ii && kh) face(10, C.eT[2], o - syb, C.mur[2], cy, rz, v.ez, v.ez_jm, true);
+            if (il && kz) face(0, C.eT(0), o - syb, 2, rx, v.ex, v.ex_jm, true);
+            if (ii && kh) face(10, C.eT(2), o - syb, 2, rz, v.ez, v.ez_jm, true);
         }
         if (fy1) {
-            if (il && kz) face(1, C.eT[0], o + syb, C.mur[3], cy, rx, v.ex, v.ex_jp, true);
-            if (ii && kh) face(11, C.eT[2], o + syb, C.mur[3], cy, rz, v.ez, v.ez_jp, true);
+            if (il && kz) face(1, C.eT(0), o + syb, 3, rx, v.ex, v.ex_jp, true);
+            if (ii && kh) face(11, C.eT(2), o + syb, 3, rz, v.ez, v.ez_jp, true);
         }
         if (fz0) {
-            if (il && ji) face(2, C.eT[0], o - szb, C.mur[4], cz, rx, v.ex, v.ex_km, true);
-            if (ii && jl) face(6, C.eT[1], o - szb, C.mur[4], cz, ry, v.ey, v.ey_km, true);
+            if (il && ji) face(2, C.eT(0), o - szb, 4, rx, v.ex, v.ex_km, true);
+            if (ii && jl) face(6, C.eT(1), o - szb, 4, ry, v.ey, v.ey_km, true);
         }
         if (fz1) {
-            if (il && ji) face(3, C.eT[0], o + szb, C.mur[5], cz, rx, v.ex, v.ex_kp, true);
-            if (ii && jl) face(7, C.eT[1], o + szb, C.mur[5], cz, ry, v.ey, v.ey_kp, true);
+            if (il && ji) face(3, C.eT(0), o + szb, 5, rx, v.ex, v.ex_kp, true);
+            if (ii && jl) face(7, C.eT(1), o + szb, 5, ry, v.ey, v.ey_kp, true);
         }
     }
     if (probe < 0) {
         if (own) {
-            st(C.h1[0], o, hx); st(C.h1[1], o, hy); st(C.h1[2], o, hz);
-            if (rdx) { st(C.dT[0], o, dxu); st(C.eT[0], o, exn); }
-            if (rdy) st(C.dT[1], o, dyu);
-            if (rdz) st(C.dT[2], o, dzu);
+            st(C.h1(0), o, hx); st(C.h1(1), o, hy); st(C.h1(2), o, hz);
+            if (rdx) { st(C.dT(0), o, dxu); st(C.eT(0), o, exn); }
+            if (rdy) st(C.dT(1), o, dyu);
+            if (rdz) st(C.dT(2), o, dzu);
             // face cells that a segment covers are stored by their neighbour's lane
             const bool fy = (i == nx - 1 && jl && kz) || (k == nz - 1 && ii && jl);
             const bool fz = (i == nx - 1 && ji && kh) || ((j == 0 || j == ny - 1) && ii && kh);
-            if (reyz && !fy) st(C.eT[1], o, eyn);
-            if (reyz && !fz) st(C.eT[2], o, ezn);
+            if (reyz && !fy) st(C.eT(1), o, eyn);
+            if (reyz && !fz) st(C.eT(2), o, ezn);
         }
         return;
     }
     // the value probe pf records: what this step stores, or what the target slot keeps
     switch (pf) {
-    case 0: pv = rdx ? X::rnd(dxu) : ld(C.dT[0], o); break;
-    case 1: pv = rdy ? X::rnd(dyu) : ld(C.dT[1], o); break;
-    case 2: pv = rdz ? X::rnd(dzu) : ld(C.dT[2], o); break;
+    case 0: pv = rdx ? X::rnd(dxu) : ld(C.dT(0), o); break;
+    case 1: pv = rdy ? X::rnd(dyu) : ld(C.dT(1), o); break;
+    case 2: pv = rdz ? X::rnd(dzu) : ld(C.dT(2), o); break;
     case 3: pv = X::rnd(hx); break;
     case 4: pv = X::rnd(hy); break;
     case 5: pv = X::rnd(hz); break;
     default:
         if (pseg < 0) {
-            if (pf == 6) pv = rdx ? X::rnd(exn) : ld(C.eT[0], o);
-            else if (pf == 7) pv = reyz ? X::rnd(eyn) : ld(C.eT[1], o);
-            else pv = reyz ? X::rnd(ezn) : ld(C.eT[2], o);
+            if (pf == 6) pv = rdx ? X::rnd(exn) : ld(C.eT(0), o);
+            else if (pf == 7) pv = reyz ? X::rnd(eyn) : ld(C.eT(1), o);
+            else pv = reyz ? X::rnd(ezn) : ld(C.eT(2), o);
         }
         break;
     }
-    if ((threadIdx.x & 63) == 0) C.p.out[(long long)C.p.row * C.p.nprobe + probe] = (double)pv * C.p.factor[pf];
+    if ((threadIdx.x & 63) == 0) C.record(probe, pf, pv);
+}
+
+template <typename T, bool EXACT, int BXL>
+__global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
+{
+    cell_block<T, EXACT, BXL>(OneStep{C}, (int)blockIdx.x, (int)blockIdx.y);
+}
+
+// One step of a group of a batch's grids: blocks [start[q], start[q + 1]) of
+// the launch are grid q's, a multiple of 8, so that cell_block's mapping of
+// tiles to XCDs holds.  Grids outside their step window are skipped.
+template <typename T, bool EXACT>
+__global__ __launch_bounds__(kCellBlock) void cell_batch(const CellInst *inst, const CellGroups *groups, int first,
+                                                         int count, int step)
+{
+    Const<CellGroups> *S = (Const<CellGroups> *)groups;
+    const int b = (int)blockIdx.x + S->start[first];
+    int lo = first, hi = first + count - 1;
+    while (lo < hi) {   // the last grid whose blocks start at or before b
+        const int mid = (lo + hi + 1) / 2;
+        if (S->start[mid] <= b) lo = mid;
+        else hi = mid - 1;
+    }
+    Const<CellInst> *d = (Const<CellInst> *)inst + S->idx[lo];
+    const int n = step - d->start;
+    if (n < 0 || n >= d->nsteps) return;
+    const int local = b - S->start[lo], gx = 8 * d->run;
+    const int bz = local / gx, bx = local - bz * gx;
+    const BatchStep C{d, (n + 2) % 3, (n + 1) % 3, n % 3, n & 1, n};
+    if (d->bxl == 6) cell_block<T, EXACT, 6>(C, bx, bz);
+    else cell_block<T, EXACT, 5>(C, bx, bz);
 }
 
 template <typename T, bool EXACT>
@@ -384,15 +524,9 @@ __global__ __launch_bounds__(kCellBlock) void mur_coefs(const MurCoefArgs a)
     const float *rp = axis == 0 ? a.rp[end ? 3 : 0] : axis == 1 ? a.rp[end ? 4 : 1] : a.rp[end ? 5 : 2];
     const float rpf = rp[at + (end ? step : 0)], rpn = rp[at + (end ? 0 : step)];
     const float h = axis == 0 ? a.h[0] : axis == 1 ? a.h[1] : a.h[2];
-    const float sf = sqrtf(a.mu0 * a.eps0 * rpf), sn = sqrtf(a.mu0 * a.eps0 * rpn);
-    float4 c;
-    c.x = 1 / (a.dt + h * sf);
-    c.y = a.dt - h * sn;
-    c.z = a.dt + h * sn;
-    c.w = a.dt - h * sf;
     const long long nyz = (long long)a.ny * a.nz, nxz = (long long)a.nx * a.nz;
     const long long base = axis == 0 ? 0 : axis == 1 ? 2 * nyz : 2 * (nyz + nxz);
-    a.out[base + end * n + q] = c;
+    a.out[base + end * n + q] = mur_coef(a.dt, h, a.mu0, a.eps0, rpf, rpn);
 }
 
 }  // namespace
@@ -413,4 +547,18 @@ hipError_t launch_cell_step(const CellArgs &c, int storage, hipStream_t s, hipEv
     case kStoreBF16: return launch_cell_t<__hip_bfloat16, false>(c, s, t0, t1);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
+                             int storage, hipStream_t s)
+{
+    const dim3 grid((unsigned)blocks), block(kCellBlock);
+    switch (storage) {
+    case kStoreF32: cell_batch<float, true><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    case kStoreF32Fast: cell_batch<float, false><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    case kStoreF16: cell_batch<__half, false><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    case kStoreBF16: cell_batch<__hip_bfloat16, false><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }

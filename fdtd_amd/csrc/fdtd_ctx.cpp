@@ -146,13 +146,7 @@ int upload_lut(fdtd_ctx *c)
     HIP_TRY(hipDeviceSynchronize());
     HIP_TRY(hipMemcpy(c->lut, lut.data(), sizeof(MatCoef) * c->nmat, hipMemcpyHostToDevice));
     c->lut_dirty = false;
-    c->zmask = 0;
-    for (int m = 0; m < std::min(c->nmat, 32); m++) {
-        uint32_t a, g[2];
-        memcpy(&a, &lut[m].a, 4);
-        memcpy(g, &lut[m].g3, 8);
-        if (a == 0 && g[0] == 0 && g[1] == 0) c->zmask |= 1u << m;
-    }
+    c->zmask = cell_zmask(lut.data(), c->nmat);
     return 0;
 }
 
@@ -609,13 +603,8 @@ void fill_cell_args(fdtd_ctx *c, const StepArgs &a, CellArgs &q)
     q.cd[0] = a.cdx; q.cd[1] = a.cdy; q.cd[2] = a.cdz;
     q.jz = a.jz;
     q.zmask = a.zskip ? c->zmask : 0;
-    q.bxl = cell_lanes_log2(c->nx);
     q.hi_once = a.mur_x == 2;
-    const int bx = 1 << q.bxl, by = 256 / bx;
-    q.tiles_x = (c->nx + bx - 1) / bx;
-    q.tx_mul = (uint32_t)(((1ull << 32) + q.tiles_x - 1) / q.tiles_x);
-    q.tiles = q.tiles_x * ((c->ny + by - 1) / by);
-    q.run = (q.tiles + 7) / 8;
+    cell_tiles(c->nx, c->ny, q);
     const size_t nyz = (size_t)c->ny * c->nz, nxz = (size_t)c->nx * c->nz, nxy = (size_t)c->nx * c->ny;
     const float4 *m = c->mur;
     const size_t step[6] = {nyz, nyz, nxz, nxz, nxy, nxy};

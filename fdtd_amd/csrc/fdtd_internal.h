@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
+#include <string.h>
 #include <algorithm>
 #include <initializer_list>
 #include <stdint.h>
@@ -218,6 +219,29 @@ inline int cell_lanes_log2(int nx)
     const double e6 = (double)nx / (64 * ((nx + 63) / 64)), e5 = (double)nx / (32 * ((nx + 31) / 32));
     return e6 < 0.8 * e5 ? 5 : 6;
 }
+// The tile geometry of a grid (CellArgs, CellInst) and the materials whose
+// cells skip levels n-1.
+template <typename A>
+inline void cell_tiles(int nx, int ny, A &a)
+{
+    a.bxl = cell_lanes_log2(nx);
+    const int bx = 1 << a.bxl, by = 256 / bx;
+    a.tiles_x = (nx + bx - 1) / bx;
+    a.tx_mul = (uint32_t)(((1ull << 32) + a.tiles_x - 1) / a.tiles_x);
+    a.tiles = a.tiles_x * ((ny + by - 1) / by);
+    a.run = (a.tiles + 7) / 8;
+}
+inline uint32_t cell_zmask(const MatCoef *lut, int nmat)
+{
+    uint32_t z = 0;
+    for (int m = 0; m < std::min(nmat, 32); m++) {
+        uint32_t a, g[2];
+        memcpy(&a, &lut[m].a, 4);
+        memcpy(g, &lut[m].g3, 8);
+        if (a == 0 && g[0] == 0 && g[1] == 0) z |= 1u << m;
+    }
+    return z;
+}
 hipError_t launch_cell_step(const CellArgs &c, int storage, hipStream_t s, hipEvent_t t0 = nullptr,
                             hipEvent_t t1 = nullptr);
 
@@ -421,6 +445,43 @@ struct BatchShared {
     int nrec;
     int rec[kBatchMaxInst * kBatchMaxProbes][2];   // (instance, probe)
 };
+
+// A batch's grid as cell_batch steps it.  Field and id pointers as in
+// CellArgs, by ring slot and H buffer.
+struct CellInst {
+    char *E[3][3], *D[3][3], *H[2][3];
+    const uint8_t *ids;
+    const MatCoef *lut;
+    const float *jz;
+    const float *rp[6];
+    const float4 *murx0, *murx1;
+    const int *probes;
+    double *probe_out;
+    double factor[9];
+    int nx, ny, nz;
+    uint32_t o0, sy, sz;
+    int tiles_x, tiles, run;
+    uint32_t tx_mul;
+    float ch[3], cd[3];
+    uint32_t zmask;
+    int hi_once, bxl;
+    int nprobe, probe_rows, jz_len, jz_hold3, start, nsteps;
+    float dt, h[3], mu0, eps0;
+};
+
+// The groups' grids one after another, and prefix sums of their blocks.
+struct CellGroups {
+    int idx[kBatchMaxInst];
+    int start[kBatchMaxInst + 1];
+};
+// Blocks of a grid's step: its planes' and its probes' (four a block).
+inline int cell_blocks(const CellInst &d)
+{
+    const int gx = 8 * d.run, pb = (d.nprobe + 3) / 4;
+    return gx * (d.nz + (pb + gx - 1) / gx);
+}
+hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
+                             int storage, hipStream_t s);
 
 struct BatchLaunch {
     const BatchInst *inst;

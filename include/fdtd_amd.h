@@ -289,9 +289,10 @@ int fdtd_load_phantom_ids(const char *dir, int nx, int ny, int nz, int mode, int
 /* ---- batches of independent grids --------------------------------------
  *
  * A batch holds many grids of different sizes, materials, sources, storage
- * forms and step counts in one device arena.  Each step of the batch is one
- * persistent fused kernel per storage form present, one Mur launch and one
- * probe launch over every running grid, replayed from captured HIP graphs;
+ * forms and step counts in one device arena.  Small grids are stepped in
+ * groups whose state fits the Infinity Cache, one launch per group and step;
+ * a step of the others is one persistent fused kernel per storage form
+ * present, one Mur launch and one probe launch, replayed from captured graphs;
  * grids join (fdtd_batch_add) and leave (fdtd_batch_remove) between calls.
  * A grid's results are those of a single fdtd_ctx with the same inputs, bit
  * for bit (the per-cell arithmetic does not depend on the batch). */
@@ -355,10 +356,14 @@ int fdtd_batch_probe_peak_units(fdtd_batch *b, int id, double *peak, int nprobe)
 /* Waits for the device; level as fdtd_ctx_get_field, after the grid's
  * steps so far. */
 int fdtd_batch_get_field(fdtd_batch *b, int id, int field, int level, float *host);
-/* tile_y in {2,4,8}, kchunk >= 1, graph_steps >= 1 (0 keeps a value). */
+/* tile_y in {2,4,8}, kchunk >= 1, graph_steps >= 1 (0 keeps a value).  With a
+ * tile_y or kchunk every grid is stepped in tiles of that shape; otherwise
+ * grids whose state fits the Infinity Cache are stepped in groups that do, one
+ * lane per cell (same results). */
 int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int graph_steps);
 /* Times every (tile_y in {2,4,8}, kchunk in {3,4,6,8,16}) candidate on the batch's own grids for
- * trial_steps steps each, keeps the fastest and restores the grids to
+ * trial_steps steps each, and the groups of small grids, keeps the fastest (tile_y and kchunk: of the
+ * shapes) and restores the grids to
  * their zero initial state.  Every grid must be unstepped. */
 int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t stream, int *tile_y, int *kchunk);
 int fdtd_batch_info(fdtd_batch *b, FdtdBatchInfo *info);

@@ -100,3 +100,37 @@ def test_cells_equal_the_oracle(shape):
             a, b = ctx.get(f, lv), sim.get(f, lv)
             assert bits_equal(a, b), f"{F.FIELDS[f]} level {lv}: {first_diff(a, b)}"
     assert np.array_equal(ctx.probes().astype(np.float32).view(np.uint32), ref.astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+def test_batch_groups_equal_single_grids():
+    """Grids of a batch stepped in groups: several grids of one storage form
+    in a launch, forms in groups of their own, probes past the planes' blocks,
+    grids that join and finish inside a run, 32- and 64-lane tiles."""
+    from tests.test_gpu_batch import assert_same, make_case, single
+    cases = [((20, 24, 28), 4, 17, F.STORE_F32, F.JZ_STEP, False, 6), ((33, 17, 40), 12, 70, F.STORE_F32, F.JZ_HOLD3, True, 64),
+             ((66, 9, 12), 6, 45, F.STORE_F16, F.JZ_STEP, True, 6), ((96, 16, 16), 5, 33, F.STORE_F16, F.JZ_STEP, False, 0),
+             ((16, 16, 16), 5, 9, F.STORE_F32_FAST, F.JZ_STEP, False, 6), ((48, 40, 20), 8, 40, F.STORE_BF16, F.JZ_STEP, True, 6),
+             ((65, 5, 7), 4, 33, F.STORE_F32, F.JZ_STEP, False, 9), ((3, 3, 3), 2, 50, F.STORE_F32, F.JZ_STEP, False, 64)]
+    insts = [make_case(300 + q, *c[:6], nprobe=c[6]) for q, c in enumerate(cases)]
+    refs = [single(x) for x in insts]
+    with F.Batch(1 << 30) as b:
+        ids = [b.add(x) for x in insts[:5]]
+        b.run(11)
+        ids += [b.add(x) for x in insts[5:]]
+        b.run(1)
+        b.run(90)
+        for q, (i, x) in enumerate(zip(ids, insts)):
+            assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
+
+
+@pytest.mark.parametrize("count,edge", [(3, 100), (2, 148)])   # two groups of fp32 grids; one group and one grid in tiles
+def test_batch_groups_and_tiles(count, edge):
+    from tests.test_gpu_batch import assert_same, make_case, single
+    insts = [make_case(400 + q, (edge + q, edge, edge - 3 * q), 5, 40 + q) for q in range(count)]
+    refs = [single(x) for x in insts]
+    with F.Batch(4 << 30) as b:
+        ids = [b.add(x) for x in insts]
+        b.run(45)
+        for q, (i, x) in enumerate(zip(ids, insts)):
+            assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
