@@ -238,10 +238,10 @@ bool is_running(const fdtd_batch *b, int s)
     return I.used && b->step - I.start < I.steps;
 }
 
-// Whether cell_batch steps the grid: as a context's default_cell.
+// Whether cell_batch steps the grid.
 bool cell_grid(const fdtd_batch *b, const fdtd_batch::Inst &I)
 {
-    return b->by_cell && I.d.nz <= kCellMaxPlanes && 24 * I.L.Np * I.L.esz <= cell_state_limit(I.L.esz);
+    return b->by_cell && I.d.nz <= kCellMaxPlanes && 24 * I.L.Np * I.L.esz <= cell_near_limit(I.L.esz);
 }
 
 // Groups of the grids `cell` whose state fits kCellGroupBytes together (one
@@ -626,7 +626,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.o0 = (uint32_t)gb;
     c.sy = (uint32_t)(L.pitch * L.esz);
     c.sz = (uint32_t)(L.plane * L.esz);
-    cell_tiles(nx, ny, c);
+    cell_tiles(nx, ny, kCellNear, c);
     for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
     c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : 0;
     c.nprobe = d.nprobe;

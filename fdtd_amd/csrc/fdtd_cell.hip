@@ -1,16 +1,27 @@
 // cell_step: one time step of a grid in one launch, one cell per lane and no
-// z-march, for grids whose state fits the 256 MB Infinity Cache (or nearly).
-// A tiled launch (fused_step) of such a grid is bound by the latency of its
-// blocks' marches, not by bytes: at 64^3 it runs 256 blocks for 16 us.
+// z-march.  A tiled launch (fused_step) of a grid in the 256 MB Infinity Cache
+// is bound by the latency of its blocks' marches, not by bytes: at 64^3 it
+// runs 256 blocks for 16 us.
 //
 // A lane computes its cell's H^{n+1/2}, D^{n+1} (with the source) and
 // E^{n+1} from loads that depend on nothing but the cell's index: the six
 // halo H values that curl H needs (at i-1, j-1, k-1) are recomputed from
 // H^{n-1/2} and E^n, operation for operation as fused_tile does, so the two
 // kernels give identical results.  All loads of a wave go out together;
-// there is no LDS and no barrier.  Loads and stores are cached ones: the next
-// step reads what this one wrote, and streaming stores would send it to HBM
-// (128^3 fp32: 45 us with them, 32 us without).
+// there is no LDS and no barrier.
+//
+// Forms, by the size of the state (cell_form):
+//   * near, in the Infinity Cache: all loads and stores cached, as the next
+//     step reads what this one wrote, and streaming stores would send it to
+//     HBM (128^3 fp32: 38 us with them, 30 us without);
+//   * mid: the lanes take their neighbours along x from each other.  In a near
+//     grid the eleven loads of them cost nothing; here they hit lines that are
+//     still on their way from HBM, and hold up the vector cache.  The values
+//     past a row's ends come through the scalar cache;
+//   * part: and D streams past the Infinity Cache, which holds E and H;
+//   * far: and so do E^{n-1} and the stores of E; H and E^n stay for longer.
+// Every other step takes the planes from the highest down (flip): it starts
+// on those that the last step left in the cache.
 //
 // The first-order Mur faces and the probe row are part of the same launch:
 //   * a face cell's new E needs E^{n+1} of its inward neighbour, E^n of both
@@ -24,12 +35,14 @@
 //     for, so it waits for no other wave.
 //
 // Measured on MI355X, whole steps, against fused_step and the Mur launch
-// (us): fp32 24^3 5.7 (15.1), 64^3 7.4 (16.6), 100^3 20.6 (31.2), 128^3 31
-// (47), 160x160x100 35 (60); fp16 64^3 6.7 (18.0), 96x121x77 13.0 (27.6),
-// 151x138x188 45 (78).  The kernel itself takes 27.4 us at 128^3 (5.3 TB/s at
-// the L2's far side, where a stream of the same arrays reaches 8.0): it is
-// held by instruction issue and resident waves (7 of 8 a SIMD), with 55
-// memory instructions and 216 vector ones a wave.
+// (us): fp32 24^3 5.7 (15.1), 64^3 7.4 (16.6), 100^3 20.5 (31.2), 128^3 28
+// (47), 160x160x100 34 (60), 151x138x188 77 (83), 256^3 280 (304); fp16 64^3
+// 6.9 (18.0), 96x121x77 13.4 (27.6), 256^3 181 (206), 320x320x300 318 (377).
+// 128^3 moves 178 MB, 6.4 TB/s at the L2's far side, where a stream of the same
+// arrays reaches 8.0; with 4 waves a SIMD instead of 7 it takes as long.  Past
+// the cache fp32 waits for HBM (85 bytes a cell at 5.1 TB/s at 320x320x224;
+// occupancy again makes no difference); 16-bit fields have half the bytes in
+// flight a wave, and each wave less than 8 a SIMD shows.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -77,6 +90,40 @@ __device__ __forceinline__ float at(const char *p, uint32_t b, int d = 0)
     else
         return Elem<T>::cvt(__hip_atomic_load((const unsigned short *)(p + b) + d, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_WAVEFRONT));
+}
+
+template <typename V> using Const = const __attribute__((address_space(4))) V;
+
+// The element at a wave-uniform offset, through the scalar cache: its own path
+// beside the vector loads'.  Only for arrays that the launch does not write.
+template <typename T>
+__device__ __forceinline__ float at_uniform(const char *p, uint32_t b)
+{
+    if constexpr (sizeof(T) == 4) {
+        return *(Const<float> *)(p + b);
+    } else {
+        const uintptr_t q = (uintptr_t)(p + b);
+        return Elem<T>::cvt((unsigned short)(*(Const<uint32_t> *)(q & ~(uintptr_t)3) >> ((q & 2) * 8)));
+    }
+}
+
+// The value of the lane below (above); the wave's first (last) lane gets `end`.
+__device__ __forceinline__ float lane_below(float v, float end)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_above(float v, float end)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x130, 0xf, 0xf, false));
+}
+
+// A value that the next step does not read soon enough to find it in the
+// Infinity Cache (NT): a streaming load.
+template <typename T, bool NT>
+__device__ __forceinline__ float at_once(const char *p, uint32_t b)
+{
+    if constexpr (NT) return Elem<T>::ld_nt((const T *)p, b);
+    else return at<T>(p, b);
 }
 
 // A Mur face's new value q * x as storage type T holds it.  The compiler
@@ -129,6 +176,7 @@ struct OneStep {
     __device__ __forceinline__ float cd(int q) const { return a.cd[q]; }
     __device__ __forceinline__ uint32_t zmask() const { return a.zmask; }
     __device__ __forceinline__ int hi_once() const { return a.hi_once; }
+    __device__ __forceinline__ int flip() const { return a.flip; }
     __device__ __forceinline__ const char * e0(int q) const { return a.e0[q]; }
     __device__ __forceinline__ const char * e1(int q) const { return a.e1[q]; }
     __device__ __forceinline__ const char * d0(int q) const { return a.d0[q]; }
@@ -156,7 +204,6 @@ struct OneStep {
 // The same of a batch's grid at its step n, from its descriptor: the ring
 // slot and H buffer roles follow n as a single grid's do.  The y and z faces'
 // coefficients come from the rp planes (a batch keeps no table of them).
-template <typename V> using Const = const __attribute__((address_space(4))) V;
 struct BatchStep {
     Const<CellInst> *d;
     int s0, s1, sT, hb;     // slots of levels n, n-1, n+1; buffer of H^{n-1/2}
@@ -177,6 +224,7 @@ struct BatchStep {
     __device__ __forceinline__ float cd(int q) const { return d->cd[q]; }
     __device__ __forceinline__ uint32_t zmask() const { return d->zmask; }
     __device__ __forceinline__ int hi_once() const { return d->hi_once; }
+    __device__ __forceinline__ int flip() const { return 0; }
     __device__ __forceinline__ const char * e0(int q) const { return d->E[s0][q]; }
     __device__ __forceinline__ const char * e1(int q) const { return d->E[s1][q]; }
     __device__ __forceinline__ const char * d0(int q) const { return d->D[s0][q]; }
@@ -227,12 +275,13 @@ struct Ops {
 // load E^{n-1} and D^{n-1}, as fused_tile's zero-term rows, decided per lane;
 // a grid that always loads them has zmask = 0.  C: where the step's operands
 // are (OneStep, BatchStep); block bx of the 8 * C.run() of plane bz.
-template <typename T, bool EXACT, int BXL, typename G>
+template <typename T, bool EXACT, int BXL, int FORM, typename G>
 __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
 {
     using X = Elem<T>;
     constexpr uint32_t ES = sizeof(T);
     constexpr int BX = 1 << BXL, BY = kCellBlock / BX, WY = 64 / BX;
+    constexpr bool LANES = FORM != kCellNear, ND = FORM >= kCellPart, NE = FORM == kCellFar;
     const int nx = C.nx(), ny = C.ny(), nz = C.nz();
 
     // Blocks (bx, k) of plane k in 8 runs of tiles, one run per XCD (workgroups
@@ -240,20 +289,21 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     // tile's neighbours in the plane and the same tiles of the planes around it
     // share its L2.  Rows past nz hold the probes.
     int i, j, k;
-    bool own = true, deep = false, edge = false;
+    int i0, jw;                              // the wave's first column and row
+    bool deep = false, edge = false;
     int probe = -1, pf = -1, pseg = -1;      // probe: its index, field and face segment
     if (bz < nz) {
         const int t = (bx & 7) * C.run() + (bx >> 3);
         if (t >= C.tiles()) return;
         const int ty = C.tiles_x() == 1 ? t : (int)__umulhi((unsigned)t, C.tx_mul()), tx = t - ty * C.tiles_x();
         const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = (int)threadIdx.x & 63;
-        const int jw = ty * BY + w * WY;     // the wave's first row
+        jw = ty * BY + w * WY;
         if (jw >= ny) return;
-        i = tx * BX + (l & (BX - 1));
+        i0 = tx * BX;
+        i = i0 + (l & (BX - 1));
         j = BX >= 64 ? jw : jw + (l >> BXL);
-        k = bz;
-        own = i < nx && j < ny;
-        j = min(j, ny - 1);
+        k = C.flip() ? nz - 1 - bz : bz;
+        if (i >= nx || j >= ny) return;
         deep = jw >= 2 && jw + WY <= ny - 2 && k >= 2 && k < nz - 2 && nx > 3;
         edge = tx == 0 || (nx - 2 >= tx * BX && nx - 2 < tx * BX + BX);
     } else {
@@ -267,6 +317,10 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
             pseg = face_of(pf - 6, i, j, k, nx, ny, nz, di, dj, dk);
             i += di; j += dj; k += dk;
         }
+        // lane 1 holds the cell, the lanes beside it its neighbours along x
+        i0 = i - 1;
+        jw = j;
+        i = min(max(i0 + min((int)threadIdx.x & 63, 2), 0), nx - 1);
     }
 
     // deep: the wave's rows and plane are at least two cells inside the y and z faces, so that of the faces only
@@ -279,19 +333,35 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     Ops v;
     const char *px = C.e0(0), *py = C.e0(1), *pz = C.e0(2), *qx = C.h0(0), *qy = C.h0(1), *qz = C.h0(2);
     v.ex = at<T>(px, o); v.ey = at<T>(py, o); v.ez = at<T>(pz, o);
-    v.ex_im = at<T>(px, o, -1); v.ey_im = at<T>(py, o, -1); v.ez_im = at<T>(pz, o, -1);
-    v.ey_ip = at<T>(py, o, 1); v.ez_ip = at<T>(pz, o, 1);
-    v.ex_jp = at<T>(px, ojp); v.ez_jp = at<T>(pz, ojp); v.ex_jp_im = at<T>(px, ojp, -1);
-    v.ex_jm = at<T>(px, ojm); v.ey_jm = at<T>(py, ojm); v.ez_jm = at<T>(pz, ojm); v.ey_jm_ip = at<T>(py, ojm, 1);
-    v.ex_kp = at<T>(px, okp); v.ey_kp = at<T>(py, okp); v.ex_kp_im = at<T>(px, okp, -1);
+    v.ex_jp = at<T>(px, ojp); v.ez_jp = at<T>(pz, ojp);
+    v.ex_jm = at<T>(px, ojm); v.ey_jm = at<T>(py, ojm); v.ez_jm = at<T>(pz, ojm);
+    v.ex_kp = at<T>(px, okp); v.ey_kp = at<T>(py, okp);
     v.ey_kp_jm = at<T>(py, okp - syb);
-    v.ex_km = at<T>(px, okm); v.ey_km = at<T>(py, okm); v.ez_km = at<T>(pz, okm); v.ez_km_ip = at<T>(pz, okm, 1);
+    v.ex_km = at<T>(px, okm); v.ey_km = at<T>(py, okm); v.ez_km = at<T>(pz, okm);
     v.ez_km_jp = at<T>(pz, okm + syb);
     v.hx = at<T>(qx, o); v.hy = at<T>(qy, o); v.hz = at<T>(qz, o);
-    v.hy_im = at<T>(qy, o, -1); v.hz_im = at<T>(qz, o, -1);
     v.hx_jm = at<T>(qx, ojm); v.hz_jm = at<T>(qz, ojm);
     v.hx_km = at<T>(qx, okm); v.hy_km = at<T>(qy, okm);
-    v.dx = at<T>(C.d0(0), o); v.dy = at<T>(C.d0(1), o); v.dz = at<T>(C.d0(2), o);
+    // Neighbours along x: near, loads of their own; else from the lanes beside
+    // (below), and past the wave's ends from these.
+    float end[11] = {};
+    if constexpr (LANES) {
+        const uint32_t lo = C.o0() + (uint32_t)k * szb + (uint32_t)jw * syb + (uint32_t)((i0 - 1) * (int)ES);
+        const uint32_t hi = lo + (BX + 1) * ES;
+        end[0] = at_uniform<T>(px, lo); end[1] = at_uniform<T>(py, lo); end[2] = at_uniform<T>(pz, lo);
+        end[3] = at_uniform<T>(py, hi); end[4] = at_uniform<T>(pz, hi);
+        end[5] = at_uniform<T>(px, lo + syb); end[6] = at_uniform<T>(py, hi - syb);
+        end[7] = at_uniform<T>(px, lo + szb); end[8] = at_uniform<T>(pz, hi - szb);
+        end[9] = at_uniform<T>(qy, lo); end[10] = at_uniform<T>(qz, lo);
+    }
+    if constexpr (!LANES) {
+        v.ex_im = at<T>(px, o, -1); v.ey_im = at<T>(py, o, -1); v.ez_im = at<T>(pz, o, -1);
+        v.ey_ip = at<T>(py, o, 1); v.ez_ip = at<T>(pz, o, 1);
+        v.ex_jp_im = at<T>(px, ojp, -1); v.ey_jm_ip = at<T>(py, ojm, 1);
+        v.ex_kp_im = at<T>(px, okp, -1); v.ez_km_ip = at<T>(pz, okm, 1);
+        v.hy_im = at<T>(qy, o, -1); v.hz_im = at<T>(qz, o, -1);
+    }
+    v.dx = at_once<T, ND>(C.d0(0), o); v.dy = at_once<T, ND>(C.d0(1), o); v.dz = at_once<T, ND>(C.d0(2), o);
     float4 mc = {0.0f, 0.0f, 0.0f, 0.0f};
     if (deep && edge && (i == 1 || i == nx - 2)) mc = C.coef(i == 1 ? 0 : 1, i, j, k);
     const uint32_t m = id & kMaterialMask;
@@ -306,11 +376,18 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         v.k1 = q->k1; v.k2 = q->k2; v.k3 = q->k3; v.k5 = q->k5;
     }
     bool need = true;
-    if constexpr (EXACT) need = own && !(m < 32 && (C.zmask() >> m & 1u));
+    if constexpr (EXACT) need = !(m < 32 && (C.zmask() >> m & 1u));
     v.exm = v.eym = v.ezm = v.dxm = v.dym = v.dzm = 0.0f;
     if (need) {
-        v.exm = at<T>(C.e1(0), o); v.eym = at<T>(C.e1(1), o); v.ezm = at<T>(C.e1(2), o);
-        v.dxm = at<T>(C.d1(0), o); v.dym = at<T>(C.d1(1), o); v.dzm = at<T>(C.d1(2), o);
+        v.exm = at_once<T, NE>(C.e1(0), o); v.eym = at_once<T, NE>(C.e1(1), o); v.ezm = at_once<T, NE>(C.e1(2), o);
+        v.dxm = at_once<T, ND>(C.d1(0), o); v.dym = at_once<T, ND>(C.d1(1), o); v.dzm = at_once<T, ND>(C.d1(2), o);
+    }
+    if constexpr (LANES) {   // (after the loads above are out: each of these waits for its operand)
+        v.ex_im = lane_below(v.ex, end[0]); v.ey_im = lane_below(v.ey, end[1]); v.ez_im = lane_below(v.ez, end[2]);
+        v.ey_ip = lane_above(v.ey, end[3]); v.ez_ip = lane_above(v.ez, end[4]);
+        v.ex_jp_im = lane_below(v.ex_jp, end[5]); v.ey_jm_ip = lane_above(v.ey_jm, end[6]);
+        v.ex_kp_im = lane_below(v.ex_kp, end[7]); v.ez_km_ip = lane_above(v.ez_km, end[8]);
+        v.hy_im = lane_below(v.hy, end[9]); v.hz_im = lane_below(v.hz, end[10]);
     }
 
     const float chx = C.ch(0), chy = C.ch(1), chz = C.ch(2);
@@ -319,6 +396,14 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     auto up_y = [&](float h, float x, float xkp, float z, float zip) { return h - chz * (xkp - x) + chx * (zip - z); };
     auto up_z = [&](float h, float y, float yip, float x, float xjp) { return h - chx * (yip - y) + chy * (xjp - x); };
     auto st = [&](char *p, uint32_t b, float x) { X::st((T *)p, b, x); };
+    auto st_d = [&](char *p, uint32_t b, float x) {
+        if constexpr (ND) X::st_nt((T *)p, b, x);
+        else X::st((T *)p, b, x);
+    };
+    auto st_e = [&](char *p, uint32_t b, float x) {
+        if constexpr (NE) X::st_nt((T *)p, b, x);
+        else X::st((T *)p, b, x);
+    };
     auto ld = [&](const char *p, uint32_t b) { return X::ld((const T *)p, b); };
 
     const bool kh = k < nz - 1, kz = k >= 1 && kh;
@@ -345,7 +430,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     float dyp = dyu, dzp = dzu;
     // E cells whose D is not updated read the target slot's value (in deep rows those are the cells of the high x
     // face, whose E the face takes over).
-    if (!deep && own && reyz && !(rdy && rdz)) {
+    if (!deep && reyz && !(rdy && rdz)) {
         if (!rdy) dyp = ld(C.dT(1), o);
         if (!rdz) dzp = ld(C.dT(2), o);
     }
@@ -360,9 +445,9 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
             const int z = min(min(__float_as_int(v.d * v.ex), __float_as_int(v.d * v.ey)), __float_as_int(v.d * v.ez));
             const float mag = __builtin_fabsf(v.ex) + __builtin_fabsf(v.ey) + __builtin_fabsf(v.ez) +
                               __builtin_fabsf(v.dx) + __builtin_fabsf(v.dy) + __builtin_fabsf(v.dz);
-            if (!need && own && (z == (int)0x80000000 || !__builtin_isfinite(mag))) {
-                v.exm = at<T>(C.e1(0), o); v.eym = at<T>(C.e1(1), o); v.ezm = at<T>(C.e1(2), o);
-                v.dxm = at<T>(C.d1(0), o); v.dym = at<T>(C.d1(1), o); v.dzm = at<T>(C.d1(2), o);
+            if (!need && (z == (int)0x80000000 || !__builtin_isfinite(mag))) {
+                v.exm = at_once<T, NE>(C.e1(0), o); v.eym = at_once<T, NE>(C.e1(1), o); v.ezm = at_once<T, NE>(C.e1(2), o);
+                v.dxm = at_once<T, ND>(C.d1(0), o); v.dym = at_once<T, ND>(C.d1(1), o); v.dzm = at_once<T, ND>(C.d1(2), o);
             }
         }
         exn = e_update(v.c, v.d, v.a, v.g1, v.g2, v.g3, v.ex, v.exm, dxu, v.dx, v.dxm);
@@ -381,20 +466,18 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     };
     const bool hi = C.hi_once() != 0;
     if (deep) {   // only the x faces are near
-        if (own) {
-            st(C.h1(0), o, hx); st(C.h1(1), o, hy); st(C.h1(2), o, hz);
-            if (il) { st(C.dT(0), o, dxu); st(C.eT(0), o, exn); }
-            if (ii) { st(C.dT(1), o, dyu); st(C.eT(1), o, eyn); st(C.eT(2), o, ezn); }
-            if (rdz) st(C.dT(2), o, dzu);
-            if (i == 1) {
-                st(C.eT(1), o - ES, mur(mc, X::rnd(eyn), v.ey, v.ey_im, false));
-                st(C.eT(2), o - ES, mur(mc, X::rnd(ezn), v.ez, v.ez_im, false));
-            }
-            if (i == nx - 2) {
-                // the x-high Ey face reads the source neighbour twice (fdtd_calculations.cu:323-325)
-                st(C.eT(1), o + ES, mur(mc, v.ey, v.ey, v.ey_ip, hi));
-                st(C.eT(2), o + ES, mur(mc, X::rnd(ezn), v.ez, v.ez_ip, hi));
-            }
+        st(C.h1(0), o, hx); st(C.h1(1), o, hy); st(C.h1(2), o, hz);
+        if (il) { st_d(C.dT(0), o, dxu); st_e(C.eT(0), o, exn); }
+        if (ii) { st_d(C.dT(1), o, dyu); st_e(C.eT(1), o, eyn); st_e(C.eT(2), o, ezn); }
+        if (rdz) st_d(C.dT(2), o, dzu);
+        if (i == 1) {
+            st_e(C.eT(1), o - ES, mur(mc, X::rnd(eyn), v.ey, v.ey_im, false));
+            st_e(C.eT(2), o - ES, mur(mc, X::rnd(ezn), v.ez, v.ez_im, false));
+        }
+        if (i == nx - 2) {
+            // the x-high Ey face reads the source neighbour twice (fdtd_calculations.cu:323-325)
+            st_e(C.eT(1), o + ES, mur(mc, v.ey, v.ey, v.ey_ip, hi));
+            st_e(C.eT(2), o + ES, mur(mc, X::rnd(ezn), v.ez, v.ez_ip, hi));
         }
         return;
     }
@@ -405,7 +488,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         else if (seg == pseg) pv = x;
     };
     const bool fx0 = i == 1, fx1 = i == nx - 2, fy0 = j == 1, fy1 = j == ny - 2, fz0 = k == 1, fz1 = k == nz - 2;
-    if (own && (fx0 || fx1 || fy0 || fy1 || fz0 || fz1)) {
+    if (fx0 || fx1 || fy0 || fy1 || fz0 || fz1) {
         const float rx = X::rnd(exn), ry = X::rnd(eyn);
         // Ez at k = 0 is outside the E update: a face there reads the target slot (not written in this step)
         float rz = X::rnd(ezn);
@@ -436,17 +519,15 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         }
     }
     if (probe < 0) {
-        if (own) {
-            st(C.h1(0), o, hx); st(C.h1(1), o, hy); st(C.h1(2), o, hz);
-            if (rdx) { st(C.dT(0), o, dxu); st(C.eT(0), o, exn); }
-            if (rdy) st(C.dT(1), o, dyu);
-            if (rdz) st(C.dT(2), o, dzu);
-            // face cells that a segment covers are stored by their neighbour's lane
-            const bool fy = (i == nx - 1 && jl && kz) || (k == nz - 1 && ii && jl);
-            const bool fz = (i == nx - 1 && ji && kh) || ((j == 0 || j == ny - 1) && ii && kh);
-            if (reyz && !fy) st(C.eT(1), o, eyn);
-            if (reyz && !fz) st(C.eT(2), o, ezn);
-        }
+        st(C.h1(0), o, hx); st(C.h1(1), o, hy); st(C.h1(2), o, hz);
+        if (rdx) { st_d(C.dT(0), o, dxu); st_e(C.eT(0), o, exn); }
+        if (rdy) st_d(C.dT(1), o, dyu);
+        if (rdz) st_d(C.dT(2), o, dzu);
+        // face cells that a segment covers are stored by their neighbour's lane
+        const bool fy = (i == nx - 1 && jl && kz) || (k == nz - 1 && ii && jl);
+        const bool fz = (i == nx - 1 && ji && kh) || ((j == 0 || j == ny - 1) && ii && kh);
+        if (reyz && !fy) st_e(C.eT(1), o, eyn);
+        if (reyz && !fz) st_e(C.eT(2), o, ezn);
         return;
     }
     // the value probe pf records: what this step stores, or what the target slot keeps
@@ -465,13 +546,13 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         }
         break;
     }
-    if ((threadIdx.x & 63) == 0) C.record(probe, pf, pv);
+    if ((threadIdx.x & 63) == 1) C.record(probe, pf, pv);
 }
 
-template <typename T, bool EXACT, int BXL>
+template <typename T, bool EXACT, int BXL, int FORM>
 __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
 {
-    cell_block<T, EXACT, BXL>(OneStep{C}, (int)blockIdx.x, (int)blockIdx.y);
+    cell_block<T, EXACT, BXL, FORM>(OneStep{C}, (int)blockIdx.x, (int)blockIdx.y);
 }
 
 // One step of a group of a batch's grids: blocks [start[q], start[q + 1]) of
@@ -495,14 +576,18 @@ __global__ __launch_bounds__(kCellBlock) void cell_batch(const CellInst *inst, c
     const int local = b - S->start[lo], gx = 8 * d->run;
     const int bz = local / gx, bx = local - bz * gx;
     const BatchStep C{d, (n + 2) % 3, (n + 1) % 3, n % 3, n & 1, n};
-    if (d->bxl == 6) cell_block<T, EXACT, 6>(C, bx, bz);
-    else cell_block<T, EXACT, 5>(C, bx, bz);
+    if (d->bxl == 6) cell_block<T, EXACT, 6, kCellNear>(C, bx, bz);
+    else cell_block<T, EXACT, 5, kCellNear>(C, bx, bz);
 }
 
 template <typename T, bool EXACT>
 hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
 {
-    const void *k = c.bxl == 6 ? (const void *)cell_step<T, EXACT, 6> : (const void *)cell_step<T, EXACT, 5>;
+    const void *k = c.form == kCellFar   ? (const void *)cell_step<T, EXACT, 6, kCellFar>
+                    : c.form == kCellPart ? (const void *)cell_step<T, EXACT, 6, kCellPart>
+                    : c.form == kCellMid ? (const void *)cell_step<T, EXACT, 6, kCellMid>
+                    : c.bxl == 6         ? (const void *)cell_step<T, EXACT, 6, kCellNear>
+                                         : (const void *)cell_step<T, EXACT, 5, kCellNear>;
     const unsigned gx = 8u * (unsigned)c.run;
     const unsigned waves = kCellBlock / 64, pb = ((unsigned)c.p.nprobe + waves - 1) / waves;
     const dim3 grid(gx, (unsigned)c.nz + (pb + gx - 1) / gx);

@@ -21,9 +21,10 @@
 namespace {
 
 // Extra elements between consecutive field arrays in the blob: staggers the
-// arrays' starts across HBM channels (a no-compute 15-read/9-write stream
-// probe measured ~4% more bandwidth with 64 Ki elements of stagger).
-constexpr size_t kArraySkew = 65536;
+// arrays' starts across HBM channels, also where a plane is a power of two
+// (256^3 fp32, us a step: 327 with 0, 1024 or 65536, 280 to 285 with 64, 4160
+// or this; 320x320x880 in tiles 1553 with 65536, 1535).
+constexpr size_t kArraySkew = 33856;
 
 }  // namespace
 
@@ -604,7 +605,9 @@ void fill_cell_args(fdtd_ctx *c, const StepArgs &a, CellArgs &q)
     q.jz = a.jz;
     q.zmask = a.zskip ? c->zmask : 0;
     q.hi_once = a.mur_x == 2;
-    cell_tiles(c->nx, c->ny, q);
+    q.flip = c->n & 1;
+    q.form = cell_form(24 * c->Np * c->esz, c->esz);
+    cell_tiles(c->nx, c->ny, q.form, q);
     const size_t nyz = (size_t)c->ny * c->nz, nxz = (size_t)c->nx * c->nz, nxy = (size_t)c->nx * c->ny;
     const float4 *m = c->mur;
     const size_t step[6] = {nyz, nyz, nxz, nxz, nxy, nxy};

@@ -186,6 +186,10 @@ hipError_t launch_energy(const EnergyArgs &a, int storage, hipStream_t s);
 // One step of a grid in one launch, one cell per lane, with its Mur faces and
 // probe row (fdtd_cell.hip).  The field and id pointers lie fused_guard
 // elements before the arrays' origins; o0 = the guard in bytes.
+// Forms of cell_step: its state in the Infinity Cache; x neighbours from the
+// lanes beside instead of loads; the same with D past the cache; with D and
+// all but the loads of E^n past it.
+enum { kCellNear, kCellMid, kCellPart, kCellFar };
 struct CellArgs {
     const char *e0[3], *e1[3], *d0[3], *d1[3], *h0[3];   // E, D at levels n and n-1, H^{n-1/2}
     char *eT[3], *dT[3], *h1[3];                         // E, D at level n+1, H^{n+1/2}
@@ -199,18 +203,39 @@ struct CellArgs {
     uint32_t zmask;                // bit m: material m < 32 has a = g3 = +0 and its cells do not load levels n-1
     int bxl;                       // 5 or 6: 32 or 64 lanes of a 256-lane tile along x
     int hi_once;                   // the tiled step leaves the x-high faces to the Mur kernel (fused_mur_x 2)
+    int form;                      // kCellNear, ...
+    int flip;                      // planes from the highest down: every other step, so that a step starts where
+                                   // the last one ended
     const float4 *mur[6];          // launch_mur_coefs: x low, x high, y low, ...
     ProbeArgs p;                   // p.nprobe = 0: no probe row; p.field is not read
 };
 // Padded state (bytes of the 24 field arrays) up to which a context steps
-// with cell_step.  fp32 crosses the tiled launch where the Infinity Cache
-// (256 MB) no longer holds most of the state: 54 against 69 us at 285 MB
-// (160x160x116), 57.6 against 64.4 at 283 MB (128x128x180), even at 344 MB
-// (160x160x140, 79.5 against 78.7), 98 against 83 at 398 MB.  The 16-bit tiled
-// kernels are held by instructions: even at 566 MB (fp16 256x256x180, 155
-// against 153.5), 173 against 181 at 629 MB, 215 against 205 at 805 MB.
+// with cell_step.  Far past the Infinity Cache both launches wait for HBM, and
+// the tiled one keeps more of it in flight; what cell_step gains there is the
+// part of the state that the last step left in the cache.  fp32, us against
+// tiles: 2.2 GB 388 (397), 3.1 GB 556 (560), 4.0 GB 725 (704), 4.4 GB 812
+// (782).  fp16: 1.5 GB 333 (377), 4.3 GB 991 (1051), 6.4 GB 1555 (1544).
 constexpr int kCellMaxPlanes = 60000;   // planes and probe rows are blockIdx.y
-inline size_t cell_state_limit(size_t esz) { return esz == 2 ? 640000000 : 320000000; }
+inline size_t cell_state_limit(size_t esz) { return esz == 2 ? 6000000000 : 3200000000; }
+// Its form, in us (near, mid, part, far; means over six placements of the
+// state, which differ by up to 15 %).  fp32: 201 MB 30.2, 30.4, 38, 38; 246 MB
+// 34.4, 33.4, 44.9, 45.6; 285 MB 54.6, 51.5, 54.9, 55.9; 344 MB 68.6, 62.8,
+// 63.4, 65.5; 398 MB 85.2, 77.9, 76.8, 77.4; 491 MB 95.9, 89.6, 87.8, 88.1;
+// 679 MB 131, 126, 122, 119; 1.6 GB (one placement) 331, 310, 298, 293.  fp16:
+// 197 MB 43.4, 44.8, -, 57.8; 246 MB 74.5, 70.7, 65.3, 69.3; 340 MB 89.2, 84.0,
+// 78.0, 85.1; 403 MB 103, 95.9, 94.9, 99.1 (where E and H alone no longer fit
+// the cache); 566 MB 137, 129, 135, 135; 805 MB 194, 181, 183, 187; 1.1 GB 270,
+// 252, 249, 253; 1.5 GB 354, 327, 318, 320.
+inline int cell_form(size_t state, size_t esz)
+{
+    if (state <= 220000000) return kCellNear;
+    if (esz == 2) return state <= 400000000 ? kCellPart : state <= 1000000000 ? kCellMid : kCellFar;
+    return state <= 360000000 ? kCellMid : kCellFar;
+}
+// Padded state up to which cell_batch steps a batch's grid, in the near form,
+// in us against tiles: fp32 285 MB 54 (69), 344 MB 79.5 (78.7); 16-bit 566 MB
+// 155 (153.5).
+inline size_t cell_near_limit(size_t esz) { return esz == 2 ? 640000000 : 320000000; }
 // log2 of the lanes of its tiles along x: 64, or 32 where those leave clearly
 // fewer lanes idle (96 wide: 16.1 against 16.8 us in fp32, 13.0 against 13.8
 // in fp16; 160 wide, where 32 lanes would fill 20 % more: 35.2 against 37.5).
@@ -222,9 +247,9 @@ inline int cell_lanes_log2(int nx)
 // The tile geometry of a grid (CellArgs, CellInst) and the materials whose
 // cells skip levels n-1.
 template <typename A>
-inline void cell_tiles(int nx, int ny, A &a)
+inline void cell_tiles(int nx, int ny, int form, A &a)
 {
-    a.bxl = cell_lanes_log2(nx);
+    a.bxl = form == kCellNear ? cell_lanes_log2(nx) : 6;
     const int bx = 1 << a.bxl, by = 256 / bx;
     a.tiles_x = (nx + bx - 1) / bx;
     a.tx_mul = (uint32_t)(((1ull << 32) + a.tiles_x - 1) / a.tiles_x);

@@ -71,6 +71,22 @@ def test_cells_equal_tiles_f16_faces(shape):
         assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
 
 
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("shape,storage", [((65, 90, 420), F.STORE_F32), ((3, 300, 600), F.STORE_F32),
+                                           ((64, 64, 1300), F.STORE_F32), ((130, 127, 260), F.STORE_F32_FAST),
+                                           ((65, 90, 620), F.STORE_F16), ((130, 160, 1000), F.STORE_BF16)])
+def test_cells_equal_tiles_past_the_cache(shape, storage):
+    """States larger than the Infinity Cache, whose lanes take their x
+    neighbours from each other: one and more waves a row, a few lanes of one,
+    with cached and with streaming accesses."""
+    a, pa = _run(shape, storage, 4, False)
+    b, pb = _run(shape, storage, 4, True)
+    for key in a:
+        assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
+    assert np.array_equal(pa.view(np.uint64), pb.view(np.uint64))
+    assert np.isfinite(pa).all() and np.abs(pa).max() > 0
+
+
 @pytest.mark.parametrize("shape", [(3, 9, 5), (33, 20, 11), (64, 24, 9)])
 def test_cells_equal_the_oracle(shape):
     from oracle import oracle as O
