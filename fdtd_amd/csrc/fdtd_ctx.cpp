@@ -173,7 +173,7 @@ bool default_cell(const fdtd_ctx *c)
     FdtdExt d;
     fdtd_ext_defaults(&d);
     if (e.xcd_remap != d.xcd_remap) return false;
-    return c->nz <= kCellMaxPlanes && 24 * c->Np * c->esz <= cell_state_limit(c->esz);
+    return c->nz <= kCellMaxPlanes && 24 * c->Np * c->esz <= cell_state_limit(c->nx, c->esz);
 }
 
 // Launch shape a context takes for a grid, from launch-shape sweeps on

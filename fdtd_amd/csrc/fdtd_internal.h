@@ -212,11 +212,16 @@ struct CellArgs {
 // Padded state (bytes of the 24 field arrays) up to which a context steps
 // with cell_step.  Far past the Infinity Cache both launches wait for HBM, and
 // the tiled one keeps more of it in flight; what cell_step gains there is the
-// part of the state that the last step left in the cache.  fp32, us against
-// tiles: 2.2 GB 388 (397), 3.1 GB 556 (560), 4.0 GB 725 (704), 4.4 GB 812
-// (782).  fp16: 1.5 GB 333 (377), 4.3 GB 991 (1051), 6.4 GB 1555 (1544).
+// part of the state that the last step left in the cache, less where waves at
+// the rows' ends are part empty.  fp32, us against tiles: rows of whole waves
+// 2.2 GB 385 (397), 3.1 GB 549 (549), 4.0 GB 725 (704); others 1.1 GB 201
+// (202), 330x330x200 400 (391), 350x330x200 420 (405).  16 bits: 1.5 GB 340
+// (383), 3.9 GB 844 (981), 4.3 GB 991 (1051), 6.4 GB 1555 (1544).
 constexpr int kCellMaxPlanes = 60000;   // planes and probe rows are blockIdx.y
-inline size_t cell_state_limit(size_t esz) { return esz == 2 ? 6000000000 : 3200000000; }
+inline size_t cell_state_limit(int nx, size_t esz)
+{
+    return esz == 2 ? 6000000000 : nx % 64 == 0 ? 3200000000 : 1200000000;
+}
 // Its form, in us (near, mid, part, far; means over six placements of the
 // state, which differ by up to 15 %).  fp32: 201 MB 30.2, 30.4, 38, 38; 246 MB
 // 34.4, 33.4, 44.9, 45.6; 285 MB 54.6, 51.5, 54.9, 55.9; 344 MB 68.6, 62.8,
