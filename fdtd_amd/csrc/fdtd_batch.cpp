@@ -64,7 +64,7 @@ Layout layout_of(int nx, int ny, int nz, int storage, int nmat, int jz_n, int np
     L.Np = (size_t)L.plane * nz;
     // Channel stagger between the 24 field arrays of large grids (as in a
     // single context); small grids are not worth the memory.
-    L.skew = L.Np >= (size_t)1 << 20 ? 65536 : 0;
+    L.skew = L.Np >= (size_t)1 << 20 ? 1088 : 0;
     L.guard = fused_guard(L.pitch, L.plane);
     L.jz_n = jz_n;
     size_t o = 0;

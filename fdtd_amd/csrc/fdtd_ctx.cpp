@@ -23,8 +23,8 @@ namespace {
 // Extra elements between consecutive field arrays in the blob: staggers the
 // arrays' starts across HBM channels, also where a plane is a power of two
 // (256^3 fp32, us a step: 327 with 0, 1024 or 65536, 280 to 285 with 64, 4160
-// or this; 320x320x880 in tiles 1553 with 65536, 1535).
-constexpr size_t kArraySkew = 33856;
+// or this; 320x320x880 in tiles 1553 with 65536, 1529).
+constexpr size_t kArraySkew = 1088;
 
 }  // namespace
 
