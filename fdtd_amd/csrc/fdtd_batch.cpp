@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <tuple>
 #include <vector>
 
@@ -497,8 +498,8 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     const int nx = p->nx, ny = p->ny, nz = p->nz;
     const size_t N = (size_t)nx * ny * nz;
     if (in->ids)
-        for (size_t t = 0; t < N; t++)
-            if (in->ids[t] >= in->nmat) return fdtd_fail(FDTD_ERANGE, "material id %d at cell %zu >= nmat %d", in->ids[t], t, in->nmat);
+        if (const size_t t = fdtd_first_bad_id(in->ids, N, in->nmat); t < N)
+            return fdtd_fail(FDTD_ERANGE, "material id %d at cell %zu >= nmat %d", in->ids[t], t, in->nmat);
     if (b->step + in->steps >= INT_MAX) return fdtd_fail(FDTD_ERANGE, "batch step counter would overflow");
     int slot = -1;
     for (int s = 0; s < (int)b->in.size(); s++)
@@ -523,8 +524,9 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
 
     char *base = b->arena_base + off;
     // ids with source bits, coefficient table, stored waveform, Mur planes, probes
-    std::vector<unsigned char> ids(L.Np, 0);
-    if (in->ids) fdtd_pitch_bytes(in->ids, nx, (size_t)ny * nz, L.pitch, ids.data());
+    std::unique_ptr<unsigned char[]> ids(new unsigned char[L.Np]);
+    if (in->ids) fdtd_pitch_bytes(in->ids, nx, (size_t)ny * nz, L.pitch, ids.get());
+    else memset(ids.get(), 0, L.Np);
     for (int s = 0; s < in->nsrc; s++) {
         const int *q = in->src_xyz + 3 * s;
         ids[(size_t)q[2] * L.plane + (size_t)q[1] * L.pitch + q[0]] |= kSourceBit;
@@ -535,30 +537,23 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     for (int t = 0; t < jz_n; t++) jz[t] = fdtd_jz_stored(in->jz[t], e.storage, p->eps0, I.sD);
     const size_t rps[6] = {(size_t)2 * ny * nz, (size_t)nx * 2 * nz, (size_t)nx * ny * 2,
                            (size_t)2 * ny * nz, (size_t)nx * 2 * nz, (size_t)nx * ny * 2};
-    std::vector<float> ones;
-    // x-face Mur coefficients from the rp planes (or vacuum)
-    std::vector<float4> murx(2 * (size_t)ny * nz);
-    {
-        std::vector<float> one_x((size_t)2 * ny * nz, 1.0f);
-        mur_x_coefs(ny, nz, p->dt, p->dx, p->mu0, p->eps0, in->rp[0] ? in->rp[0] : one_x.data(),
-                    in->rp[3] ? in->rp[3] : one_x.data(), murx.data(), murx.data() + (size_t)ny * nz);
-    }
     hipError_t he = hipMemsetAsync(base, 0, L.ids + L.Np + 2 * (size_t)L.guard, b->up);
-    if (he == hipSuccess)
-        he = hipMemcpyAsync(base + L.murx, murx.data(), sizeof(float4) * murx.size(), hipMemcpyHostToDevice, b->up);
     if (he == hipSuccess) he = hipMemsetAsync(base + L.out, 0, L.out_bytes, b->up);
-    if (he == hipSuccess) he = hipMemcpyAsync(base + L.ids + L.guard, ids.data(), L.Np, hipMemcpyHostToDevice, b->up);
+    if (he == hipSuccess) he = hipMemcpyAsync(base + L.ids + L.guard, ids.get(), L.Np, hipMemcpyHostToDevice, b->up);
     if (he == hipSuccess) he = hipMemcpyAsync(base + L.lut, lut.data(), sizeof(MatCoef) * in->nmat, hipMemcpyHostToDevice, b->up);
     if (he == hipSuccess && jz_n > 0) he = hipMemcpyAsync(base + L.jz, jz.data(), sizeof(float) * jz_n, hipMemcpyHostToDevice, b->up);
+    // The rp planes (vacuum where none are given) and from them, on the device, the x faces' Mur coefficients.
+    MurCoefArgs mc{};
     for (int r = 0; r < 6 && he == hipSuccess; r++) {
-        const float *src = in->rp[r];
-        if (!src) {
-            ones.assign(rps[r], 1.0f);
-            src = ones.data();
-        }
-        he = hipMemcpyAsync(base + L.rp[r], src, rps[r] * sizeof(float), hipMemcpyHostToDevice, b->up);
-        if (he == hipSuccess && !in->rp[r]) he = hipStreamSynchronize(b->up);  // `ones` is reused
+        mc.rp[r] = (const float *)(base + L.rp[r]);
+        he = in->rp[r] ? hipMemcpyAsync(base + L.rp[r], in->rp[r], rps[r] * sizeof(float), hipMemcpyHostToDevice, b->up)
+                       : hipMemsetD32Async((hipDeviceptr_t)(base + L.rp[r]), 0x3f800000, rps[r], b->up);   // 1.0f
     }
+    mc.out = (float4 *)(base + L.murx);
+    mc.nx = nx; mc.ny = ny; mc.nz = nz;
+    mc.dt = p->dt; mc.mu0 = p->mu0; mc.eps0 = p->eps0;
+    mc.h[0] = p->dx; mc.h[1] = p->dy; mc.h[2] = p->dz;
+    if (he == hipSuccess) he = launch_mur_coefs(mc, 2, b->up);
     if (he == hipSuccess && in->nprobe > 0)
         he = hipMemcpyAsync(base + L.probes, in->probes, sizeof(int) * 4 * in->nprobe, hipMemcpyHostToDevice, b->up);
     if (he == hipSuccess) he = hipStreamSynchronize(b->up);

@@ -626,10 +626,10 @@ __global__ __launch_bounds__(kCellBlock) void mur_coefs(const MurCoefArgs a)
 
 }  // namespace
 
-hipError_t launch_mur_coefs(const MurCoefArgs &a, hipStream_t s)
+hipError_t launch_mur_coefs(const MurCoefArgs &a, int faces, hipStream_t s)
 {
     const long long m = std::max({(long long)a.ny * a.nz, (long long)a.nx * a.nz, (long long)a.nx * a.ny});
-    mur_coefs<<<dim3((unsigned)((m + kCellBlock - 1) / kCellBlock), 6), kCellBlock, 0, s>>>(a);
+    mur_coefs<<<dim3((unsigned)((m + kCellBlock - 1) / kCellBlock), (unsigned)faces), kCellBlock, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -4,6 +4,7 @@
 // the same grid stepped inside a batch see identical coefficients.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -322,24 +323,17 @@ void fdtd_pitch_bytes(const unsigned char *in, int nx, size_t rows, int pitch, u
     }
 }
 
-void mur_x_coefs(int ny, int nz, float dt, float hx, float mu0, float eps0, const float *rpx0, const float *rpxEnd,
-                 float4 *out0, float4 *out1)
+size_t fdtd_first_bad_id(const unsigned char *ids, size_t n, int nmat)
 {
-    auto one = [&](float rpf, float rpn) {
-        const float sf = std::sqrt(mu0 * eps0 * rpf), sn = std::sqrt(mu0 * eps0 * rpn);
-        float4 c;
-        c.x = 1 / (dt + hx * sf);
-        c.y = dt - hx * sn;
-        c.z = dt + hx * sn;
-        c.w = dt - hx * sf;
-        return c;
-    };
-    for (int k = 0; k < nz; k++)
-        for (int j = 0; j < ny; j++) {
-            const size_t r = ((size_t)k * ny + j) * 2, q = (size_t)k * ny + j;
-            out0[q] = one(rpx0[r], rpx0[r + 1]);
-            out1[q] = one(rpxEnd[r + 1], rpxEnd[r]);
-        }
+    for (size_t t = 0; t < n; t += 4096) {
+        const size_t e = std::min(n, t + 4096);
+        unsigned char top = 0;   // no exit inside: 16 ids an instruction
+        for (size_t q = t; q < e; q++) top = std::max(top, ids[q]);
+        if (top >= nmat)
+            while (t < n && ids[t] < nmat) t++;
+        if (top >= nmat) return t;
+    }
+    return n;
 }
 
 extern "C" int fdtd_stream_probe_layout(long long cells, int row, int blocks, int reps, double *gbs,

@@ -208,7 +208,7 @@ hipError_t set_mur(fdtd_ctx *c)
     a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
     a.dt = c->dt; a.mu0 = c->mu0; a.eps0 = c->eps0;
     a.h[0] = c->dx; a.h[1] = c->dy; a.h[2] = c->dz;
-    const hipError_t e = launch_mur_coefs(a, nullptr);
+    const hipError_t e = launch_mur_coefs(a, 6, nullptr);
     return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
 }
 
@@ -351,8 +351,8 @@ extern "C" int fdtd_ctx_set_materials(fdtd_ctx *c, const unsigned char *ids, int
 {
     if (!c || !ids || !table) return fdtd_fail(FDTD_EINVAL, "null argument");
     if (nmat < 1 || nmat > kMaxMaterials) return fdtd_fail(FDTD_ERANGE, "nmat %d not in [1,%d]", nmat, kMaxMaterials);
-    for (size_t t = 0; t < c->N; t++)
-        if (ids[t] >= nmat) return fdtd_fail(FDTD_ERANGE, "material id %d at cell %zu >= nmat %d", ids[t], t, nmat);
+    if (const size_t t = fdtd_first_bad_id(ids, c->N, nmat); t < c->N)
+        return fdtd_fail(FDTD_ERANGE, "material id %d at cell %zu >= nmat %d", ids[t], t, nmat);
     // the device ids first: the table changes only once they match it
     std::vector<unsigned char> prev(ids, ids + c->N);
     c->ids_host.swap(prev);

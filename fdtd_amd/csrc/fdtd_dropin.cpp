@@ -55,8 +55,8 @@ int dropin_check(const FdtdParams *p, const FdtdExt *ext, const FdtdInstance *in
     if (int rc = fdtd_check_probes(nx, ny, nz, in->nprobe, in->probes)) return rc;
     if (in->ids) {
         const size_t N = (size_t)nx * ny * nz;
-        for (size_t t = 0; t < N; t++)
-            if (in->ids[t] >= in->nmat) return fdtd_fail(FDTD_ERANGE, "material id %d >= nmat", in->ids[t]);
+        if (const size_t t = fdtd_first_bad_id(in->ids, N, in->nmat); t < N)
+            return fdtd_fail(FDTD_ERANGE, "material id %d >= nmat", in->ids[t]);
     }
     *out = e;
     return 0;

@@ -64,7 +64,7 @@ struct StepArgs {
     // Mur x faces updated inside the fused kernel (fused_mur_x): 0 none, 1
     // all four (Ey, Ez at i = 0 and nx-1), 2 the two at i = 0 only.
     int mur_x;
-    const float4 *murx0, *murx1;    // per (k, j) coefficients of the x-low / x-high faces (mur_x_coefs)
+    const float4 *murx0, *murx1;    // per (k, j) coefficients of the x-low / x-high faces (launch_mur_coefs)
     int cpl;                        // cells per lane: 1, or 2 for 16-bit storage (128-cell tiles)
     int txw;                        // threads per tile row with one cell per lane: 64 or 128
     // Exact fp32 form: a half wave (32 cells of a tile row) whose cells all
@@ -79,14 +79,10 @@ struct StepArgs {
 // reference's expression (fdtd_calculations.cu:216-428) rounds
 // them: q = 1/(dt + h sqrt(mu0 eps0 rp_face)), A = dt - h sqrt(mu0 eps0
 // rp_nb), B = dt + h sqrt(mu0 eps0 rp_nb), C = dt - h sqrt(mu0 eps0
-// rp_face).  mur_x_coefs: planes of ny*nz entries, (k, j) order: out0 from
-// rpx0 (face index 0), out1 from rpxEnd (face index 1).
-void mur_x_coefs(int ny, int nz, float dt, float hx, float mu0, float eps0, const float *rpx0, const float *rpxEnd,
-                 float4 *out0, float4 *out1);
-
-// The same on the device for the six faces of a grid, from its rp planes in
-// fdtd_ctx_set_rp's order: out holds x low, x high in (k, j) order, y low, y
-// high in (k, i) order, z low, z high in (j, i) order, one after the other.
+// rp_face).  launch_mur_coefs: of the first `faces` of a grid's six, from its rp
+// planes in fdtd_ctx_set_rp's order: out holds x low, x high in (k, j) order,
+// y low, y high in (k, i) order, z low, z high in (j, i) order, one after the
+// other.
 struct MurCoefArgs {
     const float *rp[6];
     float4 *out;
@@ -97,7 +93,7 @@ inline size_t mur_coef_count(int nx, int ny, int nz)
 {
     return 2 * ((size_t)ny * nz + (size_t)nx * nz + (size_t)nx * ny);
 }
-hipError_t launch_mur_coefs(const MurCoefArgs &a, hipStream_t s);
+hipError_t launch_mur_coefs(const MurCoefArgs &a, int faces, hipStream_t s);
 
 // Which Mur x faces the fused kernel takes over.  The x-high faces need the
 // cell at i = nx-2 from the face's wave: E^{n+1}_z from the previous lane
@@ -565,6 +561,8 @@ void fdtd_from_storage(int storage, const void *in, size_t n, double factor, flo
 void fdtd_to_storage_pitched(int storage, const float *in, int nx, size_t rows, int pitch, double factor, void *out);
 void fdtd_from_storage_pitched(int storage, const void *in, int nx, size_t rows, int pitch, double factor, float *out);
 void fdtd_pitch_bytes(const unsigned char *in, int nx, size_t rows, int pitch, unsigned char *out);
+// First cell whose material id is not below nmat; n: none.
+size_t fdtd_first_bad_id(const unsigned char *ids, size_t n, int nmat);
 int fdtd_check_ext(const FdtdExt &e);
 
 // Phantom input (fdtd_phantom.cpp).  phantom_read_table fills a 95-row

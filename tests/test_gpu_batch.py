@@ -190,3 +190,11 @@ def test_batch_reference_debye_mode():
         assert_same(b, i, x, r, f"debye case {q}")
     assert np.isfinite(refs[0][1]).all()
     b.close()
+
+
+@pytest.mark.parametrize("cell", [0, 1, 4095, 4096, 4097, 8191, 8192, 17 * 19 * 29 - 1])   # 4096 cells are checked at a time
+def test_bad_material_id_names_its_cell(cell):
+    x = make_case(77, (17, 19, 29), 3, 4)
+    x.ids.reshape(-1)[[cell, -1]] = 3
+    with F.Batch(64 << 20) as b, pytest.raises(F.FdtdError, match=f"material id 3 at cell {cell} >= nmat 3"):
+        b.add(x)
