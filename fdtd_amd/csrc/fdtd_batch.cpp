@@ -39,11 +39,12 @@ struct DevTables {
 // Padded state of the grids that cell_batch steps together, and the steps it
 // takes with one group before it goes on to the next: a group's state stays
 // in the Infinity Cache (256 MB) meanwhile.  Twelve fp32 grids around 96^3
-// (1.1 GB) on MI355X, in Gcell-updates/s: 51.5 as set; 45.3 with groups of
-// 120 MB, 48.8 with 180, 42.3 with 300, 38.3 with 400; 45.6 with 8 steps at a
-// time, 52.6 with 64; 38.8 where field_step_batch steps all of them together.
+// (1.1 GB) on MI355X, in Gcell-updates/s: 53.0 as set; 51.6 with groups of
+// 210 MB, 53.1 with 250, 43 with 300, 39 with 400; 45.6 with 8 steps at a time,
+// 52.0 with 32, 53.5 with 128 (a grid that ends keeps its place in the launches
+// of those steps); 38.8 where fused_batch steps all of them together.
 constexpr size_t kCellGroupBytes = 240000000;
-constexpr int kCellRunSteps = 32;
+constexpr int kCellRunSteps = 64;
 
 // Byte layout of one grid's arena region.
 struct Layout {
