@@ -622,7 +622,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.o0 = (uint32_t)gb;
     c.sy = (uint32_t)(L.pitch * L.esz);
     c.sz = (uint32_t)(L.plane * L.esz);
-    cell_tiles(nx, ny, kCellNear, c);
+    cell_tiles(nx, ny, kCellNear, L.esz, c);
     for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
     c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : 0;
     c.nprobe = d.nprobe;

@@ -36,7 +36,7 @@
 //
 // Measured on MI355X, whole steps, against fused_step and the Mur launch
 // (us): fp32 24^3 5.7 (15.1), 64^3 7.4 (16.6), 100^3 20.5 (31.2), 128^3 28
-// (47), 160x160x100 34 (60), 151x138x188 77 (83), 256^3 280 (304); fp16 64^3
+// (47), 160x160x100 34 (60), 151x138x188 75 (83), 256^3 280 (304); fp16 64^3
 // 6.9 (18.0), 96x121x77 13.4 (27.6), 256^3 181 (206), 320x320x300 318 (377).
 // 128^3 moves 178 MB, 6.4 TB/s at the L2's far side, where a stream of the same
 // arrays reaches 8.0; with 4 waves a SIMD instead of 7 it takes as long.  Past
@@ -107,14 +107,20 @@ __device__ __forceinline__ float at_uniform(const char *p, uint32_t b)
     }
 }
 
-// The value of the lane below (above); the wave's first (last) lane gets `end`.
-__device__ __forceinline__ float lane_below(float v, float end)
+// The value of the lane below (above) in a wave's row of 1 << BXL lanes; the
+// first (last) lane of the row gets `end`, in the wave's second row `end1`.
+template <int BXL>
+__device__ __forceinline__ float lane_below(float v, float end, float end1)
 {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x138, 0xf, 0xf, false));
+    const float r = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x138, 0xf, 0xf, false));
+    return BXL < 6 && (threadIdx.x & 63) == 32 ? end1 : r;
 }
-__device__ __forceinline__ float lane_above(float v, float end)
+template <int BXL>
+__device__ __forceinline__ float lane_above(float v, float end, float end1)
 {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x130, 0xf, 0xf, false));
+    const float r = __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(BXL < 6 ? end1 : end), __float_as_int(v), 0x130, 0xf, 0xf, false));
+    return BXL < 6 && (threadIdx.x & 63) == 31 ? end : r;
 }
 
 // A value that the next step does not read soon enough to find it in the
@@ -344,15 +350,19 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     v.hx_km = at<T>(qx, okm); v.hy_km = at<T>(qy, okm);
     // Neighbours along x: near, loads of their own; else from the lanes beside
     // (below), and past the wave's ends from these.
-    float end[11] = {};
+    float end[2][11] = {};
     if constexpr (LANES) {
-        const uint32_t lo = C.o0() + (uint32_t)k * szb + (uint32_t)jw * syb + (uint32_t)((i0 - 1) * (int)ES);
-        const uint32_t hi = lo + (BX + 1) * ES;
-        end[0] = at_uniform<T>(px, lo); end[1] = at_uniform<T>(py, lo); end[2] = at_uniform<T>(pz, lo);
-        end[3] = at_uniform<T>(py, hi); end[4] = at_uniform<T>(pz, hi);
-        end[5] = at_uniform<T>(px, lo + syb); end[6] = at_uniform<T>(py, hi - syb);
-        end[7] = at_uniform<T>(px, lo + szb); end[8] = at_uniform<T>(pz, hi - szb);
-        end[9] = at_uniform<T>(qy, lo); end[10] = at_uniform<T>(qz, lo);
+        const uint32_t first = C.o0() + (uint32_t)k * szb + (uint32_t)((i0 - 1) * (int)ES);
+#pragma unroll
+        for (int r = 0; r < (BXL < 6 ? 2 : 1); r++) {
+            const uint32_t lo = first + (uint32_t)min(jw + r, ny - 1) * syb, hi = lo + (BX + 1) * ES;
+            float *e = end[r];
+            e[0] = at_uniform<T>(px, lo); e[1] = at_uniform<T>(py, lo); e[2] = at_uniform<T>(pz, lo);
+            e[3] = at_uniform<T>(py, hi); e[4] = at_uniform<T>(pz, hi);
+            e[5] = at_uniform<T>(px, lo + syb); e[6] = at_uniform<T>(py, hi - syb);
+            e[7] = at_uniform<T>(px, lo + szb); e[8] = at_uniform<T>(pz, hi - szb);
+            e[9] = at_uniform<T>(qy, lo); e[10] = at_uniform<T>(qz, lo);
+        }
     }
     if constexpr (!LANES) {
         v.ex_im = at<T>(px, o, -1); v.ey_im = at<T>(py, o, -1); v.ez_im = at<T>(pz, o, -1);
@@ -383,11 +393,13 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         v.dxm = at_once<T, ND>(C.d1(0), o); v.dym = at_once<T, ND>(C.d1(1), o); v.dzm = at_once<T, ND>(C.d1(2), o);
     }
     if constexpr (LANES) {   // (after the loads above are out: each of these waits for its operand)
-        v.ex_im = lane_below(v.ex, end[0]); v.ey_im = lane_below(v.ey, end[1]); v.ez_im = lane_below(v.ez, end[2]);
-        v.ey_ip = lane_above(v.ey, end[3]); v.ez_ip = lane_above(v.ez, end[4]);
-        v.ex_jp_im = lane_below(v.ex_jp, end[5]); v.ey_jm_ip = lane_above(v.ey_jm, end[6]);
-        v.ex_kp_im = lane_below(v.ex_kp, end[7]); v.ez_km_ip = lane_above(v.ez_km, end[8]);
-        v.hy_im = lane_below(v.hy, end[9]); v.hz_im = lane_below(v.hz, end[10]);
+        auto below = [&](float x, int q) { return lane_below<BXL>(x, end[0][q], end[1][q]); };
+        auto above = [&](float x, int q) { return lane_above<BXL>(x, end[0][q], end[1][q]); };
+        v.ex_im = below(v.ex, 0); v.ey_im = below(v.ey, 1); v.ez_im = below(v.ez, 2);
+        v.ey_ip = above(v.ey, 3); v.ez_ip = above(v.ez, 4);
+        v.ex_jp_im = below(v.ex_jp, 5); v.ey_jm_ip = above(v.ey_jm, 6);
+        v.ex_kp_im = below(v.ex_kp, 7); v.ez_km_ip = above(v.ez_km, 8);
+        v.hy_im = below(v.hy, 9); v.hz_im = below(v.hz, 10);
     }
 
     const float chx = C.ch(0), chy = C.ch(1), chz = C.ch(2);
@@ -593,11 +605,17 @@ __global__ __launch_bounds__(kCellBlock) void cell_batch(const CellInst *inst, c
 template <typename T, bool EXACT>
 hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
 {
-    const void *k = c.form == kCellFar   ? (const void *)cell_step<T, EXACT, 6, kCellFar>
-                    : c.form == kCellPart ? (const void *)cell_step<T, EXACT, 6, kCellPart>
-                    : c.form == kCellMid ? (const void *)cell_step<T, EXACT, 6, kCellMid>
-                    : c.bxl == 6         ? (const void *)cell_step<T, EXACT, 6, kCellNear>
-                                         : (const void *)cell_step<T, EXACT, 5, kCellNear>;
+    const void *wide[] = {(const void *)cell_step<T, EXACT, 6, kCellNear>, (const void *)cell_step<T, EXACT, 6, kCellMid>,
+                          (const void *)cell_step<T, EXACT, 6, sizeof(T) == 2 ? kCellPart : kCellFar>,
+                          (const void *)cell_step<T, EXACT, 6, kCellFar>};
+    const void *k = wide[c.form];
+    if (c.bxl == 5) {   // cell_lanes_log2, cell_form: fp32 near, mid and far, 16 bits near
+        k = (const void *)cell_step<T, EXACT, 5, kCellNear>;
+        if constexpr (sizeof(T) == 4) {
+            if (c.form == kCellMid) k = (const void *)cell_step<T, EXACT, 5, kCellMid>;
+            if (c.form == kCellFar) k = (const void *)cell_step<T, EXACT, 5, kCellFar>;
+        }
+    }
     const unsigned gx = 8u * (unsigned)c.run;
     const unsigned waves = kCellBlock / 64, pb = ((unsigned)c.p.nprobe + waves - 1) / waves;
     const dim3 grid(gx, (unsigned)c.nz + (pb + gx - 1) / gx);

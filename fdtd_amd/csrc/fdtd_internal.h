@@ -210,13 +210,13 @@ struct CellArgs {
 // the tiled one keeps more of it in flight; what cell_step gains there is the
 // part of the state that the last step left in the cache, less where waves at
 // the rows' ends are part empty.  fp32, us against tiles: rows of whole waves
-// 2.2 GB 385 (397), 3.1 GB 549 (549), 4.0 GB 725 (704); others 1.1 GB 201
-// (202), 330x330x200 400 (391), 350x330x200 420 (405).  16 bits: 1.5 GB 340
+// 2.2 GB 387 (396), 3.1 GB 570 (565), 4.0 GB 725 (704); others 1.1 GB 203
+// (208), 300^3 504 (491), 350x330x200 421 (414).  16 bits: 1.5 GB 340
 // (383), 3.9 GB 844 (981), 4.3 GB 991 (1051), 6.4 GB 1555 (1544).
 constexpr int kCellMaxPlanes = 60000;   // planes and probe rows are blockIdx.y
 inline size_t cell_state_limit(int nx, size_t esz)
 {
-    return esz == 2 ? 6000000000 : nx % 64 == 0 ? 3200000000 : 1200000000;
+    return esz == 2 ? 6000000000 : nx % 64 == 0 ? 2600000000 : 1200000000;
 }
 // Its form, in us (near, mid, part, far; means over six placements of the
 // state, which differ by up to 15 %).  fp32: 201 MB 30.2, 30.4, 38, 38; 246 MB
@@ -237,20 +237,25 @@ inline int cell_form(size_t state, size_t esz)
 // in us against tiles: fp32 285 MB 54 (69), 344 MB 79.5 (78.7); 16-bit 566 MB
 // 155 (153.5).
 inline size_t cell_near_limit(size_t esz) { return esz == 2 ? 640000000 : 320000000; }
-// log2 of the lanes of its tiles along x: 64, or 32 where those leave clearly
-// fewer lanes idle (96 wide: 16.1 against 16.8 us in fp32, 13.0 against 13.8
-// in fp16; 160 wide, where 32 lanes would fill 20 % more: 35.2 against 37.5).
-inline int cell_lanes_log2(int nx)
+// log2 of the lanes of its tiles along x: 64, or 32.  Near: 32 where 64 leave
+// clearly more lanes idle (96 wide: 16.1 against 16.8 us in fp32, 13.0 against
+// 13.8 in fp16; 160 wide, where 32 lanes would fill 20 % more: 35.2 against
+// 37.5).  Else in fp32 wherever they take fewer lanes (90x150x300 88 against 101
+// us, 151x138x188 77.8 against 81.1, 210x150x150 84.2 against 87.1; as many:
+// 256^3 299 against 291); not for 16-bit fields, whose second row's ends cost
+// more (71x79x1000 140 against 119).
+inline int cell_lanes_log2(int nx, int form, size_t esz)
 {
+    if (form != kCellNear) return esz == 4 && ((nx + 31) / 32) % 2 ? 5 : 6;
     const double e6 = (double)nx / (64 * ((nx + 63) / 64)), e5 = (double)nx / (32 * ((nx + 31) / 32));
     return e6 < 0.8 * e5 ? 5 : 6;
 }
 // The tile geometry of a grid (CellArgs, CellInst) and the materials whose
 // cells skip levels n-1.
 template <typename A>
-inline void cell_tiles(int nx, int ny, int form, A &a)
+inline void cell_tiles(int nx, int ny, int form, size_t esz, A &a)
 {
-    a.bxl = form == kCellNear ? cell_lanes_log2(nx) : 6;
+    a.bxl = cell_lanes_log2(nx, form, esz);
     const int bx = 1 << a.bxl, by = 256 / bx;
     a.tiles_x = (nx + bx - 1) / bx;
     a.tx_mul = (uint32_t)(((1ull << 32) + a.tiles_x - 1) / a.tiles_x);

@@ -74,11 +74,13 @@ def test_cells_equal_tiles_f16_faces(shape):
 @pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
 @pytest.mark.parametrize("shape,storage", [((65, 90, 420), F.STORE_F32), ((3, 300, 600), F.STORE_F32),
                                            ((64, 64, 1300), F.STORE_F32), ((130, 127, 260), F.STORE_F32_FAST),
-                                           ((65, 90, 620), F.STORE_F16), ((130, 160, 1000), F.STORE_BF16)])
+                                           ((65, 90, 620), F.STORE_F16), ((130, 160, 1000), F.STORE_BF16),
+                                           ((70, 91, 420), F.STORE_F32), ((64, 64, 800), F.STORE_F32),
+                                           ((100, 121, 900), F.STORE_F16)])
 def test_cells_equal_tiles_past_the_cache(shape, storage):
     """States larger than the Infinity Cache, whose lanes take their x
     neighbours from each other: one and more waves a row, a few lanes of one,
-    with cached and with streaming accesses."""
+    two rows a wave, a single last row, with cached and with streaming accesses."""
     a, pa = _run(shape, storage, 4, False)
     b, pb = _run(shape, storage, 4, True)
     for key in a:
