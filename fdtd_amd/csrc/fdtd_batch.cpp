@@ -662,7 +662,7 @@ extern "C" int fdtd_batch_run(fdtd_batch *b, int steps, hipStream_t stream)
     int left = steps;
     while (left > 0) {
         if (int rc = sync_tables(b, stream)) return rc;
-        const int g = std::min(left, b->mask ? b->graph_steps : std::max(b->graph_steps, kCellRunSteps));
+        const int g = std::min(left, b->groups.empty() ? b->graph_steps : std::max(b->graph_steps, kCellRunSteps));
         if (b->running.empty()) {
             // nothing runs: the counter moves on the host; the next table
             // upload carries it to the device
@@ -672,9 +672,10 @@ extern "C" int fdtd_batch_run(fdtd_batch *b, int steps, hipStream_t stream)
         }
         b->ran = true;
         b->last = stream;
-        if (b->mask) {
+        for (int t = 0, n; b->mask && t < g; t += n) {
             hipGraphExec_t exec = nullptr;
-            if (int rc = graph_for(b, b->mask, g, &exec)) return rc;
+            n = std::min(g - t, b->graph_steps);
+            if (int rc = graph_for(b, b->mask, n, &exec)) return rc;
             HIP_TRY(hipGraphLaunch(exec, stream));
         }
         for (const auto &G : b->groups)
