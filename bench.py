@@ -308,11 +308,14 @@ def main():
     achieved = bpc * cells * per_launch / kavg_s / 1e9
     shape = ctx.launch_shape()
     launch = f"{shape['tile_x']}x{shape['tile_y']}x{shape['kchunk']}"
+    by_cells = ctx.by_cells()
     traffic, traffic_src = None, None
     if a.traffic_kib:
         traffic, traffic_src = int((a.traffic_kib[0] + a.traffic_kib[1]) * 1024), "--traffic-kib"
     elif per_launch != 1:
         traffic, traffic_src = None, "no counter profile of the two-step kernel under profiles/"
+    elif by_cells:
+        traffic, traffic_src = None, f"no counter profile of cell_step on {w.name} under profiles/"
     else:
         traffic, prof = profiled_traffic(w.name, a.storage, launch, bool(a.load_zero_terms), remap)
         traffic_src = (os.path.relpath(prof, ROOT) + f" (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE, 1 GiB copy "
@@ -335,13 +338,13 @@ def main():
                  else "synthetic (seeded phantom)"),
         "config": {"workload": w.name, "grid": [nx, ny, nz], "cells": cells, "materials": int(w.table.shape[0]),
                    "sources": int(w.sources.shape[0]), "probes": int(w.probes.shape[0]),
-                   "slice_every": w.slice_every, "launch": shape, "xcd_remap": remap, "time_steps": a.time_steps,
+                   "slice_every": w.slice_every, "launch": "one lane per cell" if by_cells else shape, "xcd_remap": remap, "time_steps": a.time_steps,
                    "autotuned": tuned is not None,
                    "timed_steps": [first, first + a.steps], "untimed_advance": a.advance,
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": "fused_step" if per_launch == 1 else "fused_step2",
+                     "kernel": "cell_step" if by_cells else "fused_step" if per_launch == 1 else "fused_step2",
                      "steps_per_launch": per_launch, "kernel_avg_ms": round(kms / launches, 5),
                      "launches_timed": launches,
                      "timed_launch_steps": [first + a.steps, first + a.steps + launches * per_launch],

@@ -47,7 +47,7 @@ EXPORTS = {
                    "fdtd_ctx_set_sources", "fdtd_ctx_set_probes", "fdtd_ctx_set_slices", "fdtd_ctx_set_field",
                    "fdtd_ctx_get_field", "fdtd_ctx_field_ptr", "fdtd_step_fused", "fdtd_run",
                    "fdtd_ctx_steps_done", "fdtd_ctx_snapshot", "fdtd_probe_read", "fdtd_probe_peak_units", "fdtd_slices_read",
-                   "fdtd_ctx_launch_shape", "fdtd_default_launch_shape",
+                   "fdtd_ctx_launch_shape", "fdtd_ctx_by_cells", "fdtd_default_launch_shape",
                    "fdtd_ctx_set_timing", "fdtd_ctx_kernel_time", "fdtd_ctx_timed_steps", "fdtd_ctx_scales", "fdtd_ctx_layout",
                    "fdtd_ctx_set_energy", "fdtd_energy_read", "fdtd_ctx_save", "fdtd_ctx_load",
                    "fdtd_ctx_autotune", "fdtd_ctx_halo_bytes", "fdtd_ctx_halo_pack", "fdtd_ctx_halo_unpack",
@@ -171,6 +171,7 @@ def lib():
         L.fdtd_probe_peak_units.argtypes = [vp, vp, i]
         L.fdtd_slices_read.argtypes = [vp, vp, vp, i]
         L.fdtd_ctx_launch_shape.argtypes = [vp, vp, vp, vp, vp]
+        L.fdtd_ctx_by_cells.argtypes = [vp]
         L.fdtd_default_launch_shape.argtypes = [C.POINTER(FdtdParams), C.POINTER(FdtdExt), i, vp, vp, vp, vp]
         L.fdtd_ctx_set_timing.argtypes = [vp, i, i]
         L.fdtd_ctx_kernel_time.argtypes = [vp, C.POINTER(C.c_double), C.POINTER(C.c_int)]
@@ -470,6 +471,10 @@ class Context:
         v = [C.c_int() for _ in range(4)]
         check(lib().fdtd_ctx_launch_shape(self._h, *[C.byref(x) for x in v]), "launch_shape")
         return dict(tile_x=v[0].value, tile_y=v[1].value, kchunk=v[2].value, blocks=v[3].value)
+
+    def by_cells(self):
+        """Whether steps run with one lane per cell, not in tiles of launch_shape."""
+        return lib().fdtd_ctx_by_cells(self._h) == 1
 
 
 def make_ext(debye=DEBYE_FIXED, jz_mode=JZ_STEP, jz_limit=0, storage=STORE_F32, scales=(0.0, 0.0, 0.0),

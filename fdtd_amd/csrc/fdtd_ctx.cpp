@@ -886,6 +886,8 @@ extern "C" int fdtd_ctx_launch_shape(fdtd_ctx *c, int *tile_x, int *tile_y, int 
     return 0;
 }
 
+extern "C" int fdtd_ctx_by_cells(fdtd_ctx *c) { return c ? (c->cell ? 1 : 0) : FDTD_EINVAL; }
+
 extern "C" int fdtd_ctx_set_timing(fdtd_ctx *c, int capacity, int every)
 {
     if (!c || capacity < 0 || every < 1) return fdtd_fail(FDTD_EINVAL, "bad timing capacity or stride");

@@ -183,7 +183,7 @@ int fdtd_ctx_load(fdtd_ctx *ctx, const char *path);
  * the five launches of one step of the reference's loop (fdtd.cu:129-214,
  * updateHField ... updateMurBoundary, with the ring rotation of
  * fdtd.cu:115-530) as two launches, the fused H/D/source/E kernel and the
- * Mur faces with the step's probe row, or for a small grid as one. */
+ * Mur faces with the step's probe row, or as one (fdtd_ctx_by_cells). */
 int fdtd_step_fused(fdtd_ctx *ctx, hipStream_t stream);
 /* `steps` steps; enqueues only (no host synchronisation). */
 int fdtd_run(fdtd_ctx *ctx, int steps, hipStream_t stream);
@@ -227,9 +227,12 @@ int fdtd_slices_read(fdtd_ctx *ctx, int *steps, float *data, int max_slices);
 int fdtd_ctx_autotune(fdtd_ctx *ctx, int trial_steps, hipStream_t stream, int *tile_y, int *kchunk, int *lane_cells);
 
 /* The launch shape chosen for the context's fused kernel.  A context whose
- * state fits the Infinity Cache, and whose FdtdExt fixes no part of the shape,
- * steps with one lane per cell instead (same results) and does not use it. */
+ * FdtdExt fixes no part of the shape, and whose state is not too large (fp32:
+ * 1.2 GB, rows of whole waves 2.6 GB; 16 bits: 6 GB), steps with one lane per
+ * cell instead, one launch per step (same results), and does not use it:
+ * fdtd_ctx_by_cells returns 1. */
 int fdtd_ctx_launch_shape(fdtd_ctx *ctx, int *tile_x, int *tile_y, int *kchunk, int *blocks);
+int fdtd_ctx_by_cells(fdtd_ctx *ctx);
 /* The launch shape fdtd_ctx_create would take for this grid and extension
  * (no counterpart in the reference, whose launch geometry is fixed at
  * (ceil(nx/128), ny, nz) x 128 threads, fdtd.cu:129-490): 4 tile rows; for
