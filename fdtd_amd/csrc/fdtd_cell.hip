@@ -35,14 +35,14 @@
 //     for, so it waits for no other wave.
 //
 // Measured on MI355X, whole steps, against fused_step and the Mur launch
-// (us): fp32 24^3 5.7 (15.1), 64^3 7.4 (16.6), 100^3 20.5 (31.2), 128^3 28
-// (47), 160x160x100 34 (60), 151x138x188 75 (83), 256^3 280 (304); fp16 64^3
-// 6.9 (18.0), 96x121x77 13.4 (27.6), 256^3 181 (206), 320x320x300 318 (377).
-// 128^3 moves 178 MB, 6.4 TB/s at the L2's far side, where a stream of the same
+// (us): fp32 24^3 5.2 (15.1), 64^3 7.2 (16.6), 100^3 20.4 (31.2), 128^3 30
+// (47), 160x160x100 34 (60), 151x138x188 78 (83), 256^3 285 (304); fp16 64^3
+// 6.8 (18.0), 96x121x77 13.2 (27.6), 256^3 181 (206), 320x320x300 318 (377).
+// 128^3 moves 180 MB, 6.4 TB/s at the L2's far side, where a stream of the same
 // arrays reaches 8.0; with 4 waves a SIMD instead of 7 it takes as long.  Past
-// the cache fp32 waits for HBM (85 bytes a cell at 5.1 TB/s at 320x320x224;
-// occupancy again makes no difference); 16-bit fields have half the bytes in
-// flight a wave, and each wave less than 8 a SIMD shows.
+// the cache fp32 waits for HBM (85 bytes a cell at 5.0 TB/s at 320x320x224;
+// occupancy again makes no difference).  16-bit grids are held by the waves in
+// flight: 8 a SIMD, the most there are, take 186 us at 256^3, 6 take 225.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 

@@ -261,8 +261,8 @@ int fdtd_ctx_timed_steps(fdtd_ctx *ctx);
 
 /* Memory-ceiling calibration (no counterpart in the reference): streams the
  * fused step's access mix without its arithmetic, 15 arrays read and 9
- * written element for element (cells floats each, 64 Ki elements apart as
- * in a context, every access nontemporal), `reps` timed passes on `blocks`
+ * written element for element (cells floats each, 64 Ki elements
+ * apart, every access nontemporal), `reps` timed passes on `blocks`
  * blocks of 256 threads (0 = as many as fit resident).  Allocates and frees
  * 96 bytes per cell.  gbs receives 96 * cells bytes over the mean pass
  * time, ms_per_pass (optional) that time. */
