@@ -1,7 +1,8 @@
 // Batches of independent grids (fdtd_amd.h, fdtd_batch_*): one device arena
-// holds every grid's state.  Small grids are stepped in groups whose state
-// fits the Infinity Cache, one launch per group and step (cell_batch), many
-// steps of a group in a row.  The others take one persistent fused launch per
+// holds every grid's state.  Grids that a context would step by cells are
+// stepped in groups, the small ones several to a group whose state fits the
+// Infinity Cache, one launch per group and step (cell_batch), many steps of a
+// group in a row.  The others take one persistent fused launch per
 // storage form present, one Mur launch and one probe launch per step over all
 // of them.  The launches read the grids' descriptors, the per-form
 // tile lists and a step counter from device memory, so a sequence of steps
@@ -204,8 +205,8 @@ struct fdtd_batch {
     bool dirty = true;                 // device tables out of date
     std::vector<int> running;          // slots in the device tables
     int mask = 0;                      // kernel classes in the device tables
-    bool by_cell = true;               // small grids step by cell_batch, the others in tiles
-    struct Group { int first, count, blocks, storage; };
+    bool by_cell = true;               // grids that may (cell_grid) step by cell_batch, the others in tiles
+    struct Group { int first, count, blocks, form, storage; };
     std::vector<Group> groups;         // of the device tables
     int grid[kBatchClasses] = {};
     int tiles[kBatchClasses] = {};
@@ -240,19 +241,20 @@ bool is_running(const fdtd_batch *b, int s)
     return I.used && b->step - I.start < I.steps;
 }
 
-// Whether cell_batch steps the grid.
+// Whether cell_batch steps the grid: as a context's default_cell.
 bool cell_grid(const fdtd_batch *b, const fdtd_batch::Inst &I)
 {
-    return b->by_cell && I.d.nz <= kCellMaxPlanes && 24 * I.L.Np * I.L.esz <= cell_near_limit(I.L.esz);
+    return b->by_cell && I.d.nz <= kCellMaxPlanes && 24 * I.L.Np * I.L.esz <= cell_state_limit(I.d.nx, I.L.esz);
 }
 
-// Groups of the grids `cell` whose state fits kCellGroupBytes together (one
-// larger grid makes a group), storage by storage, largest first; fills the
-// group tables.
+// Groups of the grids `cell` whose state fits kCellGroupBytes together (a grid
+// past the near form makes a group), storage by storage, largest first; fills
+// the group tables.
 void make_groups(fdtd_batch *b, std::vector<int> cell, DevTables *T)
 {
     b->groups.clear();
     auto bytes = [&](int s) { return 24 * b->in[s].L.Np * b->in[s].L.esz; };
+    auto form = [&](int s) { return cell_form(bytes(s), b->in[s].L.esz); };
     std::sort(cell.begin(), cell.end(), [&](int p, int q) {
         const int sp = b->in[p].d.storage, sq = b->in[q].d.storage;
         if (sp != sq) return sp < sq;
@@ -265,10 +267,11 @@ void make_groups(fdtd_batch *b, std::vector<int> cell, DevTables *T)
         const int s = cell[t];
         if (t > 0 && b->in[s].d.storage != b->in[cell[t - 1]].d.storage) open = bins.size();
         size_t w = open;
+        if (form(s) != kCellNear) w = bins.size();
         while (w < bins.size() && room[w] < bytes(s)) w++;
         if (w == bins.size()) {
             bins.push_back({});
-            room.push_back(std::max(kCellGroupBytes, bytes(s)));
+            room.push_back(form(s) == kCellNear ? kCellGroupBytes : bytes(s));
         }
         bins[w].push_back(s);
         room[w] -= bytes(s);
@@ -282,7 +285,8 @@ void make_groups(fdtd_batch *b, std::vector<int> cell, DevTables *T)
             T->groups.start[at + 1] = T->groups.start[at] + cell_blocks(b->in[s].c);
             at++;
         }
-        b->groups.push_back({first, at - first, T->groups.start[at] - T->groups.start[first], b->in[bin[0]].d.storage});
+        b->groups.push_back({first, at - first, T->groups.start[at] - T->groups.start[first], form(bin[0]),
+                             b->in[bin[0]].d.storage});
     }
 }
 
@@ -622,7 +626,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.o0 = (uint32_t)gb;
     c.sy = (uint32_t)(L.pitch * L.esz);
     c.sz = (uint32_t)(L.plane * L.esz);
-    cell_tiles(nx, ny, kCellNear, L.esz, c);
+    cell_tiles(nx, ny, cell_form(24 * L.Np * L.esz, L.esz), L.esz, c);
     for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
     c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : 0;
     c.nprobe = d.nprobe;
@@ -681,7 +685,7 @@ extern "C" int fdtd_batch_run(fdtd_batch *b, int steps, hipStream_t stream)
         for (const auto &G : b->groups)
             for (int t = 0; t < g; t++)
                 HIP_TRY(launch_cell_batch(b->dev->cell, &b->dev->groups, G.first, G.count, G.blocks, (int)b->step + t,
-                                          G.storage, stream));
+                                          G.form, G.storage, stream));
         b->step += g;
         left -= g;
     }

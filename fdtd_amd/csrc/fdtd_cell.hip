@@ -230,7 +230,7 @@ struct BatchStep {
     __device__ __forceinline__ float cd(int q) const { return d->cd[q]; }
     __device__ __forceinline__ uint32_t zmask() const { return d->zmask; }
     __device__ __forceinline__ int hi_once() const { return d->hi_once; }
-    __device__ __forceinline__ int flip() const { return 0; }
+    __device__ __forceinline__ int flip() const { return n & 1; }
     __device__ __forceinline__ const char * e0(int q) const { return d->E[s0][q]; }
     __device__ __forceinline__ const char * e1(int q) const { return d->E[s1][q]; }
     __device__ __forceinline__ const char * d0(int q) const { return d->D[s0][q]; }
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
 // One step of a group of a batch's grids: blocks [start[q], start[q + 1]) of
 // the launch are grid q's, a multiple of 8, so that cell_block's mapping of
 // tiles to XCDs holds.  Grids outside their step window are skipped.
-template <typename T, bool EXACT>
+template <typename T, bool EXACT, int FORM>
 __global__ __launch_bounds__(kCellBlock) void cell_batch(const CellInst *inst, const CellGroups *groups, int first,
                                                          int count, int step)
 {
@@ -598,8 +598,13 @@ __global__ __launch_bounds__(kCellBlock) void cell_batch(const CellInst *inst, c
     const int local = b - S->start[lo], gx = 8 * d->run;
     const int bz = local / gx, bx = local - bz * gx;
     const BatchStep C{d, (n + 2) % 3, (n + 1) % 3, n % 3, n & 1, n};
-    if (d->bxl == 6) cell_block<T, EXACT, 6, kCellNear>(C, bx, bz);
-    else cell_block<T, EXACT, 5, kCellNear>(C, bx, bz);
+    if constexpr (sizeof(T) == 4 || FORM == kCellNear) {   // cell_lanes_log2
+        if (d->bxl == 5) {
+            cell_block<T, EXACT, 5, FORM>(C, bx, bz);
+            return;
+        }
+    }
+    cell_block<T, EXACT, 6, FORM>(C, bx, bz);
 }
 
 template <typename T, bool EXACT>
@@ -662,16 +667,29 @@ hipError_t launch_cell_step(const CellArgs &c, int storage, hipStream_t s, hipEv
     }
 }
 
-hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
-                             int storage, hipStream_t s)
+template <typename T, bool EXACT>
+static hipError_t launch_cell_batch_t(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks,
+                                      int step, int form, hipStream_t s)
 {
     const dim3 grid((unsigned)blocks), block(kCellBlock);
-    switch (storage) {
-    case kStoreF32: cell_batch<float, true><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
-    case kStoreF32Fast: cell_batch<float, false><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
-    case kStoreF16: cell_batch<__half, false><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
-    case kStoreBF16: cell_batch<__hip_bfloat16, false><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
-    default: return hipErrorInvalidValue;
+    constexpr int kPart = sizeof(T) == 2 ? kCellPart : kCellFar;   // 16 bits only
+    switch (form) {
+    case kCellNear: cell_batch<T, EXACT, kCellNear><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    case kCellMid: cell_batch<T, EXACT, kCellMid><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    case kCellPart: cell_batch<T, EXACT, kPart><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    default: cell_batch<T, EXACT, kCellFar><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
     }
     return hipGetLastError();
+}
+
+hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
+                             int form, int storage, hipStream_t s)
+{
+    switch (storage) {
+    case kStoreF32: return launch_cell_batch_t<float, true>(inst, groups, first, count, blocks, step, form, s);
+    case kStoreF32Fast: return launch_cell_batch_t<float, false>(inst, groups, first, count, blocks, step, form, s);
+    case kStoreF16: return launch_cell_batch_t<__half, false>(inst, groups, first, count, blocks, step, form, s);
+    case kStoreBF16: return launch_cell_batch_t<__hip_bfloat16, false>(inst, groups, first, count, blocks, step, form, s);
+    default: return hipErrorInvalidValue;
+    }
 }

@@ -233,10 +233,6 @@ inline int cell_form(size_t state, size_t esz)
     if (esz == 2) return state <= 400000000 ? kCellPart : state <= 1000000000 ? kCellMid : kCellFar;
     return state <= 360000000 ? kCellMid : kCellFar;
 }
-// Padded state up to which cell_batch steps a batch's grid, in the near form,
-// in us against tiles: fp32 285 MB 54 (69), 344 MB 79.5 (78.7); 16-bit 566 MB
-// 155 (153.5).
-inline size_t cell_near_limit(size_t esz) { return esz == 2 ? 640000000 : 320000000; }
 // log2 of the lanes of its tiles along x: 64, or 32.  Near: 32 where 64 leave
 // clearly more lanes idle (96 wide: 16.1 against 16.8 us in fp32, 13.0 against
 // 13.8 in fp16; 160 wide, where 32 lanes would fill 20 % more: 35.2 against
@@ -512,7 +508,7 @@ inline int cell_blocks(const CellInst &d)
     return gx * (d.nz + (pb + gx - 1) / gx);
 }
 hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
-                             int storage, hipStream_t s);
+                             int form, int storage, hipStream_t s);
 
 struct BatchLaunch {
     const BatchInst *inst;

@@ -292,10 +292,11 @@ int fdtd_load_phantom_ids(const char *dir, int nx, int ny, int nz, int mode, int
 /* ---- batches of independent grids --------------------------------------
  *
  * A batch holds many grids of different sizes, materials, sources, storage
- * forms and step counts in one device arena.  Small grids are stepped in
- * groups whose state fits the Infinity Cache, one launch per group and step;
- * a step of the others is one persistent fused kernel per storage form
- * present, one Mur launch and one probe launch, replayed from captured graphs;
+ * forms and step counts in one device arena.  Grids that a
+ * context would step by cells (fdtd_ctx_by_cells) are stepped in groups, the
+ * small ones several to a group whose state fits the Infinity Cache, one launch
+ * per group and step; a step of the others is one persistent fused kernel per
+ * storage form present, one Mur launch and one probe launch, replayed from captured graphs;
  * grids join (fdtd_batch_add) and leave (fdtd_batch_remove) between calls.
  * A grid's results are those of a single fdtd_ctx with the same inputs, bit
  * for bit (the per-cell arithmetic does not depend on the batch). */
@@ -361,8 +362,8 @@ int fdtd_batch_probe_peak_units(fdtd_batch *b, int id, double *peak, int nprobe)
 int fdtd_batch_get_field(fdtd_batch *b, int id, int field, int level, float *host);
 /* tile_y in {2,4,8}, kchunk >= 1, graph_steps >= 1 (0 keeps a value).  With a
  * tile_y or kchunk every grid is stepped in tiles of that shape; otherwise
- * grids whose state fits the Infinity Cache are stepped in groups that do, one
- * lane per cell (same results). */
+ * grids that a context would step by cells are stepped in groups (same
+ * results). */
 int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int graph_steps);
 /* Times every (tile_y in {2,4,8}, kchunk in {3,4,6,8,16}) candidate on the batch's own grids for
  * trial_steps steps each, and the groups of small grids, keeps the fastest (tile_y and kchunk: of the

@@ -152,3 +152,21 @@ def test_batch_groups_and_tiles(count, edge):
         b.run(45)
         for q, (i, x) in enumerate(zip(ids, insts)):
             assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("shape,storage", [((96, 130, 300), F.STORE_F32), ((64, 128, 420), F.STORE_F32), ((130, 127, 260), F.STORE_F32),
+                                           ((100, 121, 500), F.STORE_F16), ((100, 121, 900), F.STORE_BF16)])
+def test_batch_grids_past_the_cache(shape, storage):
+    """Grids that make a group of their own, in the forms past the cache, with
+    a small one that ends first and joins again."""
+    from tests.test_gpu_batch import assert_same, make_case, single
+    insts = [make_case(500, shape, 5, 9, storage), make_case(501, (30, 20, 25), 5, 4, storage)]
+    refs = [single(x) for x in insts]
+    with F.Batch(4 << 30) as b:
+        ids = [b.add(x) for x in insts]
+        b.run(5)
+        ids.append(b.add(insts[1]))
+        b.run(6)
+        for i, q in zip(ids, (0, 1, 1)):
+            assert_same(b, i, insts[q], refs[q], f"grid {q} {insts[q].shape}")
