@@ -206,7 +206,7 @@ struct fdtd_batch {
     std::vector<int> running;          // slots in the device tables
     int mask = 0;                      // kernel classes in the device tables
     bool by_cell = true;               // grids that may (cell_grid) step by cell_batch, the others in tiles
-    struct Group { int first, count, blocks, form, storage; };
+    struct Group { int first, count, blocks, form, lanes, storage; };
     std::vector<Group> groups;         // of the device tables
     int grid[kBatchClasses] = {};
     int tiles[kBatchClasses] = {};
@@ -285,7 +285,7 @@ void make_groups(fdtd_batch *b, std::vector<int> cell, DevTables *T)
             T->groups.start[at + 1] = T->groups.start[at] + cell_blocks(b->in[s].c);
             at++;
         }
-        b->groups.push_back({first, at - first, T->groups.start[at] - T->groups.start[first], form(bin[0]),
+        b->groups.push_back({first, at - first, T->groups.start[at] - T->groups.start[first], form(bin[0]), b->in[bin[0]].c.lanes,
                              b->in[bin[0]].d.storage});
     }
 }
@@ -685,7 +685,7 @@ extern "C" int fdtd_batch_run(fdtd_batch *b, int steps, hipStream_t stream)
         for (const auto &G : b->groups)
             for (int t = 0; t < g; t++)
                 HIP_TRY(launch_cell_batch(b->dev->cell, &b->dev->groups, G.first, G.count, G.blocks, (int)b->step + t,
-                                          G.form, G.storage, stream));
+                                          G.form, G.lanes, G.storage, stream));
         b->step += g;
         left -= g;
     }

@@ -54,7 +54,7 @@
 
 namespace {
 
-constexpr int kCellBlock = 256;
+constexpr int kCoefBlock = 256;
 
 // The Mur segment (numbered as in mur_segments) that writes E component c at
 // (i, j, k), and the step towards the cell whose lane evaluates it; -1: none.
@@ -276,8 +276,8 @@ struct Ops {
 };
 
 // One block's cells (or, past the planes, its probes) of a grid's step.
-// BXL: log2 of the lanes of a block along x (32 or 64); the other lanes are
-// rows.  Exact form: cells whose material has a = g3 = +0 (zmask) do not
+// BXL: log2 of the lanes of a block along x (32 or 64); the other lanes of its
+// cell_block_lanes are rows.  Exact form: cells whose material has a = g3 = +0 (zmask) do not
 // load E^{n-1} and D^{n-1}, as fused_tile's zero-term rows, decided per lane;
 // a grid that always loads them has zmask = 0.  C: where the step's operands
 // are (OneStep, BatchStep); block bx of the 8 * C.run() of plane bz.
@@ -286,7 +286,8 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
 {
     using X = Elem<T>;
     constexpr uint32_t ES = sizeof(T);
-    constexpr int BX = 1 << BXL, BY = kCellBlock / BX, WY = 64 / BX;
+    constexpr int LB = cell_block_lanes(FORM, sizeof(T), BXL);
+    constexpr int BX = 1 << BXL, BY = LB / BX, WY = 64 / BX;
     constexpr bool LANES = FORM != kCellNear, ND = FORM >= kCellPart, NE = FORM == kCellFar;
     const int nx = C.nx(), ny = C.ny(), nz = C.nz();
 
@@ -313,7 +314,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         deep = jw >= 2 && jw + WY <= ny - 2 && k >= 2 && k < nz - 2 && nx > 3;
         edge = tx == 0 || (nx - 2 >= tx * BX && nx - 2 < tx * BX + BX);
     } else {
-        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * 8 * C.run() + bx) * (kCellBlock / 64) +
+        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * 8 * C.run() + bx) * (LB / 64) +
                                                ((int)threadIdx.x >> 6));
         if (probe >= C.nprobe()) return;
         const int *q = C.probes() + 4 * probe;
@@ -562,7 +563,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
 }
 
 template <typename T, bool EXACT, int BXL, int FORM>
-__global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
+__global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), BXL)) void cell_step(const CellArgs C)
 {
     // What the lanes need of the arguments before their loads can go out, and
     // something of the other cache lines, in one go: left alone, each first use
@@ -581,7 +582,7 @@ __global__ __launch_bounds__(kCellBlock) void cell_step(const CellArgs C)
 // the launch are grid q's, a multiple of 8, so that cell_block's mapping of
 // tiles to XCDs holds.  Grids outside their step window are skipped.
 template <typename T, bool EXACT, int FORM>
-__global__ __launch_bounds__(kCellBlock) void cell_batch(const CellInst *inst, const CellGroups *groups, int first,
+__global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), 6)) void cell_batch(const CellInst *inst, const CellGroups *groups, int first,
                                                          int count, int step)
 {
     Const<CellGroups> *S = (Const<CellGroups> *)groups;
@@ -622,19 +623,19 @@ hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEve
         }
     }
     const unsigned gx = 8u * (unsigned)c.run;
-    const unsigned waves = kCellBlock / 64, pb = ((unsigned)c.p.nprobe + waves - 1) / waves;
+    const unsigned waves = (unsigned)c.lanes / 64, pb = ((unsigned)c.p.nprobe + waves - 1) / waves;
     const dim3 grid(gx, (unsigned)c.nz + (pb + gx - 1) / gx);
     CellArgs arg = c;
     void *args[] = {&arg};
-    return hipExtLaunchKernel(k, grid, dim3(kCellBlock), args, 0, s, t0, t1, 0);
+    return hipExtLaunchKernel(k, grid, dim3((unsigned)c.lanes), args, 0, s, t0, t1, 0);
 }
 
 // One coefficient per thread; blockIdx.y: the face.
-__global__ __launch_bounds__(kCellBlock) void mur_coefs(const MurCoefArgs a)
+__global__ __launch_bounds__(kCoefBlock) void mur_coefs(const MurCoefArgs a)
 {
     const int f = (int)blockIdx.y, axis = f >> 1, end = f & 1;
     const long long n = axis == 0 ? (long long)a.ny * a.nz : axis == 1 ? (long long)a.nx * a.nz : (long long)a.nx * a.ny;
-    const long long q = (long long)blockIdx.x * kCellBlock + threadIdx.x;
+    const long long q = (long long)blockIdx.x * kCoefBlock + threadIdx.x;
     if (q >= n) return;
     // the two cells of the pair in the reference's plane: x (k, j, 2), y (k, 2, i), z (2, j, i)
     const long long k = q / a.nx, at = axis == 0 ? 2 * q : axis == 1 ? 2 * k * a.nx + (q - k * a.nx) : q;
@@ -652,7 +653,7 @@ __global__ __launch_bounds__(kCellBlock) void mur_coefs(const MurCoefArgs a)
 hipError_t launch_mur_coefs(const MurCoefArgs &a, int faces, hipStream_t s)
 {
     const long long m = std::max({(long long)a.ny * a.nz, (long long)a.nx * a.nz, (long long)a.nx * a.ny});
-    mur_coefs<<<dim3((unsigned)((m + kCellBlock - 1) / kCellBlock), (unsigned)faces), kCellBlock, 0, s>>>(a);
+    mur_coefs<<<dim3((unsigned)((m + kCoefBlock - 1) / kCoefBlock), (unsigned)faces), kCoefBlock, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -669,9 +670,9 @@ hipError_t launch_cell_step(const CellArgs &c, int storage, hipStream_t s, hipEv
 
 template <typename T, bool EXACT>
 static hipError_t launch_cell_batch_t(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks,
-                                      int step, int form, hipStream_t s)
+                                      int step, int form, int lanes, hipStream_t s)
 {
-    const dim3 grid((unsigned)blocks), block(kCellBlock);
+    const dim3 grid((unsigned)blocks), block((unsigned)lanes);
     constexpr int kPart = sizeof(T) == 2 ? kCellPart : kCellFar;   // 16 bits only
     switch (form) {
     case kCellNear: cell_batch<T, EXACT, kCellNear><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
@@ -683,13 +684,13 @@ static hipError_t launch_cell_batch_t(const CellInst *inst, const CellGroups *gr
 }
 
 hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
-                             int form, int storage, hipStream_t s)
+                             int form, int lanes, int storage, hipStream_t s)
 {
     switch (storage) {
-    case kStoreF32: return launch_cell_batch_t<float, true>(inst, groups, first, count, blocks, step, form, s);
-    case kStoreF32Fast: return launch_cell_batch_t<float, false>(inst, groups, first, count, blocks, step, form, s);
-    case kStoreF16: return launch_cell_batch_t<__half, false>(inst, groups, first, count, blocks, step, form, s);
-    case kStoreBF16: return launch_cell_batch_t<__hip_bfloat16, false>(inst, groups, first, count, blocks, step, form, s);
+    case kStoreF32: return launch_cell_batch_t<float, true>(inst, groups, first, count, blocks, step, form, lanes, s);
+    case kStoreF32Fast: return launch_cell_batch_t<float, false>(inst, groups, first, count, blocks, step, form, lanes, s);
+    case kStoreF16: return launch_cell_batch_t<__half, false>(inst, groups, first, count, blocks, step, form, lanes, s);
+    case kStoreBF16: return launch_cell_batch_t<__hip_bfloat16, false>(inst, groups, first, count, blocks, step, form, lanes, s);
     default: return hipErrorInvalidValue;
     }
 }

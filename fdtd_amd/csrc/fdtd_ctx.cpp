@@ -176,6 +176,9 @@ bool default_cell(const fdtd_ctx *c)
     return c->nz <= kCellMaxPlanes && 24 * c->Np * c->esz <= cell_state_limit(c->nx, c->esz);
 }
 
+// Whether its next step is cell_step's.
+bool by_cells(const fdtd_ctx *c) { return c->cell && c->nprobe <= kCellMaxProbes; }
+
 // Launch shape a context takes for a grid, from launch-shape sweeps on
 // MI355X: 4 tile rows (8 rows gain 1-5% at 256^3 and lose at 320x320x880 and
 // on small grids), identity block order; two cells per lane for 16-bit
@@ -767,7 +770,7 @@ extern "C" int fdtd_step_fused(fdtd_ctx *c, hipStream_t stream)
     fill_step_args(c, n, a);
     const bool timed = timed_launch(c, 1);
     hipEvent_t t0 = timed ? c->tev[2 * c->tused] : nullptr, t1 = timed ? c->tev[2 * c->tused + 1] : nullptr;
-    if (c->cell) {
+    if (by_cells(c)) {
         c->n = n + 1;
         c->hcur ^= 1;
         CellArgs q;
@@ -886,7 +889,7 @@ extern "C" int fdtd_ctx_launch_shape(fdtd_ctx *c, int *tile_x, int *tile_y, int 
     return 0;
 }
 
-extern "C" int fdtd_ctx_by_cells(fdtd_ctx *c) { return c ? (c->cell ? 1 : 0) : FDTD_EINVAL; }
+extern "C" int fdtd_ctx_by_cells(fdtd_ctx *c) { return c ? (by_cells(c) ? 1 : 0) : FDTD_EINVAL; }
 
 extern "C" int fdtd_ctx_set_timing(fdtd_ctx *c, int capacity, int every)
 {

@@ -197,7 +197,7 @@ struct CellArgs {
     uint32_t tx_mul;               // ceil(2^32 / tiles_x)
     float ch[3], cd[3], jz;
     uint32_t zmask;                // bit m: material m < 32 has a = g3 = +0 and its cells do not load levels n-1
-    int bxl;                       // 5 or 6: 32 or 64 lanes of a 256-lane tile along x
+    int bxl, lanes;                // 5 or 6: 32 or 64 lanes of a tile along x; lanes of a tile and block
     int hi_once;                   // the tiled step leaves the x-high faces to the Mur kernel (fused_mur_x 2)
     int form;                      // kCellNear, ...
     int flip;                      // planes from the highest down: every other step, so that a step starts where
@@ -213,7 +213,8 @@ struct CellArgs {
 // 2.2 GB 387 (396), 3.1 GB 570 (565), 4.0 GB 725 (704); others 1.1 GB 203
 // (208), 300^3 504 (491), 350x330x200 421 (414).  16 bits: 1.5 GB 340
 // (383), 3.9 GB 844 (981), 4.3 GB 991 (1051), 6.4 GB 1555 (1544).
-constexpr int kCellMaxPlanes = 60000;   // planes and probe rows are blockIdx.y
+constexpr int kCellMaxPlanes = 60000;   // planes and, in rows of at least 8 blocks, probes are blockIdx.y
+constexpr int kCellMaxProbes = 40000;
 inline size_t cell_state_limit(int nx, size_t esz)
 {
     return esz == 2 ? 6000000000 : nx % 64 == 0 ? 2600000000 : 1200000000;
@@ -246,13 +247,24 @@ inline int cell_lanes_log2(int nx, int form, size_t esz)
     const double e6 = (double)nx / (64 * ((nx + 63) / 64)), e5 = (double)nx / (32 * ((nx + 31) / 32));
     return e6 < 0.8 * e5 ? 5 : 6;
 }
+// Lanes of a block: one wave, or four where fp32 streams past the cache in
+// 64-lane tiles and the rows of a block share their halo rows' lines (us, 64
+// against 256: 256^3 298, 289; 192^3 126, 122).  Elsewhere a block of one wave
+// leaves and makes room at once: 32^3 4.8, 5.4; 100^3 18.9, 20.5; 151x138x188
+// 74.6, 78.7; fp16 96x121x77 13.1, 13.4, 320x320x300 320, 323; twelve batched
+// grids 28.2, 29.7 ms (128 lanes in between).
+constexpr int cell_block_lanes(int form, size_t esz, int bxl)
+{
+    return form == kCellFar && esz == 4 && bxl == 6 ? 256 : 64;
+}
 // The tile geometry of a grid (CellArgs, CellInst) and the materials whose
 // cells skip levels n-1.
 template <typename A>
 inline void cell_tiles(int nx, int ny, int form, size_t esz, A &a)
 {
     a.bxl = cell_lanes_log2(nx, form, esz);
-    const int bx = 1 << a.bxl, by = 256 / bx;
+    a.lanes = cell_block_lanes(form, esz, a.bxl);
+    const int bx = 1 << a.bxl, by = a.lanes / bx;
     a.tiles_x = (nx + bx - 1) / bx;
     a.tx_mul = (uint32_t)(((1ull << 32) + a.tiles_x - 1) / a.tiles_x);
     a.tiles = a.tiles_x * ((ny + by - 1) / by);
@@ -491,7 +503,7 @@ struct CellInst {
     uint32_t tx_mul;
     float ch[3], cd[3];
     uint32_t zmask;
-    int hi_once, bxl;
+    int hi_once, bxl, lanes;
     int nprobe, probe_rows, jz_len, jz_hold3, start, nsteps;
     float dt, h[3], mu0, eps0;
 };
@@ -501,14 +513,14 @@ struct CellGroups {
     int idx[kBatchMaxInst];
     int start[kBatchMaxInst + 1];
 };
-// Blocks of a grid's step: its planes' and its probes' (four a block).
+// Blocks of a grid's step: its planes' and its probes' (one a wave).
 inline int cell_blocks(const CellInst &d)
 {
-    const int gx = 8 * d.run, pb = (d.nprobe + 3) / 4;
+    const int gx = 8 * d.run, w = d.lanes / 64, pb = (d.nprobe + w - 1) / w;
     return gx * (d.nz + (pb + gx - 1) / gx);
 }
 hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,
-                             int form, int storage, hipStream_t s);
+                             int form, int lanes, int storage, hipStream_t s);
 
 struct BatchLaunch {
     const BatchInst *inst;

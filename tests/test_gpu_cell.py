@@ -170,3 +170,19 @@ def test_batch_grids_past_the_cache(shape, storage):
         b.run(6)
         for i, q in zip(ids, (0, 1, 1)):
             assert_same(b, i, insts[q], refs[q], f"grid {q} {insts[q].shape}")
+
+
+def test_more_probes_than_blocks_take_tiles():
+    """A context with more probes than the launch has room for steps in tiles;
+    up to there by cells, with the same series."""
+    shape, out = (20, 18, 16), {}
+    for n in (40000, 40001):
+        probes = np.tile(_probes(shape), (n // 108 + 1, 1))[:n]
+        with F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0)) as ctx:
+            ctx.set_sources(np.asarray([(9, 8, 7)], np.int32), np.linspace(1.0, 2.0, 9).astype(np.float32))
+            ctx.set_probes(probes, 9)
+            assert ctx.by_cells() == (n == 40000)
+            ctx.run(9)
+            out[n] = ctx.probes()[:, :108]
+            assert np.array_equal(ctx.probes()[:, 108:216], out[n])
+    assert np.array_equal(out[40000], out[40001]) and np.abs(out[40000]).max() > 0
