@@ -40,10 +40,11 @@ struct DevTables {
 // Padded state of the grids that cell_batch steps together, and the steps it
 // takes with one group before it goes on to the next: a group's state stays
 // in the Infinity Cache (256 MB) meanwhile.  Twelve fp32 grids around 96^3
-// (1.1 GB) on MI355X, in Gcell-updates/s: 53.0 as set; 51.6 with groups of
-// 210 MB, 53.1 with 250, 43 with 300, 39 with 400; 45.6 with 8 steps at a time,
-// 52.0 with 32, 53.5 with 128 (a grid that ends keeps its place in the launches
-// of those steps); 38.8 where fused_batch steps all of them together.
+// (1.1 GB) on MI355X, in Gcell-updates/s: 55.9 as set, 53.0 with blocks of four
+// waves; with these 51.6 in groups of 210 MB, 53.1 of 250, 43 of 300, 39 of 400;
+// 45.6 with 8 steps at a time, 52.0 with 32, 53.5 with 128 (a grid that ends
+// keeps its place in the launches of those steps); 38.8 where fused_batch steps
+// all of them together.
 constexpr size_t kCellGroupBytes = 240000000;
 constexpr int kCellRunSteps = 64;
 

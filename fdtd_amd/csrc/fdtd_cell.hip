@@ -35,9 +35,9 @@
 //     for, so it waits for no other wave.
 //
 // Measured on MI355X, whole steps, against fused_step and the Mur launch
-// (us): fp32 24^3 5.2 (15.1), 64^3 7.2 (16.6), 100^3 20.4 (31.2), 128^3 30
-// (47), 160x160x100 34 (60), 151x138x188 78 (83), 256^3 285 (304); fp16 64^3
-// 6.8 (18.0), 96x121x77 13.2 (27.6), 256^3 181 (206), 320x320x300 318 (377).
+// (us): fp32 32^3 4.8 (14.7), 64^3 7.2 (16.6), 100^3 18.9 (31.2), 128^3 30
+// (47), 160x160x100 34 (60), 151x138x188 75 (83), 256^3 285 (304); fp16 64^3
+// 6.8 (18.0), 96x121x77 13.0 (27.6), 256^3 181 (206), 320x320x300 318 (377).
 // 128^3 moves 180 MB, 6.4 TB/s at the L2's far side, where a stream of the same
 // arrays reaches 8.0; with 4 waves a SIMD instead of 7 it takes as long.  Past
 // the cache fp32 waits for HBM (85 bytes a cell at 5.0 TB/s at 320x320x224;

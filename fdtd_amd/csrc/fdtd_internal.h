@@ -210,14 +210,17 @@ struct CellArgs {
 // the tiled one keeps more of it in flight; what cell_step gains there is the
 // part of the state that the last step left in the cache, less where waves at
 // the rows' ends are part empty.  fp32, us against tiles: rows of whole waves
-// 2.2 GB 387 (396), 3.1 GB 570 (565), 4.0 GB 725 (704); others 1.1 GB 203
-// (208), 300^3 504 (491), 350x330x200 421 (414).  16 bits: 1.5 GB 340
-// (383), 3.9 GB 844 (981), 4.3 GB 991 (1051), 6.4 GB 1555 (1544).
+// 2.2 GB 387 (396), 3.1 GB 570 (565), 4.0 GB 725 (704); an odd number of half
+// waves (cell_lanes_log2) 340x300x170 318 (323), 160x400x300 352 (359), 2.1 GB
+// 392 (393), 2.2 GB 417 (414); others 1.1 GB 205 (206), 300x250x220 306 (307),
+// 300^3 504 (491).  16 bits: 1.5 GB 340 (383), 3.9 GB 844 (981), 4.3 GB 991
+// (1051), 6.4 GB 1555 (1544).
 constexpr int kCellMaxPlanes = 60000;   // planes and, in rows of at least 8 blocks, probes are blockIdx.y
 constexpr int kCellMaxProbes = 40000;
 inline size_t cell_state_limit(int nx, size_t esz)
 {
-    return esz == 2 ? 6000000000 : nx % 64 == 0 ? 2600000000 : 1200000000;
+    if (esz == 2) return 6000000000;
+    return nx % 64 == 0 ? 2600000000 : (nx + 31) / 32 % 2 ? 2000000000 : 1200000000;
 }
 // Its form, in us (near, mid, part, far; means over six placements of the
 // state, which differ by up to 15 %).  fp32: 201 MB 30.2, 30.4, 38, 38; 246 MB
