@@ -22,9 +22,10 @@ namespace {
 
 // Extra elements between consecutive field arrays in the blob: staggers the
 // arrays' starts across HBM channels, also where a plane is a power of two
-// (256^3 fp32, us a step: 327 with 0, 1024 or 65536, 280 to 285 with 64, 4160
-// or this; 320x320x880 in tiles 1553 with 65536, 1529).
-constexpr size_t kArraySkew = 1088;
+// (256^3 fp32 by cells, us a step: 327 with 0, 1024 or 65536, 280 to 285 with
+// 64, 4160 or 1088; 320x320x880 in tiles 1553 with 65536, 1534 with 1088 or
+// 66624; 300x250x220 in tiles 307 with 1088, 298 with 66624).
+constexpr size_t kCellSkew = 1088, kTileSkew = 66624;
 
 }  // namespace
 
@@ -42,6 +43,7 @@ struct fdtd_ctx {
     int cpl = 1;                         // cells per lane of the fused kernel
     int txw = 64;                        // threads per tile row (one cell per lane)
     bool cell = false;                   // steps run as cell_step, not in tiles
+    size_t skew = 0;                     // elements between the field arrays
     bool fields_set = false;             // set_field or load gave non-zero state
 
     long long guard = 0;                 // elements before/after the field arrays and the ids
@@ -290,11 +292,12 @@ extern "C" int fdtd_ctx_create(const FdtdParams *p, const FdtdExt *ext, fdtd_ctx
 
     const size_t nf = 24;  // 9 E + 9 D + 6 H
     c->guard = fused_guard(c->pitch, c->plane);
-    const size_t blob_elems = nf * (c->Np + kArraySkew) + 2 * (size_t)c->guard;
+    c->skew = c->cell ? kCellSkew : kTileSkew;
+    const size_t blob_elems = nf * (c->Np + c->skew) + 2 * (size_t)c->guard;
     hipError_t he = hipMalloc(&c->blob, blob_elems * c->esz);
     if (he != hipSuccess) { delete c; return fdtd_hip_fail(he, "hipMalloc(fields)"); }
     char *q = c->blob + c->guard * c->esz;
-    const size_t stride = (c->Np + kArraySkew) * c->esz;
+    const size_t stride = (c->Np + c->skew) * c->esz;
     for (int s = 0; s < 3; s++)
         for (int k = 0; k < 3; k++) { c->E[s][k] = q; q += stride; }
     for (int s = 0; s < 3; s++)
@@ -686,7 +689,7 @@ bool two_step_ok(const fdtd_ctx *c)
 int alloc_spare(fdtd_ctx *c)
 {
     if (c->spare_blob) return 0;
-    const size_t stride = (c->Np + kArraySkew) * c->esz;
+    const size_t stride = (c->Np + c->skew) * c->esz;
     const size_t bytes = 6 * stride + 2 * (size_t)c->guard * c->esz;
     HIP_TRY(hipMalloc(&c->spare_blob, bytes));
     HIP_TRY(hipMemset(c->spare_blob, 0, bytes));
@@ -1199,9 +1202,9 @@ extern "C" int fdtd_ctx_autotune(fdtd_ctx *c, int trial_steps, hipStream_t strea
     if (t1) (void)hipEventDestroy(t1);
     // back to the zero state at step 0
     e = hipStreamSynchronize(stream);
-    if (e == hipSuccess) e = hipMemset(c->blob, 0, (24 * (c->Np + kArraySkew) + 2 * (size_t)c->guard) * c->esz);
+    if (e == hipSuccess) e = hipMemset(c->blob, 0, (24 * (c->Np + c->skew) + 2 * (size_t)c->guard) * c->esz);
     if (e == hipSuccess && c->spare_blob)
-        e = hipMemset(c->spare_blob, 0, (6 * (c->Np + kArraySkew) + 2 * (size_t)c->guard) * c->esz);
+        e = hipMemset(c->spare_blob, 0, (6 * (c->Np + c->skew) + 2 * (size_t)c->guard) * c->esz);
     if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune reset");
     c->n = 0;
     c->hcur = 0;
