@@ -42,15 +42,8 @@ bool h_params_set = false;
 constexpr int kBlock = 256;
 
 // A cell number (Q: uint32_t, or size_t for grids of 2^32 cells and more) is
-// divided by nx and nx*ny with a multiply each (exact for every 32-bit number:
-// m = floor(2^32 (2^s - d) / d) + 1, s = ceil(log2 d)); two 64-bit divisions
+// divided by nx and nx*ny with a multiply each (div_by); two 64-bit divisions
 // cost more instructions than the whole H update.
-__device__ __forceinline__ uint32_t div_by(uint32_t q, uint32_t mul, uint32_t shift)
-{
-    const uint32_t t = __umulhi(mul, q);
-    return (t + ((q - t) >> 1)) >> shift;
-}
-
 template <typename Q>
 __device__ __forceinline__ int row_of(const LegacyParams &p, Q q)   // q / nx
 {
@@ -255,14 +248,8 @@ extern "C" int copySymbolsToDevice(FdtdParams *params)
     h_p.mu0 = params->mu0; h_p.eps0 = params->eps0;
     h_p.chx = h_p.dt / (h_p.mu0 * h_p.dx); h_p.chy = h_p.dt / (h_p.mu0 * h_p.dy); h_p.chz = h_p.dt / (h_p.mu0 * h_p.dz);
     h_p.cdx = h_p.dt / h_p.dx; h_p.cdy = h_p.dt / h_p.dy; h_p.cdz = h_p.dt / h_p.dz;
-    auto divisor = [](unsigned long long d, uint32_t &mul, uint32_t &shift) {   // 2 <= d < 2^32 (div_by)
-        uint32_t s = 0;
-        while ((1ull << s) < d) s++;
-        mul = (uint32_t)((((1ull << s) - d) << 32) / d + 1);
-        shift = s - 1;
-    };
-    divisor(h_p.nx, h_p.nx_mul, h_p.nx_shift);
-    if (!wide()) divisor((unsigned long long)h_p.nx * h_p.ny, h_p.nxy_mul, h_p.nxy_shift);
+    div_consts(h_p.nx, h_p.nx_mul, h_p.nx_shift);
+    if (!wide()) div_consts((unsigned long long)h_p.nx * h_p.ny, h_p.nxy_mul, h_p.nxy_shift);
     const int ns = std::max(0, std::min(D_MAX_SOURCES, params->sourcesCount));
     const int nj = std::max(0, std::min(D_MAX_JZ, params->jzCount));
     for (int s = 0; s < ns; s++)

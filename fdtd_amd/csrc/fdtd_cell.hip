@@ -176,6 +176,7 @@ struct OneStep {
     __device__ __forceinline__ int tiles() const { return a.tiles; }
     __device__ __forceinline__ int run() const { return a.run; }
     __device__ __forceinline__ uint32_t tx_mul() const { return a.tx_mul; }
+    __device__ __forceinline__ uint32_t tx_shift() const { return a.tx_shift; }
     __device__ __forceinline__ const uint8_t * ids() const { return a.ids; }
     __device__ __forceinline__ const MatCoef * lut() const { return a.lut; }
     __device__ __forceinline__ float ch(int q) const { return a.ch[q]; }
@@ -224,6 +225,7 @@ struct BatchStep {
     __device__ __forceinline__ int tiles() const { return d->tiles; }
     __device__ __forceinline__ int run() const { return d->run; }
     __device__ __forceinline__ uint32_t tx_mul() const { return d->tx_mul; }
+    __device__ __forceinline__ uint32_t tx_shift() const { return d->tx_shift; }
     __device__ __forceinline__ const uint8_t * ids() const { return d->ids; }
     __device__ __forceinline__ const MatCoef * lut() const { return d->lut; }
     __device__ __forceinline__ float ch(int q) const { return d->ch[q]; }
@@ -302,7 +304,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     if (bz < nz) {
         const int t = (bx & 7) * C.run() + (bx >> 3);
         if (t >= C.tiles()) return;
-        const int ty = C.tiles_x() == 1 ? t : (int)__umulhi((unsigned)t, C.tx_mul()), tx = t - ty * C.tiles_x();
+        const int ty = cell_tile_row(t, C.tiles_x(), C.tx_mul(), C.tx_shift()), tx = t - ty * C.tiles_x();
         const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = (int)threadIdx.x & 63;
         jw = ty * BY + w * WY;
         if (jw >= ny) return;

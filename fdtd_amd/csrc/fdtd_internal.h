@@ -10,6 +10,22 @@
 
 #include "fdtd_amd.h"
 
+// q / d for every 32-bit q by a multiply (Granlund and Montgomery, Division by
+// invariant integers using multiplication, 1994): with s = ceil(log2 d) and
+// mul = floor(2^32 (2^s - d) / d) + 1.  div_consts: 2 <= d < 2^32.
+inline void div_consts(unsigned long long d, uint32_t &mul, uint32_t &shift)
+{
+    uint32_t s = 0;
+    while ((1ull << s) < d) s++;
+    mul = (uint32_t)((((1ull << s) - d) << 32) / d + 1);
+    shift = s - 1;
+}
+__host__ __device__ inline uint32_t div_by(uint32_t q, uint32_t mul, uint32_t shift)
+{
+    const uint32_t t = (uint32_t)(((uint64_t)mul * q) >> 32);
+    return (t + ((q - t) >> 1)) >> shift;
+}
+
 // Per-material Debye coefficients in the precision the reference evaluates
 // them (fdtd_calculations.cu:141-155): a, c, d are double expressions rounded
 // to float; the three D weights are double.  With these, an E update
@@ -194,7 +210,7 @@ struct CellArgs {
     int nx, ny, nz;
     uint32_t o0, sy, sz;           // bytes: guard, row, plane
     int tiles_x, tiles, run;       // tiles per row and per plane, ceil(tiles / 8)
-    uint32_t tx_mul;               // ceil(2^32 / tiles_x)
+    uint32_t tx_mul, tx_shift;     // div_consts(tiles_x)
     float ch[3], cd[3], jz;
     uint32_t zmask;                // bit m: material m < 32 has a = g3 = +0 and its cells do not load levels n-1
     int bxl, lanes;                // 5 or 6: 32 or 64 lanes of a tile along x; lanes of a tile and block
@@ -269,9 +285,15 @@ inline void cell_tiles(int nx, int ny, int form, size_t esz, A &a)
     a.lanes = cell_block_lanes(form, esz, a.bxl);
     const int bx = 1 << a.bxl, by = a.lanes / bx;
     a.tiles_x = (nx + bx - 1) / bx;
-    a.tx_mul = (uint32_t)(((1ull << 32) + a.tiles_x - 1) / a.tiles_x);
+    if (a.tiles_x > 1) div_consts(a.tiles_x, a.tx_mul, a.tx_shift);
+    else a.tx_mul = a.tx_shift = 0;
     a.tiles = a.tiles_x * ((ny + by - 1) / by);
     a.run = (a.tiles + 7) / 8;
+}
+// The row of tiles that tile t of a plane lies in.
+__host__ __device__ inline int cell_tile_row(int t, int tiles_x, uint32_t tx_mul, uint32_t tx_shift)
+{
+    return tiles_x == 1 ? t : (int)div_by((uint32_t)t, tx_mul, tx_shift);
 }
 inline uint32_t cell_zmask(const MatCoef *lut, int nmat)
 {
@@ -352,7 +374,7 @@ struct SnapArgs {
     float *out;
     int nx, ny, nz, pitch;
     long long plane;
-    uint32_t nx_mul, nx_shift;     // t / nx = (m + ((t - m) >> 1)) >> nx_shift, m = hi32(nx_mul * t); set at launch
+    uint32_t nx_mul, nx_shift;     // div_consts(nx), set at launch
 };
 hipError_t launch_snapshot(const SnapArgs &a, int storage, hipStream_t s);
 // Mur faces and one probe row in one launch (p.nprobe = 0: faces only).  The
@@ -503,7 +525,7 @@ struct CellInst {
     int nx, ny, nz;
     uint32_t o0, sy, sz;
     int tiles_x, tiles, run;
-    uint32_t tx_mul;
+    uint32_t tx_mul, tx_shift;
     float ch[3], cd[3];
     uint32_t zmask;
     int hi_once, bxl, lanes;

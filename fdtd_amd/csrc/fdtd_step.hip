@@ -1665,8 +1665,7 @@ __global__ __launch_bounds__(256) void plane_copy(const PlaneCopy P)
 // Unpitches (and for scaled storage, unscales) the nine fields of a context
 // into packed fp32 volumes: lanes run along the packed cells, blockIdx.y is
 // the field.  A block moves kSnapRun cells a lane, all loads before the first
-// store.  A cell's row is its number divided by nx, by a multiply (exact for
-// 32-bit numbers, see SnapArgs); the 64-bit division it replaces held the
+// store.  A cell's row is its number divided by nx, by a multiply (div_by); the 64-bit division it replaces held the
 // kernel to 4.1 TB/s.  The copy is streamed out past the cache: the next step
 // reads the fields, not it.
 constexpr int kSnapRun = 4;
@@ -1686,7 +1685,7 @@ __global__ __launch_bounds__(256) void field_snapshot(const SnapArgs A)
 #pragma unroll
     for (int u = 0; u < kSnapRun; u++) {
         const uint32_t t = min(t0 + u * 256u, n - 1);
-        const uint32_t m = __umulhi(A.nx_mul, t), row = (m + ((t - m) >> 1)) >> A.nx_shift;
+        const uint32_t row = div_by(t, A.nx_mul, A.nx_shift);
         const uint32_t at = t + row * gap;   // row = k*ny + j, and plane = pitch*ny
         if constexpr (std::is_same<T, float>::value) v[u] = src[at];
         else v[u] = Elem<T>::cvt(((const unsigned short *)src)[at]);
@@ -1705,10 +1704,7 @@ hipError_t launch_snapshot(const SnapArgs &a, int storage, hipStream_t s)
     const long long n = (long long)a.nx * a.ny * a.nz;
     if (n <= 0 || n >= (1LL << 32) || a.nx < 2 || !a.out) return hipErrorInvalidValue;
     SnapArgs b = a;
-    uint32_t sh = 0;
-    while ((1ull << sh) < (unsigned long long)a.nx) sh++;
-    b.nx_mul = (uint32_t)((((1ull << sh) - a.nx) << 32) / a.nx + 1);
-    b.nx_shift = sh - 1;
+    div_consts(a.nx, b.nx_mul, b.nx_shift);
     const dim3 grid((unsigned)((n + 256 * kSnapRun - 1) / (256 * kSnapRun)), 9);
     switch (storage) {
     case kStoreF32: field_snapshot<float, false><<<grid, 256, 0, s>>>(b); break;

@@ -1,0 +1,59 @@
+"""Index arithmetic of the one-lane-per-cell step, on the CPU: the header that
+the kernels share is compiled for the host and every tile of a plane mapped
+to its row and column, for rows of one tile up to millions of cells."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "fdtd_internal.h"
+struct Tiles { int bxl, lanes, tiles_x, tiles, run; uint32_t tx_mul, tx_shift; };
+int main(int argc, char **argv)
+{
+    for (int q = 1; q + 3 < argc; q += 4) {   // nx ny form esz
+        Tiles a;
+        const int nx = atoi(argv[q]), ny = atoi(argv[q + 1]);
+        cell_tiles(nx, ny, atoi(argv[q + 2]), (size_t)atoi(argv[q + 3]), a);
+        long long bad = 0;
+        for (int t = 0; t < a.tiles; t++) bad += cell_tile_row(t, a.tiles_x, a.tx_mul, a.tx_shift) != t / a.tiles_x;
+        printf("%d %d %lld\n", a.tiles_x, a.tiles, bad);
+    }
+    for (unsigned long long d : {2ull, 3ull, 5ull, 7ull, 64ull, 65ull, 641ull, 65535ull, 65537ull, 1ull << 31, (1ull << 31) + 1,
+                                 (1ull << 32) - 1}) {
+        uint32_t m, s;
+        div_consts(d, m, s);
+        for (unsigned long long k = 0; k < 4000; k++)
+            for (int e = -1; e <= 1; e++) {   // around multiples of d over the whole range
+                const uint32_t v = (uint32_t)((0xffffffffull / 3999 * k) / d * d + e);
+                if (div_by(v, m, s) != v / d) { printf("%u / %llu\n", v, d); return 1; }
+            }
+    }
+    return 0;
+}
+"""
+
+# rows of one tile, of a few, and so long that a rounded reciprocal's error adds up to a tile
+SHAPES = [(3, 3), (64, 5), (65, 130), (96, 37), (150, 150), (1024, 1024), (85016, 2495), (106023, 1995), (550190, 65),
+          (950358, 33), (1900757, 3)]
+
+
+@pytest.mark.parametrize("esz", [4, 2])
+def test_tiles_map_to_rows(tmp_path, esz):
+    src, exe = tmp_path / "tiles.cpp", tmp_path / "tiles"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{ROOT}/include",
+                    f"-I{ROOT}/fdtd_amd/csrc", str(src), "-o", str(exe)], check=True)
+    cases = [(nx, ny, form) for nx, ny in SHAPES for form in (0, 1, 3)]
+    args = [str(v) for nx, ny, form in cases for v in (nx, ny, form, esz)]
+    out = subprocess.run([str(exe), *args], capture_output=True, text=True, check=True).stdout.split()
+    got = np.asarray([int(v) for v in out]).reshape(-1, 3)
+    assert len(got) == len(cases)
+    for (nx, ny, form), (tiles_x, tiles, bad) in zip(cases, got):
+        assert tiles_x * 64 >= nx and tiles >= tiles_x * ((ny + 7) // 8)
+        assert bad == 0, f"{nx}x{ny} form {form}: {bad} of {tiles} tiles in a wrong row"

@@ -1,0 +1,41 @@
+"""Which kernel steps a grid, and the two kernels against each other where the
+choice or its index arithmetic is at a limit."""
+import numpy as np
+import pytest
+import torch
+
+import fdtd_amd as F
+
+pytestmark = pytest.mark.gpu
+
+DT, DX = 3.8105118e-12, 2.0e-3
+MU0, EPS0 = 1.2566371e-06, 8.841941e-12
+
+
+def _long_row(shape, tiled):
+    """Steps a grid of few, very long rows from random fields; its nine fields."""
+    nx, ny, nz = shape
+    rng = np.random.default_rng(list(shape))
+    with F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0), tile_y=4 if tiled else 0) as ctx:
+        assert ctx.by_cells() == (not tiled)
+        table = np.asarray([(0.0, 1.0, 1.0, 0.0), (0.8, 55.0, 40.0, 8e-12)], np.float32)
+        ctx.set_materials(rng.integers(0, 2, (nz, ny, nx), np.uint8), table)
+        ctx.set_sources(np.asarray([(nx - 1, 1, 1), (nx // 2, ny - 1, 1)], np.int32), np.ones(4, np.float32))
+        for f in range(3, 9):
+            ctx.set(f, 0, rng.random((nz, ny, nx), np.float32) - 0.5)
+        ctx.run(3)
+        out = torch.empty((9, nz, ny, nx), device="cuda")
+        ctx.snapshot(out.data_ptr())
+        torch.cuda.synchronize()
+    return out
+
+
+def test_very_long_rows():
+    """Rows of tens of thousands of tiles: a tile's row is its number divided
+    by that count."""
+    shape = (1900757, 3, 3)
+    print(f"\nlong rows {shape}", flush=True)
+    a, b = _long_row(shape, False), _long_row(shape, True)
+    for f in range(9):
+        assert torch.equal(a[f].view(torch.int32), b[f].view(torch.int32)), F.FIELDS[f]
+    assert a.isfinite().all() and (a.abs().amax(dim=(1, 2, 3)) > 0).all()
