@@ -55,6 +55,7 @@ EXPORTS = {
                    "fdtd_batch_remove", "fdtd_batch_run", "fdtd_batch_status", "fdtd_batch_probe_read",
                    "fdtd_batch_probe_peak_units",
                    "fdtd_batch_get_field", "fdtd_batch_set_shape", "fdtd_batch_autotune", "fdtd_batch_info",
+                   "fdtd_batch_by_cells",
                    "fdtd_dropin_solve", "fdtd_dropin_solve_noalloc", "fdtd_stream_probe", "fdtd_stream_probe_layout", "fdtd_load_tissue_table", "fdtd_load_phantom_ids",
                    "fdtd_serve_create", "fdtd_serve_destroy", "fdtd_serve_submit", "fdtd_serve_wait",
                    "fdtd_serve_result", "fdtd_serve_release", "fdtd_serve_drain", "fdtd_serve_stats"],
@@ -200,6 +201,7 @@ def lib():
         L.fdtd_batch_set_shape.argtypes = [vp, i, i, i]
         L.fdtd_batch_autotune.argtypes = [vp, i, vp, C.POINTER(C.c_int), C.POINTER(C.c_int)]
         L.fdtd_batch_info.argtypes = [vp, C.POINTER(FdtdBatchInfo)]
+        L.fdtd_batch_by_cells.argtypes = [vp, i]
         L.fdtd_dropin_solve.argtypes = [PP, PE, PI, vp, vp]
         L.fdtd_dropin_solve_noalloc.argtypes = [PP, PE, PI, vp, vp]
         L.fdtd_stream_probe.argtypes = [C.c_longlong, i, i, C.POINTER(C.c_double), C.POINTER(C.c_double)]
@@ -677,6 +679,13 @@ class Batch:
         ty, kc = C.c_int(), C.c_int()
         check(lib().fdtd_batch_autotune(self._h, trial_steps, stream, C.byref(ty), C.byref(kc)), "autotune")
         return ty.value, kc.value
+
+    def by_cells(self, i):
+        """Whether grid i is stepped in groups by cells, not in tiles."""
+        r = lib().fdtd_batch_by_cells(self._h, i)
+        if r < 0:
+            check(r, "fdtd_batch_by_cells")
+        return r == 1
 
     def info(self):
         inf = FdtdBatchInfo()

@@ -862,6 +862,12 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
     return 0;
 }
 
+extern "C" int fdtd_batch_by_cells(fdtd_batch *b, int id)
+{
+    if (!b || id < 0 || id >= (int)b->in.size() || !b->in[id].used) return fdtd_fail(FDTD_EINVAL, "bad instance id %d", id);
+    return cell_grid(b, b->in[id]) ? 1 : 0;
+}
+
 extern "C" int fdtd_batch_info(fdtd_batch *b, FdtdBatchInfo *info)
 {
     if (!b || !info) return fdtd_fail(FDTD_EINVAL, "null argument");

@@ -372,6 +372,8 @@ int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int graph_steps)
  * their zero initial state.  Every grid must be unstepped. */
 int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t stream, int *tile_y, int *kchunk);
 int fdtd_batch_info(fdtd_batch *b, FdtdBatchInfo *info);
+/* Whether grid `id` is stepped in groups by cells (1) or in tiles (0). */
+int fdtd_batch_by_cells(fdtd_batch *b, int id);
 
 /* One grid solved through the five drop-in entry points of
  * fdtd_calculations.h, as the reference's main loop drives them

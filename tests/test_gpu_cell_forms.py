@@ -39,3 +39,36 @@ def test_very_long_rows():
     for f in range(9):
         assert torch.equal(a[f].view(torch.int32), b[f].view(torch.int32)), F.FIELDS[f]
     assert a.isfinite().all() and (a.abs().amax(dim=(1, 2, 3)) > 0).all()
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("graph_steps", [0, 7])
+def test_batch_cells_and_tiles_together(graph_steps):
+    """A batch whose grids step partly in tiles (graphs that count the steps on
+    the device) and partly in groups (step numbers from the host): runs that
+    are no multiple of a graph's steps, and grids of both kinds that join late
+    and end inside a run."""
+    from tests.test_gpu_batch import assert_same, make_case, single
+    deep = 60001   # more planes than cell_step takes
+    insts = [make_case(600, (3, 4, deep), 4, 41), make_case(601, (30, 20, 25), 5, 77),
+             make_case(602, (3, 3, deep), 3, 23, F.STORE_F16), make_case(603, (66, 9, 12), 6, 19, F.STORE_F16),
+             make_case(604, (3, 4, deep), 4, 66), make_case(605, (33, 17, 20), 4, 90)]
+    print(f"\ncells and tiles, {graph_steps} steps a graph", flush=True)
+    refs = [single(x) for x in insts]
+    with F.Batch(8 << 30) as b:
+        b.set_shape(graph_steps=graph_steps)
+        ids = [b.add(x) for x in insts[:4]]
+        assert [b.by_cells(i) for i in ids] == [False, True, False, True]
+        b.run(13)
+        ids += [b.add(x) for x in insts[4:]]
+        b.run(1)
+        b.run(45)                      # both early tiled grids end inside
+        assert b.info()["running"] == 3
+        b.run(75)
+        assert b.info()["running"] == 0
+        for q, (i, x) in enumerate(zip(ids, insts)):
+            assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
+        b.remove(ids[1])               # only tiles, then none running
+        last = b.add(insts[0])
+        b.run(50)
+        assert_same(b, last, insts[0], refs[0], "tiles alone")
