@@ -801,6 +801,10 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
     const int tys[3] = {2, 4, 8}, kcs[5] = {3, 4, 6, 8, 16};
     float best = 0.0f;
     int bty = b->ty, bkc = b->kchunk;
+    const bool by_cell0 = b->by_cell;
+    b->by_cell = true;
+    const bool any_cell = std::any_of(b->in.begin(), b->in.end(),
+                                      [&](const fdtd_batch::Inst &I) { return I.used && cell_grid(b, I); });
     auto trial = [&](int n) -> float {   // ms per step over n steps as the batch is set up now
         b->dirty = true;
         rc = fdtd_batch_run(b, 2, stream);  // builds the graphs, uploads the tables
@@ -826,13 +830,14 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
                 bkc = kcs[c];
             }
         }
-    bool bcells = false;
-    if (!rc) {
+    // The groups, if a grid may step in one; without one (or after an error) the choice stays, for the grids to come.
+    bool bcells = by_cell0;
+    if (!rc && any_cell) {
         b->by_cell = true;
         b->ty = bty;
         b->kchunk = bkc;
         const float ms = trial(std::max(trial_steps, kCellRunSteps));   // each group's steps in a row, as a run takes them
-        bcells = !rc && ms < best;
+        if (!rc) bcells = ms < best;
     }
     b->by_cell = bcells;
     if (t0) (void)hipEventDestroy(t0);

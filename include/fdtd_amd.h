@@ -367,9 +367,9 @@ int fdtd_batch_get_field(fdtd_batch *b, int id, int field, int level, float *hos
  * results). */
 int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int graph_steps);
 /* Times every (tile_y in {2,4,8}, kchunk in {3,4,6,8,16}) candidate on the batch's own grids for
- * trial_steps steps each, and the groups of small grids, keeps the fastest (tile_y and kchunk: of the
- * shapes) and restores the grids to
- * their zero initial state.  Every grid must be unstepped. */
+ * trial_steps steps each, and the groups where a grid may step in one (otherwise the batch goes on
+ * choosing by grid, or in tiles, as before), keeps the fastest (tile_y and kchunk: of the shapes) and
+ * restores the grids to their zero initial state.  Every grid must be unstepped. */
 int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t stream, int *tile_y, int *kchunk);
 int fdtd_batch_info(fdtd_batch *b, FdtdBatchInfo *info);
 /* Whether grid `id` is stepped in groups by cells (1) or in tiles (0). */

@@ -72,3 +72,23 @@ def test_batch_cells_and_tiles_together(graph_steps):
         last = b.add(insts[0])
         b.run(50)
         assert_same(b, last, insts[0], refs[0], "tiles alone")
+
+
+@pytest.mark.parametrize("fixed", [False, True])
+def test_batch_autotune_without_cell_grids_keeps_the_choice(fixed):
+    """Where no grid may step by cells there is nothing to choose: grids that
+    are added later step as they would without the autotuner."""
+    from tests.test_gpu_batch import make_case
+    with F.Batch(2 << 30) as b:
+        if fixed:
+            b.set_shape(tile_y=4, kchunk=8)
+        for _ in range(3):
+            deep = b.add(make_case(610, (3, 3, 60001), 3, 9))
+            print(f"\nautotune in tiles, fixed={fixed}", flush=True)
+            b.autotune(trial_steps=1)
+            assert not b.by_cells(deep)
+            small = b.add(make_case(611, (20, 20, 20), 3, 9))
+            assert b.by_cells(small) == (not fixed)
+            b.run(9)
+            b.remove(small)
+            b.remove(deep)
