@@ -776,10 +776,16 @@ extern "C" int fdtd_step_fused(fdtd_ctx *c, hipStream_t stream)
     if (by_cells(c)) {
         c->n = n + 1;
         c->hcur ^= 1;
+        const int rows = c->probe_rows;
         CellArgs q;
         fill_cell_args(c, a, q);
         const hipError_t e = launch_cell_step(q, c->storage, stream, t0, t1);
-        if (e != hipSuccess) return fdtd_hip_fail(e, "cell_step");
+        if (e != hipSuccess) {   // no step was made
+            c->n = n;
+            c->hcur ^= 1;
+            c->probe_rows = rows;
+            return fdtd_hip_fail(e, "cell_step");
+        }
         if (timed) c->tused++;
         return after_step(c, stream);
     }

@@ -92,3 +92,36 @@ def test_batch_autotune_without_cell_grids_keeps_the_choice(fixed):
             b.run(9)
             b.remove(small)
             b.remove(deep)
+
+
+def test_step_that_cannot_be_launched_is_not_counted():
+    """A step whose launch the runtime refuses (here: on a stream whose capture
+    is no longer valid) leaves the context as it was."""
+    import ctypes as C
+
+    from fdtd_amd import hip
+    rt = hip.rt()
+    rt.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    rt.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    out = []
+    for refuse in (False, True):
+        with F.Context(F.make_params((20, 18, 16), DT, DX, mu0=MU0, eps0=EPS0)) as ctx:
+            ctx.set_sources(np.asarray([(9, 8, 7)], np.int32), np.linspace(1.0, 2.0, 9).astype(np.float32))
+            ctx.set_probes(np.asarray([(8, 9, 8, 7), (3, 8, 8, 7)], np.int32), 9)
+            assert ctx.by_cells()
+            ctx.run(4)
+            hip.sync()
+            if refuse:
+                s, graph = hip.Stream(), C.c_void_p()
+                hip.ok(rt.hipStreamBeginCapture(s.handle, 1), "begin capture")   # thread-local
+                assert rt.hipStreamSynchronize(s.handle) != 0                    # ends its validity
+                with pytest.raises(F.FdtdError):
+                    ctx.step(s.handle)
+                rt.hipStreamEndCapture(s.handle, C.byref(graph))
+                s.destroy()
+                rt.hipGetLastError()
+                assert F.lib().fdtd_ctx_steps_done(ctx._h) == 4 and len(ctx.probes()) == 4
+            ctx.run(5)
+            out.append((ctx.probes(), ctx.get(8)))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert np.abs(out[0][0]).max() > 0
