@@ -570,13 +570,8 @@ __global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), BXL)) void cell_s
     // What the lanes need of the arguments before their loads can go out, and
     // something of the other cache lines, in one go: left alone, each first use
     // of a line, and each of these, waits in turn (24^3: 5.9 -> 5.2 us a step, 64^3
-    // 8.2 -> 8.0).  Never taken: addresses and pitches are even, counts are not
-    // negative.
-    uintptr_t odd = (uintptr_t)C.ids | (uintptr_t)C.mur[0] | (uintptr_t)C.dT[0] | (uintptr_t)C.d1[0] | (uintptr_t)C.lut;
-    for (int q = 0; q < 3; q++) odd |= (uintptr_t)C.e0[q] | (uintptr_t)C.h0[q] | (uintptr_t)C.d0[q];
-    odd |= C.o0 | C.sy | C.sz;
-    const int neg = C.nx | C.ny | C.nz | C.tiles_x | C.tiles | C.run | C.flip;
-    if (((uint32_t)odd & 1u) | ((uint32_t)neg >> 31)) return;
+    // 8.2 -> 8.0).  Never taken: the launch has checked the same.
+    if (!cell_args_ok(C)) return;
     cell_block<T, EXACT, BXL, FORM>(OneStep{C}, (int)blockIdx.x, (int)blockIdx.y);
 }
 
@@ -613,6 +608,7 @@ __global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), 6)) void cell_bat
 template <typename T, bool EXACT>
 hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
 {
+    if (!cell_args_ok(c)) return hipErrorInvalidValue;
     const void *wide[] = {(const void *)cell_step<T, EXACT, 6, kCellNear>, (const void *)cell_step<T, EXACT, 6, kCellMid>,
                           (const void *)cell_step<T, EXACT, 6, sizeof(T) == 2 ? kCellPart : kCellFar>,
                           (const void *)cell_step<T, EXACT, 6, kCellFar>};

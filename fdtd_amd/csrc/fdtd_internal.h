@@ -221,6 +221,15 @@ struct CellArgs {
     const float4 *mur[6];          // launch_mur_coefs: x low, x high, y low, ...
     ProbeArgs p;                   // p.nprobe = 0: no probe row; p.field is not read
 };
+// Even addresses and pitches, counts that are not negative.
+__host__ __device__ inline bool cell_args_ok(const CellArgs &c)
+{
+    uintptr_t odd = (uintptr_t)c.ids | (uintptr_t)c.mur[0] | (uintptr_t)c.dT[0] | (uintptr_t)c.d1[0] | (uintptr_t)c.lut;
+    for (int q = 0; q < 3; q++) odd |= (uintptr_t)c.e0[q] | (uintptr_t)c.h0[q] | (uintptr_t)c.d0[q];
+    odd |= c.o0 | c.sy | c.sz;
+    const int neg = c.nx | c.ny | c.nz | c.tiles_x | c.tiles | c.run | c.flip;
+    return !(((uint32_t)odd & 1u) | ((uint32_t)neg >> 31));
+}
 // Padded state (bytes of the 24 field arrays) up to which a context steps
 // with cell_step.  Far past the Infinity Cache both launches wait for HBM, and
 // the tiled one keeps more of it in flight; what cell_step gains there is the

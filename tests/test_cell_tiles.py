@@ -9,6 +9,27 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
+CHECK = r"""
+#include <cstdio>
+#include <cstring>
+#include "fdtd_internal.h"
+int main()
+{
+    CellArgs c;
+    memset((void *)&c, 0, sizeof c);
+    c.nx = c.ny = c.nz = 3;
+    if (!cell_args_ok(c)) return 1;
+    CellArgs d = c; d.e0[2] = (const char *)0x1001;
+    if (cell_args_ok(d)) return 2;
+    d = c; d.sy = 129;
+    if (cell_args_ok(d)) return 3;
+    d = c; d.ids = (const uint8_t *)0x77;
+    if (cell_args_ok(d)) return 4;
+    d = c; d.run = -1;
+    return cell_args_ok(d) ? 5 : 0;
+}
+"""
+
 PROGRAM = r"""
 #include <cstdio>
 #include <cstdlib>
@@ -43,12 +64,21 @@ SHAPES = [(3, 3), (64, 5), (65, 130), (96, 37), (150, 150), (1024, 1024), (85016
           (950358, 33), (1900757, 3)]
 
 
-@pytest.mark.parametrize("esz", [4, 2])
-def test_tiles_map_to_rows(tmp_path, esz):
-    src, exe = tmp_path / "tiles.cpp", tmp_path / "tiles"
-    src.write_text(PROGRAM)
+def _build(tmp_path, text):
+    src, exe = tmp_path / "cells.cpp", tmp_path / "cells"
+    src.write_text(text)
     subprocess.run(["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{ROOT}/include",
                     f"-I{ROOT}/fdtd_amd/csrc", str(src), "-o", str(exe)], check=True)
+    return exe
+
+
+def test_launch_refuses_what_the_kernel_would_skip(tmp_path):
+    assert subprocess.run([str(_build(tmp_path, CHECK))]).returncode == 0
+
+
+@pytest.mark.parametrize("esz", [4, 2])
+def test_tiles_map_to_rows(tmp_path, esz):
+    exe = _build(tmp_path, PROGRAM)
     cases = [(nx, ny, form) for nx, ny in SHAPES for form in (0, 1, 3)]
     args = [str(v) for nx, ny, form in cases for v in (nx, ny, form, esz)]
     out = subprocess.run([str(exe), *args], capture_output=True, text=True, check=True).stdout.split()
