@@ -132,23 +132,14 @@ __device__ __forceinline__ float at_once(const char *p, uint32_t b)
     else return at<T>(p, b);
 }
 
-// A Mur face's new value q * x as storage type T holds it.  The compiler
-// rounds the Mur kernel's fp16 product once, to fp16 (v_fma_mixlo_f16), and
-// the x faces that the tiled step updates twice, by way of fp32; `once` says
-// which of the two the tiled step gives this face.
+// A Mur face's new value q * x as storage type T holds it; `once` says which
+// of the two roundings the tiled step gives this face.
 template <typename T>
 __device__ __forceinline__ float mur_round(float q, float x, bool once)
 {
-    float v = q * x;
-    if constexpr (std::is_same<T, __half>::value) {
-        if (once) {
-            uint32_t r = 0;
-            asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "+v"(r) : "v"(q), "v"(x));
-            return Elem<T>::cvt((unsigned short)r);
-        }
-        asm("" : "+v"(v));
-    }
-    return Elem<T>::rnd(v);
+    if constexpr (std::is_same<T, __half>::value)
+        if (once) return mur_once<T>(q, x);
+    return Elem<T>::rnd(mur_twice<T>(q, x));
 }
 
 // The Mur coefficients of a face cell (launch_mur_coefs).

@@ -6,6 +6,8 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace {
 
 __device__ inline float e_update(float c, float d, float a, double g1, double g2, double g3, float e0, float e1,
@@ -86,6 +88,30 @@ template <> struct Elem<__hip_bfloat16> {
         __builtin_nontemporal_store(enc(v), (unsigned short *)((char *)p + b));
     }
 };
+
+// A Mur face's new value, the product q * x, as storage type T takes it.  A
+// compiler may round such a product and its conversion to fp16 together
+// (v_fma_mixlo_f16) or one after the other, so for fp16 both are spelled out:
+// mur_once rounds once, as the face kernels' faces do; mur_twice by way of fp32,
+// as the x faces do that a tile updates.  The other types know one way.
+template <typename T>
+__device__ __forceinline__ float mur_once(float q, float x)
+{
+    if constexpr (std::is_same<T, __half>::value) {
+        uint32_t r = 0;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "+v"(r) : "v"(q), "v"(x));
+        return Elem<T>::cvt((unsigned short)r);
+    } else {
+        return q * x;
+    }
+}
+template <typename T>
+__device__ __forceinline__ float mur_twice(float q, float x)
+{
+    float v = q * x;
+    if constexpr (std::is_same<T, __half>::value) asm("" : "+v"(v));
+    return v;
+}
 
 // E^{n+1} in scaled units (16-bit storage): fp32 throughout.
 __device__ inline float e_update_scaled(float k1, float k2, float k3, float k5, float e0, float e1, float dn1,

@@ -68,12 +68,21 @@ __device__ inline int xcd_unit(int mode, int tiles_x, int tiles_y)
 // First-order Mur update of one face cell (fdtd_calculations.cu:237-427):
 // rpf/rpn are the face and neighbour permittivities, tn the neighbour at
 // n+1, sn and sf the neighbour and the face at n.
+struct MurProduct {
+    float q, x;   // the face's value is q * x
+};
+__device__ inline MurProduct mur_terms(float dt, float h, float mu0, float eps0, float rpf, float rpn, float tn,
+                                       float sn, float sf)
+{
+    return {1 / (dt + h * sqrtf(mu0 * eps0 * rpf)),
+            (dt - h * sqrtf(mu0 * eps0 * rpn)) * tn + (dt + h * sqrtf(mu0 * eps0 * rpn)) * sn -
+                (dt - h * sqrtf(mu0 * eps0 * rpf)) * sf};
+}
 __device__ inline float mur1(float dt, float h, float mu0, float eps0, float rpf, float rpn, float tn, float sn,
                              float sf)
 {
-    return 1 / (dt + h * sqrtf(mu0 * eps0 * rpf)) *
-           ((dt - h * sqrtf(mu0 * eps0 * rpn)) * tn + (dt + h * sqrtf(mu0 * eps0 * rpn)) * sn -
-            (dt - h * sqrtf(mu0 * eps0 * rpf)) * sf);
+    const MurProduct p = mur_terms(dt, h, mu0, eps0, rpf, rpn, tn, sn, sf);
+    return p.q * p.x;
 }
 
 // All per-lane addresses are a 64-bit array base (uniform, in SGPRs) plus a
@@ -435,12 +444,12 @@ __device__ __forceinline__ void fused_tile(const StepArgs &A, int bx, int by, in
             if (tx == 0 && j < ny) {
                 const float4 c = sMurC[0][k - k0][ty];
                 if (j < ny - 1 && k >= 1 && k < nz - 1) {
-                    eyn = c.x * ((c.y * ey1 + c.z * sE[cur][1][ty + 1][2]) - c.w * eyk);
+                    eyn = mur_twice<T>(c.x, (c.y * ey1 + c.z * sE[cur][1][ty + 1][2]) - c.w * eyk);
                     sty = true;
                 }
                 if (j >= 1 && j < ny - 1 && k < nz - 1) {
                     const float tn = k >= 1 ? ez1 : sMurT[0][ty];
-                    ezn = c.x * ((c.y * tn + c.z * sE[cur][2][ty + 1][2]) - c.w * ezk);
+                    ezn = mur_twice<T>(c.x, (c.y * tn + c.z * sE[cur][2][ty + 1][2]) - c.w * ezk);
                     stz = true;
                 }
             }
@@ -452,12 +461,12 @@ __device__ __forceinline__ void fused_tile(const StepArgs &A, int bx, int by, in
                 if (j < ny - 1 && k >= 1 && k < nz - 1) {
                     // the x-high Ey face reads the source neighbour twice (fdtd_calculations.cu:323-325)
                     const float sn = sE[cur][1][ty + 1][tx];
-                    eyn = c.x * ((c.y * sn + c.z * sn) - c.w * eyk);
+                    eyn = mur_twice<T>(c.x, (c.y * sn + c.z * sn) - c.w * eyk);
                     sty = true;
                 }
                 if (j >= 1 && j < ny - 1 && k < nz - 1) {
                     const float tn = k >= 1 ? ezm : sMurT[1][ty];
-                    ezn = c.x * ((c.y * tn + c.z * sE[cur][2][ty + 1][tx]) - c.w * ezk);
+                    ezn = mur_twice<T>(c.x, (c.y * tn + c.z * sE[cur][2][ty + 1][tx]) - c.w * ezk);
                     stz = true;
                 }
             }
@@ -788,12 +797,12 @@ __device__ __forceinline__ void fused_tile_pair(const StepArgs &A, int bx, int b
         if (mur_lo && tx == 0 && j < ny) {  // face i = 0 is cell a of lane 0, its neighbour cell b
             const float4 cm = sMurC[0][k - k0][ty];
             if (j < ny - 1 && k >= 1 && k < nz - 1) {
-                eyn[0] = cm.x * ((cm.y * X::rnd(eyn[1]) + cm.z * lx(sE[cur][1][ty + 1], 2)) - cm.w * eyk[0]);
+                eyn[0] = mur_twice<T>(cm.x, (cm.y * X::rnd(eyn[1]) + cm.z * lx(sE[cur][1][ty + 1], 2)) - cm.w * eyk[0]);
                 sty[0] = true;
             }
             if (j >= 1 && j < ny - 1 && k < nz - 1) {
                 const float tn = k >= 1 ? X::rnd(ezn[1]) : sMurT[0][ty];
-                ezn[0] = cm.x * ((cm.y * tn + cm.z * lx(sE[cur][2][ty + 1], 2)) - cm.w * ezk[0]);
+                ezn[0] = mur_twice<T>(cm.x, (cm.y * tn + cm.z * lx(sE[cur][2][ty + 1], 2)) - cm.w * ezk[0]);
                 stz[0] = true;
             }
         }
@@ -809,12 +818,12 @@ __device__ __forceinline__ void fused_tile_pair(const StepArgs &A, int bx, int b
                 const int c = ca + h;
                 if (j < ny - 1 && k >= 1 && k < nz - 1) {
                     const float sn = lx(sE[cur][1][ty + 1], c - 1);
-                    eyn[h] = cm.x * ((cm.y * sn + cm.z * sn) - cm.w * eyk[h]);
+                    eyn[h] = mur_twice<T>(cm.x, (cm.y * sn + cm.z * sn) - cm.w * eyk[h]);
                     sty[h] = true;
                 }
                 if (j >= 1 && j < ny - 1 && k < nz - 1) {
                     const float tn = k >= 1 ? (h ? X::rnd(ezn[0]) : ezm) : sMurT[1][ty];
-                    ezn[h] = cm.x * ((cm.y * tn + cm.z * lx(sE[cur][2][ty + 1], c - 1)) - cm.w * ezk[h]);
+                    ezn[h] = mur_twice<T>(cm.x, (cm.y * tn + cm.z * lx(sE[cur][2][ty + 1], c - 1)) - cm.w * ezk[h]);
                     stz[h] = true;
                 }
             }
@@ -1359,7 +1368,7 @@ __global__ __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(PAIR ? 4
 }
 
 // New value of face cell (i, j, k) of Mur segment s (fdtd_calculations.cu:
-// 237-427): E'_f = mur1(rp_face, rp_nb, E'_nb, E^n_nb, E^n_f) with the
+// 237-427): E'_f = mur_terms(rp_face, rp_nb, E'_nb, E^n_nb, E^n_f) with the
 // neighbour one cell inward along the face normal.  Segments: 0, 1 Ex at
 // j = 0, ny-1; 2, 3 Ex at k = 0, nz-1; 4, 5 Ey at i = 0, nx-1; 6, 7 Ey at
 // k = 0, nz-1; 8, 9 Ez at i = 0, nx-1; 10, 11 Ez at j = 0, ny-1.  Every
@@ -1378,21 +1387,23 @@ __device__ __forceinline__ float mur_value(const MurArgs &M, int s, int i, int j
     auto rpy = [&](const float *p, int jj) { return p[(long long)k * 2 * nx + (long long)jj * nx + i]; };
     auto rpz = [&](const float *p, int kk) { return p[(long long)kk * ny * nx + (long long)j * nx + i]; };
     auto rpx = [&](const float *p, int ii) { return p[(long long)k * ny * 2 + (long long)j * 2 + ii]; };
+    MurProduct v;
     switch (s) {
-    case 0: return mur1(dt, M.hy, m0, e0, rpy(M.rpy0, 0), rpy(M.rpy0, 1), G(exT, o + sy), G(exS, o + sy), G(exS, o));
-    case 1: return mur1(dt, M.hy, m0, e0, rpy(M.rpyEnd, 1), rpy(M.rpyEnd, 0), G(exT, o - sy), G(exS, o - sy), G(exS, o));
-    case 2: return mur1(dt, M.hz, m0, e0, rpz(M.rpz0, 0), rpz(M.rpz0, 1), G(exT, o + sz), G(exS, o + sz), G(exS, o));
-    case 3: return mur1(dt, M.hz, m0, e0, rpz(M.rpzEnd, 1), rpz(M.rpzEnd, 0), G(exT, o - sz), G(exS, o - sz), G(exS, o));
-    case 4: return mur1(dt, M.hx, m0, e0, rpx(M.rpx0, 0), rpx(M.rpx0, 1), G(eyT, o + 1), G(eyS, o + 1), G(eyS, o));
+    case 0: v = mur_terms(dt, M.hy, m0, e0, rpy(M.rpy0, 0), rpy(M.rpy0, 1), G(exT, o + sy), G(exS, o + sy), G(exS, o)); break;
+    case 1: v = mur_terms(dt, M.hy, m0, e0, rpy(M.rpyEnd, 1), rpy(M.rpyEnd, 0), G(exT, o - sy), G(exS, o - sy), G(exS, o)); break;
+    case 2: v = mur_terms(dt, M.hz, m0, e0, rpz(M.rpz0, 0), rpz(M.rpz0, 1), G(exT, o + sz), G(exS, o + sz), G(exS, o)); break;
+    case 3: v = mur_terms(dt, M.hz, m0, e0, rpz(M.rpzEnd, 1), rpz(M.rpzEnd, 0), G(exT, o - sz), G(exS, o - sz), G(exS, o)); break;
+    case 4: v = mur_terms(dt, M.hx, m0, e0, rpx(M.rpx0, 0), rpx(M.rpx0, 1), G(eyT, o + 1), G(eyS, o + 1), G(eyS, o)); break;
     // the x-high Ey face reads the source neighbour twice (fdtd_calculations.cu:323-325)
-    case 5: return mur1(dt, M.hx, m0, e0, rpx(M.rpxEnd, 1), rpx(M.rpxEnd, 0), G(eyS, o - 1), G(eyS, o - 1), G(eyS, o));
-    case 6: return mur1(dt, M.hz, m0, e0, rpz(M.rpz0, 0), rpz(M.rpz0, 1), G(eyT, o + sz), G(eyS, o + sz), G(eyS, o));
-    case 7: return mur1(dt, M.hz, m0, e0, rpz(M.rpzEnd, 1), rpz(M.rpzEnd, 0), G(eyT, o - sz), G(eyS, o - sz), G(eyS, o));
-    case 8: return mur1(dt, M.hx, m0, e0, rpx(M.rpx0, 0), rpx(M.rpx0, 1), G(ezT, o + 1), G(ezS, o + 1), G(ezS, o));
-    case 9: return mur1(dt, M.hx, m0, e0, rpx(M.rpxEnd, 1), rpx(M.rpxEnd, 0), G(ezT, o - 1), G(ezS, o - 1), G(ezS, o));
-    case 10: return mur1(dt, M.hy, m0, e0, rpy(M.rpy0, 0), rpy(M.rpy0, 1), G(ezT, o + sy), G(ezS, o + sy), G(ezS, o));
-    default: return mur1(dt, M.hy, m0, e0, rpy(M.rpyEnd, 1), rpy(M.rpyEnd, 0), G(ezT, o - sy), G(ezS, o - sy), G(ezS, o));
+    case 5: v = mur_terms(dt, M.hx, m0, e0, rpx(M.rpxEnd, 1), rpx(M.rpxEnd, 0), G(eyS, o - 1), G(eyS, o - 1), G(eyS, o)); break;
+    case 6: v = mur_terms(dt, M.hz, m0, e0, rpz(M.rpz0, 0), rpz(M.rpz0, 1), G(eyT, o + sz), G(eyS, o + sz), G(eyS, o)); break;
+    case 7: v = mur_terms(dt, M.hz, m0, e0, rpz(M.rpzEnd, 1), rpz(M.rpzEnd, 0), G(eyT, o - sz), G(eyS, o - sz), G(eyS, o)); break;
+    case 8: v = mur_terms(dt, M.hx, m0, e0, rpx(M.rpx0, 0), rpx(M.rpx0, 1), G(ezT, o + 1), G(ezS, o + 1), G(ezS, o)); break;
+    case 9: v = mur_terms(dt, M.hx, m0, e0, rpx(M.rpxEnd, 1), rpx(M.rpxEnd, 0), G(ezT, o - 1), G(ezS, o - 1), G(ezS, o)); break;
+    case 10: v = mur_terms(dt, M.hy, m0, e0, rpy(M.rpy0, 0), rpy(M.rpy0, 1), G(ezT, o + sy), G(ezS, o + sy), G(ezS, o)); break;
+    default: v = mur_terms(dt, M.hy, m0, e0, rpy(M.rpyEnd, 1), rpy(M.rpyEnd, 0), G(ezT, o - sy), G(ezS, o - sy), G(ezS, o));
     }
+    return mur_once<T>(v.q, v.x);
 }
 
 // The Mur segment that holds cell (i, j, k) of E component c (0 Ex, 1 Ey,

@@ -125,3 +125,51 @@ def test_step_that_cannot_be_launched_is_not_counted():
             out.append((ctx.probes(), ctx.get(8)))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert np.abs(out[0][0]).max() > 0
+
+
+def _mur(h, dt, rpf, rpn, tn, sn, sf):
+    """q and x of a face's new value q * x, in fp32 (fdtd_calculations.cu:216-428)."""
+    f = np.float32
+    k = f(MU0) * f(EPS0)
+    rf, rn = np.sqrt(k * rpf), np.sqrt(k * rpn)
+    h, dt = f(h), f(dt)
+    return f(1) / (dt + h * rf), ((dt - h * rn) * tn + (dt + h * rn) * sn) - (dt - h * rf) * sf
+
+
+@pytest.mark.parametrize("nx", [96, 65])
+@pytest.mark.parametrize("tile_y", [0, 4])
+def test_fp16_faces_round_as_stated(nx, tile_y):
+    """Faces of the Mur kernel round their fp16 product once; x faces that a
+    tile updates (all but the high ones of a row that starts a tile) by way of
+    fp32; and the one-lane-per-cell step as the tiles do."""
+    ny, nz = 260, 250
+    rng = np.random.default_rng([nx, tile_y])
+    rps = [rng.uniform(1.0, 3.0, n).astype(np.float32) for n in (2 * ny * nz, nx * 2 * nz, nx * ny * 2) * 2]
+    with F.Context(F.make_params((nx, ny, nz), DT, DX, mu0=MU0, eps0=EPS0), storage=F.STORE_F16, scales=(1.0, 1.0, 1.0),
+                   tile_y=tile_y) as ctx:
+        assert ctx.by_cells() == (tile_y == 0)
+        ctx.set_rp(rps)
+        for f in range(6, 9):
+            ctx.set(f, 0, rng.uniform(-1, 1, (nz, ny, nx)).astype(np.float32))
+        old = [ctx.get(f) for f in range(6, 9)]
+        ctx.step()
+        new = [ctx.get(f) for f in range(6, 9)]
+    inner = slice(1, -1)
+    rpy, rpye = rps[1].reshape(nz, 2, nx), rps[4].reshape(nz, 2, nx)
+    rpx, rpxe = rps[0].reshape(nz, ny, 2), rps[3].reshape(nz, ny, 2)
+    faces = []   # name, stored, (q, x), rounds once
+    for name, j, jn, rf, rn in (("Ex y0", 0, 1, rpy[:, 0], rpy[:, 1]), ("Ex y1", -1, -2, rpye[:, 1], rpye[:, 0])):
+        s = (inner, slice(0, -1))
+        e = [a[:, j][s] for a in (new[0], old[0])] + [a[:, jn][s] for a in (new[0], old[0])]
+        faces.append((name, e[0], _mur(DX, DT, rf[s], rn[s], e[2], e[3], e[1]), True))
+    for name, i, im, rf, rn in (("Ez x0", 0, 1, rpx[..., 0], rpx[..., 1]), ("Ez x1", -1, -2, rpxe[..., 1], rpxe[..., 0])):
+        s = (inner, inner)
+        e = [a[:, :, i][s] for a in (new[2], old[2])] + [a[:, :, im][s] for a in (new[2], old[2])]
+        faces.append((name, e[0], _mur(DX, DT, rf[s], rn[s], e[2], e[3], e[1]), i == -1 and nx == 65))
+    for name, got, (q, x), once in faces:
+        one = (q.astype(np.float64) * x.astype(np.float64)).astype(np.float16).astype(np.float32)
+        two = (q * x).astype(np.float16).astype(np.float32)
+        want = one if once else two
+        assert np.array_equal(got, want), f"{name}: {np.count_nonzero(got != want)} cells"
+        if nx == 96 and name == "Ez x0":
+            assert (one != two).any()   # the two differ somewhere in these inputs
