@@ -629,7 +629,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.sz = (uint32_t)(L.plane * L.esz);
     cell_tiles(nx, ny, cell_form(24 * L.Np * L.esz, L.esz), L.esz, c);
     for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
-    c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : 0;
+    c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : ZeroTerms{};
     c.nprobe = d.nprobe;
     c.probe_rows = d.probe_rows;
     c.jz_len = d.jz_len;

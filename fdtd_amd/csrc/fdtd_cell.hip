@@ -172,7 +172,7 @@ struct OneStep {
     __device__ __forceinline__ const MatCoef * lut() const { return a.lut; }
     __device__ __forceinline__ float ch(int q) const { return a.ch[q]; }
     __device__ __forceinline__ float cd(int q) const { return a.cd[q]; }
-    __device__ __forceinline__ uint32_t zmask() const { return a.zmask; }
+    __device__ __forceinline__ ZeroTerms zmask() const { return a.zmask; }
     __device__ __forceinline__ int hi_once() const { return a.hi_once; }
     __device__ __forceinline__ int flip() const { return a.flip; }
     __device__ __forceinline__ const char * e0(int q) const { return a.e0[q]; }
@@ -221,7 +221,7 @@ struct BatchStep {
     __device__ __forceinline__ const MatCoef * lut() const { return d->lut; }
     __device__ __forceinline__ float ch(int q) const { return d->ch[q]; }
     __device__ __forceinline__ float cd(int q) const { return d->cd[q]; }
-    __device__ __forceinline__ uint32_t zmask() const { return d->zmask; }
+    __device__ __forceinline__ ZeroTerms zmask() const { return {{d->zmask.w[0], d->zmask.w[1], d->zmask.w[2], d->zmask.w[3]}}; }
     __device__ __forceinline__ int hi_once() const { return d->hi_once; }
     __device__ __forceinline__ int flip() const { return n & 1; }
     __device__ __forceinline__ const char * e0(int q) const { return d->E[s0][q]; }
@@ -272,7 +272,7 @@ struct Ops {
 // BXL: log2 of the lanes of a block along x (32 or 64); the other lanes of its
 // cell_block_lanes are rows.  Exact form: cells whose material has a = g3 = +0 (zmask) do not
 // load E^{n-1} and D^{n-1}, as fused_tile's zero-term rows, decided per lane;
-// a grid that always loads them has zmask = 0.  C: where the step's operands
+// a grid that always loads them has an empty zmask.  C: where the step's operands
 // are (OneStep, BatchStep); block bx of the 8 * C.run() of plane bz.
 template <typename T, bool EXACT, int BXL, int FORM, typename G>
 __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
@@ -380,7 +380,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         v.k1 = q->k1; v.k2 = q->k2; v.k3 = q->k3; v.k5 = q->k5;
     }
     bool need = true;
-    if constexpr (EXACT) need = !(m < 32 && (C.zmask() >> m & 1u));
+    if constexpr (EXACT) need = !C.zmask().has(m);
     v.exm = v.eym = v.ezm = v.dxm = v.dym = v.dzm = 0.0f;
     if (need) {
         v.exm = at_once<T, NE>(C.e1(0), o); v.eym = at_once<T, NE>(C.e1(1), o); v.ezm = at_once<T, NE>(C.e1(2), o);

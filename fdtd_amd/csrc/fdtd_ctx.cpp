@@ -60,7 +60,7 @@ struct fdtd_ctx {
     unsigned char *ids = nullptr;
     MatCoef *lut = nullptr;
     int nmat = 0;
-    uint32_t zmask = 0;                  // bit m < 32: material m has a = g3 = +0 (CellArgs)
+    ZeroTerms zmask = {};                // of lut (CellArgs)
     std::vector<float> table;             // nmat x {sigma, eps_s, eps_inf, tau}
     bool lut_dirty = true;
     float *rp[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -609,7 +609,7 @@ void fill_cell_args(fdtd_ctx *c, const StepArgs &a, CellArgs &q)
     q.ch[0] = a.chx; q.ch[1] = a.chy; q.ch[2] = a.chz;
     q.cd[0] = a.cdx; q.cd[1] = a.cdy; q.cd[2] = a.cdz;
     q.jz = a.jz;
-    q.zmask = a.zskip ? c->zmask : 0;
+    q.zmask = a.zskip ? c->zmask : ZeroTerms{};
     q.hi_once = a.mur_x == 2;
     q.flip = c->n & 1;
     q.form = cell_form(24 * c->Np * c->esz, c->esz);

@@ -72,6 +72,34 @@ def _build(tmp_path, text):
     return exe
 
 
+MASK = r"""
+#include <cstring>
+#include "fdtd_internal.h"
+int main()
+{
+    MatCoef lut[kMaxMaterials];
+    memset((void *)lut, 0, sizeof lut);
+    auto zero = [](int m) { return m * 7 % 11 < 4; };
+    for (int m = 0; m < kMaxMaterials; m++) {
+        if (zero(m)) continue;
+        if (m % 3 == 0) lut[m].a = -0.0f;          // only +0 counts
+        else if (m % 3 == 1) lut[m].g3 = 1e-300;
+        else lut[m].a = 1e-38f;
+    }
+    for (int nmat : {1, 31, 32, 33, 64, 95, 97, 128}) {
+        const ZeroTerms z = cell_zmask(lut, nmat);
+        for (int m = 0; m < kMaxMaterials; m++)
+            if (z.has(m) != (m < nmat && zero(m))) return 1 + m;
+    }
+    return 0;
+}
+"""
+
+
+def test_zero_terms_of_every_material(tmp_path):
+    assert subprocess.run([str(_build(tmp_path, MASK))]).returncode == 0
+
+
 def test_launch_refuses_what_the_kernel_would_skip(tmp_path):
     assert subprocess.run([str(_build(tmp_path, CHECK))]).returncode == 0
 

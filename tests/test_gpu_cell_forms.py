@@ -173,3 +173,27 @@ def test_fp16_faces_round_as_stated(nx, tile_y):
         assert np.array_equal(got, want), f"{name}: {np.count_nonzero(got != want)} cells"
         if nx == 96 and name == "Ez x0":
             assert (one != two).any()   # the two differ somewhere in these inputs
+
+
+@pytest.mark.parametrize("first", [31, 32, 64, 95, 127])
+def test_zero_terms_of_high_material_ids(first):
+    """Materials of every id skip their zero terms, and no other does: the same
+    bits as with every operand loaded, in a grid that holds them all."""
+    shape = (70, 40, 30)
+    nx, ny, nz = shape
+    rng = np.random.default_rng(first)
+    table = np.asarray([(0.8, 55.0, 40.0, 8e-12)] * 128, np.float32)
+    table[first] = (0.0, 1.0, 1.0, 0.0)
+    ids = np.full((nz, ny, nx), first, np.uint8)
+    ids[8:20, 10:30, 20:60] = rng.integers(0, 128, (12, 20, 40))
+    jz = rng.uniform(-1, 1, 60).astype(np.float32)
+    out = []
+    for load in (0, 1):
+        with F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0), load_zero_terms=load) as ctx:
+            assert ctx.by_cells()
+            ctx.set_materials(ids, table)
+            ctx.set_sources(np.asarray([(30, 20, 15), (5, 5, 5)], np.int32), jz)
+            ctx.run(60)
+            out.append([ctx.get(f) for f in range(9)])
+    for f, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), F.FIELDS[f]
