@@ -247,19 +247,25 @@ __host__ __device__ inline bool cell_args_ok(const CellArgs &c)
 // Padded state (bytes of the 24 field arrays) up to which a context steps
 // with cell_step.  Far past the Infinity Cache both launches wait for HBM, and
 // the tiled one keeps more of it in flight; what cell_step gains there is the
-// part of the state that the last step left in the cache, less where waves at
-// the rows' ends are part empty.  fp32, us against tiles: rows of whole waves
-// 2.2 GB 387 (396), 3.1 GB 570 (565), 4.0 GB 725 (704); an odd number of half
-// waves (cell_lanes_log2) 340x300x170 318 (323), 160x400x300 352 (359), 2.1 GB
-// 392 (393), 2.2 GB 417 (414); others 1.1 GB 205 (206), 300x250x220 306 (307),
-// 300^3 504 (491).  16 bits: 1.5 GB 340 (383), 3.9 GB 844 (981), 4.3 GB 991
-// (1051), 6.4 GB 1555 (1544).
+// part of the state that the last step left in the cache.  fp32, tiles' time
+// over cell_step's, each with its own stagger of the arrays, means over two to
+// four placements that differ by less than 1 %:
+//   an odd number of half waves a row (cell_lanes_log2: two rows a wave): 96x450x450 1.00, 151x300x420 1.01, 160x400x300
+//     1.01, 223x300x300 1.03, 280x280x255 1.03, 350x330x178 1.02 (1.8 to 2.0 GB); 350x330x260 0.99, 410x300x240 1.00 (2.9);
+//   up to four half waves: 0.6 GB 1.04 to 1.06, 0.8 GB 1.00 to 1.06, 1.0 GB 0.95 to 1.00, 2.0 GB 0.92 to 0.95;
+//   six: 0.85 GB 1.06 to 1.08, 1.1 to 1.3 GB 0.99 to 1.02, 1.5 GB 0.95 to 0.97;
+//   more, whole waves: 1.6 GB 0.98 to 1.04, 320x320x224 1.03, 256x256x384 (2.4) 1.03, 2.5 to 2.6 GB 0.98 to 1.00;
+//   more, others: 1.2 GB 1.01 to 1.05, 300x250x220 (1.7) 0.97, 300^3 0.98, 500x300x250 (3.7) 0.97.
+// 16 bits: 1.03 to 1.3 for rows of 20 to 512 cells at 4.5 to 6 GB; 6.4 GB 0.99.
 constexpr int kCellMaxPlanes = 60000;   // planes and, in rows of at least 8 blocks, probes are blockIdx.y
 constexpr int kCellMaxProbes = 40000;
 inline size_t cell_state_limit(int nx, size_t esz)
 {
     if (esz == 2) return 6000000000;
-    return nx % 64 == 0 ? 2600000000 : (nx + 31) / 32 % 2 ? 2000000000 : 1200000000;
+    const int half = (nx + 31) / 32;
+    if (half % 2) return 2000000000;
+    if (half <= 4) return 850000000;
+    return half == 6 || nx % 64 ? 1200000000 : 2450000000;
 }
 // Its form, in us (near, mid, part, far; means over six placements of the
 // state, which differ by up to 15 %).  fp32: 201 MB 30.2, 30.4, 38, 38; 246 MB

@@ -227,10 +227,10 @@ int fdtd_slices_read(fdtd_ctx *ctx, int *steps, float *data, int max_slices);
 int fdtd_ctx_autotune(fdtd_ctx *ctx, int trial_steps, hipStream_t stream, int *tile_y, int *kchunk, int *lane_cells);
 
 /* The launch shape chosen for the context's fused kernel.  A context whose
- * FdtdExt fixes no part of the shape, and whose state is not too large (fp32:
- * 1.2 GB, rows of whole waves 2.6 GB, of an odd number of half waves 2 GB; 16
- * bits: 6 GB; at most 40000 probes), steps with one lane per
- * cell instead, one launch per step (same results), and does not use it:
+ * FdtdExt fixes no part of the shape, and whose state is not too large (fp32,
+ * by the half waves of 32 cells in a row: an odd number 2 GB; two or four
+ * 0.85 GB, six 1.2 GB; more 2.45 GB in whole waves, else 1.2 GB; 16 bits 6
+ * GB; at most 40000 probes), steps with one lane per cell instead, one launch per step (same results), and does not use it:
  * fdtd_ctx_by_cells returns 1. */
 int fdtd_ctx_launch_shape(fdtd_ctx *ctx, int *tile_x, int *tile_y, int *kchunk, int *blocks);
 int fdtd_ctx_by_cells(fdtd_ctx *ctx);
