@@ -255,7 +255,7 @@ void make_groups(fdtd_batch *b, std::vector<int> cell, DevTables *T)
 {
     b->groups.clear();
     auto bytes = [&](int s) { return 24 * b->in[s].L.Np * b->in[s].L.esz; };
-    auto form = [&](int s) { return cell_form(bytes(s), b->in[s].L.esz); };
+    auto form = [&](int s) { return cell_form(b->in[s].d.nx, bytes(s), b->in[s].L.esz); };
     std::sort(cell.begin(), cell.end(), [&](int p, int q) {
         const int sp = b->in[p].d.storage, sq = b->in[q].d.storage;
         if (sp != sq) return sp < sq;
@@ -627,7 +627,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.o0 = (uint32_t)gb;
     c.sy = (uint32_t)(L.pitch * L.esz);
     c.sz = (uint32_t)(L.plane * L.esz);
-    cell_tiles(nx, ny, cell_form(24 * L.Np * L.esz, L.esz), L.esz, c);
+    cell_tiles(nx, ny, cell_form(nx, 24 * L.Np * L.esz, L.esz), L.esz, c);
     for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
     c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : ZeroTerms{};
     c.nprobe = d.nprobe;

@@ -213,8 +213,8 @@ struct ZeroTerms {
 // probe row (fdtd_cell.hip).  The field and id pointers lie fused_guard
 // elements before the arrays' origins; o0 = the guard in bytes.
 // Forms of cell_step: its state in the Infinity Cache; x neighbours from the
-// lanes beside instead of loads; the same with D past the cache; with D and
-// all but the loads of E^n past it.
+// lanes beside instead of loads; the same with D past the cache (16 bits); with
+// D and all but the loads of E^n past it (fp32).
 enum { kCellNear, kCellMid, kCellPart, kCellFar };
 struct CellArgs {
     const char *e0[3], *e1[3], *d0[3], *d1[3], *h0[3];   // E, D at levels n and n-1, H^{n-1/2}
@@ -256,7 +256,7 @@ __host__ __device__ inline bool cell_args_ok(const CellArgs &c)
 //   six: 0.85 GB 1.06 to 1.08, 1.1 to 1.3 GB 0.99 to 1.02, 1.5 GB 0.95 to 0.97;
 //   more, whole waves: 1.6 GB 0.98 to 1.04, 320x320x224 1.03, 256x256x384 (2.4) 1.03, 2.5 to 2.6 GB 0.98 to 1.00;
 //   more, others: 1.2 GB 1.01 to 1.05, 300x250x220 (1.7) 0.97, 300^3 0.98, 500x300x250 (3.7) 0.97.
-// 16 bits: 1.03 to 1.3 for rows of 20 to 512 cells at 4.5 to 6 GB; 6.4 GB 0.99.
+// 16 bits: 1.03 to 1.3 for rows of 20 to 512 cells at 4.5 to 6.4 GB.
 constexpr int kCellMaxPlanes = 60000;   // planes and, in rows of at least 8 blocks, probes are blockIdx.y
 constexpr int kCellMaxProbes = 40000;
 inline size_t cell_state_limit(int nx, size_t esz)
@@ -267,19 +267,25 @@ inline size_t cell_state_limit(int nx, size_t esz)
     if (half <= 4) return 850000000;
     return half == 6 || nx % 64 ? 1200000000 : 2450000000;
 }
-// Its form, in us (near, mid, part, far; means over six placements of the
-// state, which differ by up to 15 %).  fp32: 201 MB 30.2, 30.4, 38, 38; 246 MB
-// 34.4, 33.4, 44.9, 45.6; 285 MB 54.6, 51.5, 54.9, 55.9; 344 MB 68.6, 62.8,
-// 63.4, 65.5; 398 MB 85.2, 77.9, 76.8, 77.4; 491 MB 95.9, 89.6, 87.8, 88.1;
-// 679 MB 131, 126, 122, 119; 1.6 GB (one placement) 331, 310, 298, 293.  fp16:
-// 197 MB 43.4, 44.8, -, 57.8; 246 MB 74.5, 70.7, 65.3, 69.3; 340 MB 89.2, 84.0,
-// 78.0, 85.1; 403 MB 103, 95.9, 94.9, 99.1 (where E and H alone no longer fit
-// the cache); 566 MB 137, 129, 135, 135; 805 MB 194, 181, 183, 187; 1.1 GB 270,
-// 252, 249, 253; 1.5 GB 354, 327, 318, 320.
-inline int cell_form(size_t state, size_t esz)
+// Its form.  us of near, mid and far, or of near, mid and part, over rows of 64
+// to 320 cells, means over three or four placements, which differ by up to 2 %.
+// fp32: 220 MB 30 to 35, 30 to 35, 41 to 49; 270 MB 47 to 52, 44 to 50, 47 to 58;
+// 320 MB 65 to 70, 57 to 64, 57 to 71; 360 MB 75 to 83, 66 to 75, 60 to 76; 500 MB
+// 100 to 109, 93 to 102, 82 to 101.  16 bits: 222 MB 38 to 44, 39 to 41, 49 to 54;
+// 248 MB 44 to 51, 43 to 49, 53 to 58; 268 MB 54 to 61, 53 to 57, 58 to 63; 280 MB
+// 63 to 71, 59 to 67, 60 to 65; 360 MB 92 to 101, 83 to 92, 77 to 83.  From there
+// part over mid: rows that are no whole waves 0.93 to 1.00 at every size, most
+// 0.96 to 0.98; whole waves 0.94 to 0.99 to 450 MB, 0.99 to 1.03 at 550 to 800 MB
+// (256^3 184 mid, 188 part), 0.98 to 1.00 at 900 MB, 0.95 to 0.98 past 1 GB.  All
+// but the loads of E past the cache (far) takes 0 to 4 % longer than part past
+// 1 GB.
+inline int cell_form(int nx, size_t state, size_t esz)
 {
     if (state <= 220000000) return kCellNear;
-    if (esz == 2) return state <= 400000000 ? kCellPart : state <= 1000000000 ? kCellMid : kCellFar;
+    if (esz == 2) {
+        if (state <= 275000000) return kCellMid;
+        return nx % 64 == 0 && state > 500000000 && state <= 850000000 ? kCellMid : kCellPart;
+    }
     return state <= 360000000 ? kCellMid : kCellFar;
 }
 // log2 of the lanes of its tiles along x: 64, or 32.  Near: 32 where 64 leave

@@ -101,6 +101,39 @@ def test_state_limits(tmp_path):
     assert [int(v) for v in out] == [want for _, want in LIMITS]
 
 
+FORM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "fdtd_internal.h"
+int main(int argc, char **argv)
+{
+    for (int q = 1; q + 3 < argc; q += 4) {   // nx ny nz esz
+        const int nx = atoi(argv[q]), ny = atoi(argv[q + 1]), nz = atoi(argv[q + 2]), esz = atoi(argv[q + 3]);
+        const size_t state = 24 * (size_t)fused_pitch(nx, esz) * ny * nz * esz;
+        const int form = cell_form(nx, state, esz), l = cell_lanes_log2(nx, form, esz);
+        printf("%d %d %d %d\n", state <= cell_state_limit(nx, esz) ? 1 : 0, form, l, cell_block_lanes(form, esz, l));
+    }
+    return 0;
+}
+"""
+
+# (shape, bytes of a value) -> form (0 near, 1 mid, 2 part, 3 far), log2 of a tile's lanes along x, lanes of a block.
+# Every combination that the dispatch has; tests/test_gpu_cell_forms.py steps these grids.
+FORMS = [((100, 30, 20), 4, (0, 6, 64)), ((90, 30, 20), 4, (0, 5, 64)), ((65, 90, 420), 4, (1, 5, 64)), ((64, 90, 530), 4, (1, 6, 64)),
+         ((70, 91, 620), 4, (3, 5, 64)), ((64, 64, 1300), 4, (3, 6, 256)), ((120, 65, 600), 4, (3, 6, 256)),
+         ((100, 30, 20), 2, (0, 6, 64)), ((90, 30, 20), 2, (0, 5, 64)), ((64, 90, 900), 2, (1, 6, 64)), ((100, 121, 330), 2, (1, 6, 64)),
+         ((64, 128, 1300), 2, (1, 6, 64)), ((100, 121, 900), 2, (2, 6, 64)), ((64, 91, 1100), 2, (2, 6, 64))]
+
+
+def test_forms_and_lanes(tmp_path):
+    exe = _build(tmp_path, FORM)
+    args = [str(v) for shape, esz, _ in FORMS for v in (*shape, esz)]
+    out = subprocess.run([str(exe), *args], capture_output=True, text=True, check=True).stdout.split()
+    got = np.asarray([int(v) for v in out]).reshape(-1, 4)
+    for (shape, esz, want), (cells, *form) in zip(FORMS, got):
+        assert cells == 1 and tuple(form) == want, (shape, esz, form)
+
+
 MASK = r"""
 #include <cstring>
 #include "fdtd_internal.h"

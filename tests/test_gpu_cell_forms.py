@@ -197,3 +197,28 @@ def test_zero_terms_of_high_material_ids(first):
             out.append([ctx.get(f) for f in range(9)])
     for f, (a, b) in enumerate(zip(*out)):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), F.FIELDS[f]
+
+
+def _forms():
+    from tests.test_cell_tiles import FORMS
+    for q, (shape, esz, _) in enumerate(FORMS):
+        yield shape, (F.STORE_F32, F.STORE_F32, F.STORE_F32_FAST)[q % 3] if esz == 4 else (F.STORE_F16, F.STORE_BF16)[q % 2]
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("shape,storage", list(_forms()))
+def test_every_form_equals_tiles(shape, storage):
+    """Each form and tile width of the one-lane-per-cell step (which of them a
+    grid takes is pinned in test_cell_tiles.py) against the tiled step."""
+    from tests.test_gpu_cell import _run
+    from tests.helpers import bits_equal, first_diff
+    for tile_y in (0, 4):
+        with F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0), storage=storage, tile_y=tile_y) as ctx:
+            assert ctx.by_cells() == (tile_y == 0)
+    print(f"\n{shape} storage {storage}", flush=True)
+    a, pa = _run(shape, storage, 4, False)
+    b, pb = _run(shape, storage, 4, True)
+    for key in a:
+        assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
+    assert np.array_equal(pa.view(np.uint64), pb.view(np.uint64))
+    assert np.isfinite(pa).all() and np.abs(pa).max() > 0
