@@ -50,7 +50,7 @@ constexpr int kCellRunSteps = 64;
 
 // Byte layout of one grid's arena region.
 struct Layout {
-    size_t N, Np, esz, skew;       // cells, elements per field array, bytes per element, array stagger
+    size_t N, Np, esz, skew;       // cells, elements per field array, bytes per element, room for the arrays' stagger
     int pitch;
     long long plane;
     long long guard;
@@ -66,14 +66,14 @@ Layout layout_of(int nx, int ny, int nz, int storage, int nmat, int jz_n, int np
     L.pitch = fused_pitch(nx, L.esz);
     L.plane = (long long)L.pitch * ny;
     L.Np = (size_t)L.plane * nz;
-    // Channel stagger between the 24 field arrays of large grids (as in a
-    // single context); small grids are not worth the memory.
-    L.skew = L.Np >= (size_t)1 << 20 ? 1088 : 0;
+    // Channel stagger between the 24 field arrays of large grids: room for the
+    // larger one, of grids in tiles (place_fields); small grids are not worth the memory.
+    L.skew = L.Np >= (size_t)1 << 20 ? kTileSkew : 0;
     L.guard = fused_guard(L.pitch, L.plane);
     L.jz_n = jz_n;
     size_t o = 0;
     L.blob = o;
-    L.blob_bytes = (24 * (L.Np + L.skew) + 2 * (size_t)L.guard) * L.esz;
+    L.blob_bytes = (24 * L.Np + 23 * L.skew + 2 * (size_t)L.guard) * L.esz;
     o = round_up(o + L.blob_bytes, 256);
     L.ids = o;
     o = round_up(o + L.Np + 2 * (size_t)L.guard, 256);
@@ -246,6 +246,36 @@ bool is_running(const fdtd_batch *b, int s)
 bool cell_grid(const fdtd_batch *b, const fdtd_batch::Inst &I)
 {
     return b->by_cell && I.d.nz <= kCellMaxPlanes && 24 * I.L.Np * I.L.esz <= cell_state_limit(I.d.nx, I.L.esz);
+}
+
+// The addresses of a grid's field arrays, staggered for the kernel that steps it.
+void place_fields(fdtd_batch *b, fdtd_batch::Inst &I)
+{
+    const size_t gb = (size_t)I.L.guard * I.L.esz;
+    const size_t stride = (I.L.Np + (cell_grid(b, I) ? std::min(I.L.skew, kCellSkew) : I.L.skew)) * I.L.esz;
+    char *p = b->arena_base + I.off + I.L.blob + gb;
+    for (auto &s : I.d.E)
+        for (void *&q : s) { q = p; p += stride; }
+    for (auto &s : I.d.D)
+        for (void *&q : s) { q = p; p += stride; }
+    for (auto &s : I.d.H)
+        for (void *&q : s) { q = p; p += stride; }
+    for (int s = 0; s < 3; s++)
+        for (int q = 0; q < 3; q++) {
+            I.c.E[s][q] = (char *)I.d.E[s][q] - gb;
+            I.c.D[s][q] = (char *)I.d.D[s][q] - gb;
+            if (s < 2) I.c.H[s][q] = (char *)I.d.H[s][q] - gb;
+        }
+}
+
+// How the batch steps grids that may step by cells.  Grids that have not
+// stepped (all their fields are zero) take the stagger that goes with it.
+void set_by_cell(fdtd_batch *b, bool on)
+{
+    b->by_cell = on;
+    for (auto &I : b->in)
+        if (I.used && I.start == b->step) place_fields(b, I);
+    b->dirty = true;
 }
 
 // Groups of the grids `cell` whose state fits kCellGroupBytes together (a grid
@@ -571,14 +601,6 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
 
     BatchInst &d = I.d;
     memset(&d, 0, sizeof d);
-    char *blob = base + L.blob + (size_t)L.guard * L.esz;
-    const size_t stride = (L.Np + L.skew) * L.esz;
-    for (int s = 0; s < 3; s++)
-        for (int q = 0; q < 3; q++) d.E[s][q] = blob + (size_t)(s * 3 + q) * stride;
-    for (int s = 0; s < 3; s++)
-        for (int q = 0; q < 3; q++) d.D[s][q] = blob + (size_t)(9 + s * 3 + q) * stride;
-    for (int s = 0; s < 2; s++)
-        for (int q = 0; q < 3; q++) d.H[s][q] = blob + (size_t)(18 + s * 3 + q) * stride;
     d.ids = (const uint8_t *)(base + L.ids + L.guard);
     d.lut = (const MatCoef *)(base + L.lut);
     d.jz = (const float *)(base + L.jz);
@@ -607,13 +629,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     d.zskip = (e.storage == FDTD_STORE_F32 && e.load_zero_terms == 0) ? 1 : 0;
     CellInst &c = I.c;
     memset(&c, 0, sizeof c);
-    const size_t gb = (size_t)L.guard * L.esz;
-    for (int s = 0; s < 3; s++)
-        for (int q = 0; q < 3; q++) {
-            c.E[s][q] = (char *)d.E[s][q] - gb;
-            c.D[s][q] = (char *)d.D[s][q] - gb;
-            if (s < 2) c.H[s][q] = (char *)d.H[s][q] - gb;
-        }
+    place_fields(b, I);   // (reads d.nx, d.nz)
     c.ids = d.ids - L.guard;
     c.lut = d.lut;
     c.jz = d.jz;
@@ -624,7 +640,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.probe_out = d.probe_out;
     for (int f = 0; f < 9; f++) c.factor[f] = d.factor[f];
     c.nx = nx; c.ny = ny; c.nz = nz;
-    c.o0 = (uint32_t)gb;
+    c.o0 = (uint32_t)((size_t)L.guard * L.esz);
     c.sy = (uint32_t)(L.pitch * L.esz);
     c.sz = (uint32_t)(L.plane * L.esz);
     cell_tiles(nx, ny, cell_form(nx, 24 * L.Np * L.esz, L.esz), L.esz, c);
@@ -767,7 +783,7 @@ extern "C" int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int g
     if (kchunk < 0 || graph_steps < 0) return fdtd_fail(FDTD_EINVAL, "negative kchunk/graph_steps");
     if (tile_y) b->ty = tile_y;
     if (kchunk) b->kchunk = kchunk;
-    if (tile_y || kchunk) b->by_cell = false;
+    if (tile_y || kchunk) set_by_cell(b, false);
     if (graph_steps) b->graph_steps = graph_steps;
     b->dirty = true;
     return 0;
@@ -802,7 +818,7 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
     float best = 0.0f;
     int bty = b->ty, bkc = b->kchunk;
     const bool by_cell0 = b->by_cell;
-    b->by_cell = true;
+    b->by_cell = true;   // (for cell_grid)
     const bool any_cell = std::any_of(b->in.begin(), b->in.end(),
                                       [&](const fdtd_batch::Inst &I) { return I.used && cell_grid(b, I); });
     auto trial = [&](int n) -> float {   // ms per step over n steps as the batch is set up now
@@ -818,7 +834,18 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
         if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune timing");
         return ms / n;
     };
-    b->by_cell = false;
+    auto zero_fields = [&]() {   // and probe rows of every grid
+        for (auto &I : b->in) {
+            if (!I.used) continue;
+            char *base = b->arena_base + I.off;
+            e = hipMemsetAsync(base + I.L.blob, 0, I.L.blob_bytes, b->up);
+            if (e == hipSuccess) e = hipMemsetAsync(base + I.L.out, 0, I.L.out_bytes, b->up);
+            if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune reset");
+        }
+        e = hipStreamSynchronize(b->up);
+        if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune reset");
+    };
+    set_by_cell(b, false);
     for (int a = 0; a < 3 && !rc; a++)
         for (int c = 0; c < 5 && !rc; c++) {
             b->ty = tys[a];
@@ -833,13 +860,17 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
     // The groups, if a grid may step in one; without one (or after an error) the choice stays, for the grids to come.
     bool bcells = by_cell0;
     if (!rc && any_cell) {
-        b->by_cell = true;
+        e = hipStreamSynchronize(stream);
+        if (e != hipSuccess) rc = fdtd_hip_fail(e, "autotune");
+        zero_fields();
+        for (auto &I : b->in)
+            if (I.used) I.start = I.d.start = (int)b->step;
+        set_by_cell(b, true);
         b->ty = bty;
         b->kchunk = bkc;
-        const float ms = trial(std::max(trial_steps, kCellRunSteps));   // each group's steps in a row, as a run takes them
+        const float ms = rc ? 0.0f : trial(std::max(trial_steps, kCellRunSteps));   // each group's steps in a row, as a run takes them
         if (!rc) bcells = ms < best;
     }
-    b->by_cell = bcells;
     if (t0) (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);
     // Back to the zero initial state at step0 with the fastest shape.
@@ -849,14 +880,11 @@ extern "C" int fdtd_batch_autotune(fdtd_batch *b, int trial_steps, hipStream_t s
         auto &I = b->in[s];
         if (!I.used) continue;
         I.steps = I.d.nsteps = saved[s];
-        char *base = b->arena_base + I.off;
-        e = hipMemsetAsync(base + I.L.blob, 0, I.L.blob_bytes, b->up);
-        if (e == hipSuccess) e = hipMemsetAsync(base + I.L.out, 0, I.L.out_bytes, b->up);
-        if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune reset");
+        I.start = I.d.start = (int)step0;
     }
-    e = hipStreamSynchronize(b->up);
-    if (!rc && e != hipSuccess) rc = fdtd_hip_fail(e, "autotune reset");
+    zero_fields();
     b->step = step0;
+    set_by_cell(b, bcells);
     b->ty = bty;
     b->kchunk = bkc;
     b->dirty = true;

@@ -20,13 +20,6 @@
 
 namespace {
 
-// Extra elements between consecutive field arrays in the blob: staggers the
-// arrays' starts across HBM channels, also where a plane is a power of two
-// (256^3 fp32 by cells, us a step: 327 with 0, 1024 or 65536, 280 to 285 with
-// 64, 4160 or 1088; 320x320x880 in tiles 1553 with 65536, 1534 with 1088 or
-// 66624; 300x250x220 in tiles 307 with 1088, 298 with 66624).
-constexpr size_t kCellSkew = 1088, kTileSkew = 66624;
-
 }  // namespace
 
 struct fdtd_ctx {

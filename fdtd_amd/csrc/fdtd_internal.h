@@ -157,6 +157,13 @@ inline int fused_pitch(int nx, size_t esz)
 // Guard (in elements) the fused kernel needs around every field array and
 // the id array so that its halo loads need no bounds checks: one plane, ten
 // rows and 256 elements (tiles are at most 8 rows high and 128 cells wide).
+// Extra elements between consecutive field arrays: staggers the arrays' starts
+// across HBM channels, also where a plane is a power of two (256^3 fp32 by cells,
+// us a step: 327 with 0, 1024 or 65536, 280 to 285 with 64, 4160 or 1088).  Tiles,
+// 1088 against 65536 and 66624: 128^3 48.6, 46.3, 45.9; 223x190x170 141, 139, 138;
+// 300x250x220 304, 295, 295; 290x310x300 511, 506, 503; 320x320x880 1512, 1530,
+// 1509; but 192^3 127, 130, 130 and 256^3 287, 295, 293.
+constexpr size_t kCellSkew = 1088, kTileSkew = 66624;
 inline long long fused_guard(int pitch, long long plane) { return plane + 10LL * pitch + 256; }
 
 // Arguments of the 6-face first-order Mur kernel (fdtd_calculations.cu:216-428).

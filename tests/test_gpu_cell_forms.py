@@ -222,3 +222,31 @@ def test_every_form_equals_tiles(shape, storage):
         assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
     assert np.array_equal(pa.view(np.uint64), pb.view(np.uint64))
     assert np.isfinite(pa).all() and np.abs(pa).max() > 0
+
+
+@pytest.mark.parametrize("when", ["never", "before", "after", "late", "autotune"])
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+def test_batch_shape_fixed_at_any_time(when):
+    """A batch staggers a grid's arrays for the kernel that steps it; a grid that
+    has not stepped follows a later choice, one that has keeps its place."""
+    from tests.test_gpu_batch import assert_same, make_case, single
+    insts = [make_case(620, (96, 110, 110), 5, 21), make_case(621, (100, 128, 90), 4, 18, F.STORE_F16), make_case(622, (30, 20, 25), 4, 25)]
+    refs = [single(x) for x in insts]
+    print(f"\nshape fixed {when}", flush=True)
+    with F.Batch(1 << 30) as b:
+        if when == "before":
+            b.set_shape(tile_y=4, kchunk=8)
+        ids = [b.add(x) for x in insts[:2]]
+        if when == "after":
+            b.set_shape(tile_y=2, kchunk=6)
+        if when == "autotune":
+            b.autotune(trial_steps=1)
+        b.run(7)
+        ids.append(b.add(insts[2]))
+        if when == "late":
+            b.set_shape(tile_y=8, kchunk=4)
+        if when != "autotune":
+            assert [b.by_cells(i) for i in ids] == [when == "never"] * 3
+        b.run(30)
+        for q, (i, x) in enumerate(zip(ids, insts)):
+            assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
