@@ -250,3 +250,15 @@ def test_batch_shape_fixed_at_any_time(when):
         b.run(30)
         for q, (i, x) in enumerate(zip(ids, insts)):
             assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
+
+
+def test_comparisons_with_tiles_have_two_kernels_to_compare():
+    """The grids of test_gpu_cell.py step by cells by default and in tiles with
+    tile_y fixed, in every storage form."""
+    from tests import test_gpu_cell as T
+    past = [m.args[1] for m in T.test_cells_equal_tiles_past_the_cache.pytestmark if m.name == "parametrize"][0]
+    both = [(s, st) for s in T.SHAPES for st in (F.STORE_F32, F.STORE_F16, F.STORE_BF16, F.STORE_F32_FAST)] + past
+    for shape, storage in both:
+        for tile_y in (0, 4):
+            with F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0), storage=storage, tile_y=tile_y) as ctx:
+                assert ctx.by_cells() == (tile_y == 0), (shape, storage)
