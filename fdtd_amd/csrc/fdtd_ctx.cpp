@@ -1164,7 +1164,7 @@ extern "C" int fdtd_ctx_autotune(fdtd_ctx *c, int trial_steps, hipStream_t strea
     const int nform = c->esz == 2 ? 3 : 2;
     float best = 0.0f;
     int bty = c->ty, bkc = c->kchunk, bcpl = c->cpl, btxw = c->txw;
-    bool bcell = false;
+    bool bcell = c->cell;   // stays where cells cannot be timed, or after an error
     auto trial = [&]() -> float {   // ms of the trial steps as the context is set up now
         rc = fdtd_run(c, 2, stream);
         if (rc) return 0.0f;
@@ -1192,10 +1192,10 @@ extern "C" int fdtd_ctx_autotune(fdtd_ctx *c, int trial_steps, hipStream_t strea
                     btxw = w;
                 }
             }
-    if (!rc && c->ext.time_steps != 2 && c->nz <= kCellMaxPlanes) {
+    if (!rc && c->ext.time_steps != 2 && c->nz <= kCellMaxPlanes && c->nprobe <= kCellMaxProbes) {
         c->cell = true;
         const float ms = trial();
-        bcell = !rc && ms < best;
+        if (!rc) bcell = ms < best;
     }
     if (t0) (void)hipEventDestroy(t0);
     if (t1) (void)hipEventDestroy(t1);

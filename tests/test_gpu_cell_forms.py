@@ -262,3 +262,17 @@ def test_comparisons_with_tiles_have_two_kernels_to_compare():
         for tile_y in (0, 4):
             with F.Context(F.make_params(shape, DT, DX, mu0=MU0, eps0=EPS0), storage=storage, tile_y=tile_y) as ctx:
                 assert ctx.by_cells() == (tile_y == 0), (shape, storage)
+
+
+@pytest.mark.parametrize("tile_y", [0, 4])
+def test_autotune_that_cannot_time_cells_keeps_the_choice(tile_y):
+    """With more probes than the step by cells takes there is only one kernel to
+    time; the choice is the context's own again once it has fewer."""
+    with F.Context(F.make_params((20, 18, 16), DT, DX, mu0=MU0, eps0=EPS0), tile_y=tile_y) as ctx:
+        for _ in range(3):
+            ctx.set_probes(np.zeros((40001, 4), np.int32), 1)
+            assert not ctx.by_cells()
+            print(f"\nautotune with 40001 probes, tile_y {tile_y}", flush=True)
+            ctx.autotune(trial_steps=1)
+            ctx.set_probes(np.zeros((1, 4), np.int32), 1)
+            assert ctx.by_cells() == (tile_y == 0)
