@@ -20,10 +20,10 @@ OpenMP on this host's cores, on a bounded sample of the same workload).
 Exits with status 3 when the probes saw no finite non-zero signal.
 
 Two more workloads measure the systems patterns:
-  --workload batched  64 uneven grids (batched_set) stepped together, one
-                      persistent fused launch per step from captured graphs,
-                      shape picked by the autotuner (or fixed by --shape
-                      64xTYxKC); whole-job Gcell-updates/s
+  --workload batched  64 uneven grids (batched_set) stepped together, by cells
+                      in groups or in one persistent fused launch per step from
+                      captured graphs, as the autotuner picks (or in tiles fixed
+                      by --shape 64xTYxKC); whole-job Gcell-updates/s
                       beside running the same grids one after another.
   --workload riken    the RIKEN voxel phantom at body scale (297x522x1719 with
                       its vacuum pad), from `--phantom` (a PGM directory or
@@ -338,7 +338,8 @@ def main():
                  else "synthetic (seeded phantom)"),
         "config": {"workload": w.name, "grid": [nx, ny, nz], "cells": cells, "materials": int(w.table.shape[0]),
                    "sources": int(w.sources.shape[0]), "probes": int(w.probes.shape[0]),
-                   "slice_every": w.slice_every, "launch": "one lane per cell" if by_cells else shape, "xcd_remap": remap, "time_steps": a.time_steps,
+                   "slice_every": w.slice_every, "launch": {"by_cells": True} if by_cells else {**shape, "by_cells": False},
+                   "xcd_remap": remap, "time_steps": a.time_steps,
                    "autotuned": tuned is not None,
                    "timed_steps": [first, first + a.steps], "untimed_advance": a.advance,
                    "parallelism": "single GPU"},
@@ -651,6 +652,8 @@ def bench_batched(a):
         ty, kc = b.autotune(trial_steps=4, stream=stream.handle)
     t_tune = time.perf_counter() - t0
     info = b.info()
+    cell_grids = sum(b.by_cells(i) for i in ids)
+    in_tiles = cell_grids < len(ids)
     steps = max(w.steps for w in ws)
     e0, e1 = hip.Event(), hip.Event()
     hip.sync()
@@ -665,17 +668,21 @@ def bench_batched(a):
     b.close()
     value = work / (ms * 1e-3) / 1e9
     out = {
-        "metric": "Gcell-updates/s (64 uneven grids batched: one persistent fused launch per step)",
+        "metric": "Gcell-updates/s (64 uneven grids batched)",
         "value": round(value, 3), "unit": "Gcell-updates/s", "n_gpus": 1, "steps": steps, "warmup": 0,
         "ms_per_step": round(ms / steps, 5), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32 (f64 Debye sums)" if a.storage == "f32" else f"{a.storage} storage, f32 arithmetic",
         "data": "synthetic (seeded phantoms)",
         "config": {"workload": "batched_set", "grids": len(ws), "cells": cells, "cell_updates": work,
-                   "steps_range": [min(w.steps for w in ws), steps], "tile_y": ty, "kchunk": kc,
-                   "graph_steps": a.segment, "persistent_grid": info["grid"][0], "parallelism": "single GPU"},
+                   "steps_range": [min(w.steps for w in ws), steps], "grids_by_cells": cell_grids,
+                   "tile_y": ty if in_tiles else None, "kchunk": kc if in_tiles else None,
+                   "graph_steps": a.segment,
+                   "persistent_grid": info["grid"][0] if in_tiles else None, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(97 * work / (ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(97 * work / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                     "traffic": None, "kernel": "whole batch step (fused_batch + mur_batch with probe rows)",
+                     "traffic": None,
+                     "kernel": "whole batch step (" + " and ".join(
+                         ["cell_batch"] * (cell_grids > 0) + ["fused_batch + mur_batch with probe rows"] * in_tiles) + ")",
                      "bytes_per_cell": 97},
         "upload_s": round(t_upload, 3), "autotune_s": round(t_tune, 3), "all_finished": ok,
     }

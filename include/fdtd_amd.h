@@ -247,8 +247,10 @@ int fdtd_ctx_by_cells(fdtd_ctx *ctx);
 int fdtd_default_launch_shape(const FdtdParams *p, const FdtdExt *ext, int cus, int *tile_x, int *tile_y,
                               int *kchunk, int *lane_cells);
 
-/* Times every `every`-th fused-kernel launch (the first, then each `every`
- * launches; every >= 1), up to `capacity` of them (capacity 0 disables):
+/* Times every `every`-th launch of the step's kernel (the first, then each
+ * `every` launches; every >= 1), up to `capacity` of them (capacity 0
+ * disables).  In tiles that is the fused kernel, without the Mur faces and
+ * the probe row of its step; by cells (fdtd_ctx_by_cells) it is the whole step:
  * a HIP event pair bound to the launch's dispatch takes the kernel's own
  * start and end.  Timing every launch costs the step sequence about 1.5%,
  * so sampling keeps the timed run's wall clock close to an untimed one.

@@ -276,3 +276,19 @@ def test_autotune_that_cannot_time_cells_keeps_the_choice(tile_y):
             ctx.autotune(trial_steps=1)
             ctx.set_probes(np.zeros((1, 4), np.int32), 1)
             assert ctx.by_cells() == (tile_y == 0)
+
+
+@pytest.mark.parametrize("args,cells", [(("--shape", "64x4x8"), False), ((), True)])
+def test_bench_lines_name_the_kernels_that_ran(args, cells):
+    from tests.test_gpu_bench import _bench
+    d = _bench("--workload", "plain_small", "--steps", "8", "--warmup", "2", "--advance", "8", "--no-cpu-baseline",
+               "--timing-launches", "8", *args)
+    launch = d["config"]["launch"]
+    assert launch["by_cells"] == cells and ("tile_y" in launch) == (not cells)
+    assert d["roofline"]["kernel"] == ("cell_step" if cells else "fused_step")
+    d = _bench("--workload", "batched", "--no-sequential", *args)
+    c, kernel = d["config"], d["roofline"]["kernel"]
+    assert ("cell_batch" in kernel) == (c["grids_by_cells"] > 0) and ("fused_batch" in kernel) == (c["grids_by_cells"] < 64)
+    assert (c["tile_y"] is None) == (c["grids_by_cells"] == 64)
+    if not cells:
+        assert c["grids_by_cells"] == 0 and (c["tile_y"], c["kchunk"]) == (4, 8)
