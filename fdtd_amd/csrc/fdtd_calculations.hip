@@ -308,7 +308,10 @@ extern "C" int updateEField(float *exTarget, float *eyTarget, float *ezTarget, f
 {
     if (!h_params_set) return FDTD_ESTATE;
     (wide() ? legacy_e<size_t, true> : streaming() ? legacy_e<uint32_t, true> : legacy_e<uint32_t, false>)
-        <<<flat_grid(), kBlock, 0, stream>>>(exTarget, eyTarget, ezTarget, exSource0, eySource0, ezSource0, exSource1, eySource1, ezSource1, dxSource0, dySource0, dzSource0, dxSource1, dySource1, dzSource1, dxSource2, dySource2, dzSource2, sigma, epsI, epsS, tauD);
+        <<<flat_grid(), kBlock, 0, stream>>>(exTarget, eyTarget, ezTarget, exSource0, eySource0, ezSource0, exSource1,
+                                             eySource1, ezSource1, dxSource0, dySource0, dzSource0, dxSource1,
+                                             dySource1, dzSource1, dxSource2, dySource2, dzSource2, sigma, epsI, epsS,
+                                             tauD);
     return set_err(hipGetLastError());
 }
 

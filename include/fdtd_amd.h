@@ -335,7 +335,8 @@ typedef struct
     int tile_y, kchunk;         /* fused launch shape */
     int graph_steps;            /* steps per captured graph */
     int grid[4];                /* persistent blocks per fused launch, per storage form (largest) */
-    int tiles[4];               /* fused tiles per step of the running grids, per storage form */
+    int tiles[4];               /* fused tiles per step of the running grids, per storage form, also
+                                 * of grids that step by cells (fdtd_batch_by_cells) */
     long long cells[4];         /* cells of the running grids, per storage form */
 } FdtdBatchInfo;
 
