@@ -26,6 +26,8 @@ private:
     std::map<size_t, size_t> free_;  // offset -> length
 };
 
+// Arena bytes fdtd_batch_add takes for the grid in this batch.
+int batch_instance_bytes(fdtd_batch *b, const FdtdParams *p, const FdtdExt *ext, const FdtdInstance *inst, size_t *bytes);
 size_t batch_largest_free(fdtd_batch *b);
 size_t batch_used_bytes(fdtd_batch *b);
 long long batch_step(fdtd_batch *b);

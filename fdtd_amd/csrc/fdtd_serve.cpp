@@ -360,7 +360,7 @@ extern "C" int fdtd_serve_submit(fdtd_serve *s, const FdtdParams *p, const FdtdE
 {
     if (!s || !p || !in || !request) return fdtd_fail(FDTD_EINVAL, "null argument");
     size_t bytes = 0;
-    if (int rc = fdtd_batch_instance_bytes(p, ext, in, &bytes)) return rc;
+    if (int rc = batch_instance_bytes(s->b, p, ext, in, &bytes)) return rc;
     if (bytes > s->cfg.hbm_bytes) return fdtd_fail(FDTD_ENOMEM, "request needs %zu bytes; budget %zu", bytes, s->cfg.hbm_bytes);
     auto r = std::make_unique<Request>();
     r->p = *p;

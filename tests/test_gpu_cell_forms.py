@@ -292,3 +292,19 @@ def test_bench_lines_name_the_kernels_that_ran(args, cells):
     assert (c["tile_y"] is None) == (c["grids_by_cells"] == 64)
     if not cells:
         assert c["grids_by_cells"] == 0 and (c["tile_y"], c["kchunk"]) == (4, 8)
+
+
+def test_batch_bytes_of_a_grid():
+    """Grids by cells lie close together in the arena (their groups have to fit
+    the Infinity Cache); instance_bytes holds for either way of stepping."""
+    from tests.test_gpu_batch import make_case
+    x = make_case(630, (96, 110, 110), 5, 3)
+    for fixed in (False, True):
+        with F.Batch(x.nbytes() * 2) as b:
+            if fixed:
+                b.set_shape(tile_y=4, kchunk=8)
+            b.add(x)
+            used = b.info()["used_bytes"]
+            assert used == x.nbytes() if fixed else used + 23 * 65000 * 4 < x.nbytes()
+            b.add(x)
+            b.run(3)
