@@ -19,7 +19,7 @@
 //     still on their way from HBM, and hold up the vector cache.  The values
 //     past a row's ends come through the scalar cache;
 //   * part (16 bits): and D streams past the Infinity Cache, which holds E and H;
-//   * far (fp32): and so do E^{n-1} and the stores of E; H and E^n stay for longer.
+//   * far: and so do E^{n-1} and the stores of E; H and E^n stay for longer.
 // Every other step takes the planes from the highest down (flip): it starts
 // on those that the last step left in the cache.
 //
@@ -600,10 +600,10 @@ template <typename T, bool EXACT>
 hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
 {
     if (!cell_args_ok(c)) return hipErrorInvalidValue;
-    constexpr int kPast = sizeof(T) == 2 ? kCellPart : kCellFar;   // cell_form
-    const void *k = c.form == kCellNear ? (const void *)cell_step<T, EXACT, 6, kCellNear>
-                    : c.form == kCellMid ? (const void *)cell_step<T, EXACT, 6, kCellMid>
-                                         : (const void *)cell_step<T, EXACT, 6, kPast>;
+    constexpr int kPart = sizeof(T) == 2 ? kCellPart : kCellFar;   // 16 bits only
+    const void *wide[] = {(const void *)cell_step<T, EXACT, 6, kCellNear>, (const void *)cell_step<T, EXACT, 6, kCellMid>,
+                          (const void *)cell_step<T, EXACT, 6, kPart>, (const void *)cell_step<T, EXACT, 6, kCellFar>};
+    const void *k = wide[c.form];
     if (c.bxl == 5) {   // cell_lanes_log2, cell_form: fp32 near, mid and far, 16 bits near
         k = (const void *)cell_step<T, EXACT, 5, kCellNear>;
         if constexpr (sizeof(T) == 4) {
@@ -662,11 +662,12 @@ static hipError_t launch_cell_batch_t(const CellInst *inst, const CellGroups *gr
                                       int step, int form, int lanes, hipStream_t s)
 {
     const dim3 grid((unsigned)blocks), block((unsigned)lanes);
-    constexpr int kPast = sizeof(T) == 2 ? kCellPart : kCellFar;   // cell_form
+    constexpr int kPart = sizeof(T) == 2 ? kCellPart : kCellFar;   // 16 bits only
     switch (form) {
     case kCellNear: cell_batch<T, EXACT, kCellNear><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
     case kCellMid: cell_batch<T, EXACT, kCellMid><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
-    default: cell_batch<T, EXACT, kPast><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    case kCellPart: cell_batch<T, EXACT, kPart><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
+    default: cell_batch<T, EXACT, kCellFar><<<grid, block, 0, s>>>(inst, groups, first, count, step); break;
     }
     return hipGetLastError();
 }

@@ -220,8 +220,8 @@ struct ZeroTerms {
 // probe row (fdtd_cell.hip).  The field and id pointers lie fused_guard
 // elements before the arrays' origins; o0 = the guard in bytes.
 // Forms of cell_step: its state in the Infinity Cache; x neighbours from the
-// lanes beside instead of loads; the same with D past the cache (16 bits); with
-// D and all but the loads of E^n past it (fp32).
+// lanes beside instead of loads; the same with D past the cache (16 bits only);
+// with D and all but the loads of E^n past it.
 enum { kCellNear, kCellMid, kCellPart, kCellFar };
 struct CellArgs {
     const char *e0[3], *e1[3], *d0[3], *d1[3], *h0[3];   // E, D at levels n and n-1, H^{n-1/2}
@@ -283,14 +283,15 @@ inline size_t cell_state_limit(int nx, size_t esz)
 // 63 to 71, 59 to 67, 60 to 65; 360 MB 92 to 101, 83 to 92, 77 to 83.  From there
 // part over mid: rows that are no whole waves 0.93 to 1.00 at every size, most
 // 0.96 to 0.98; whole waves 0.94 to 0.99 to 450 MB, 0.99 to 1.03 at 550 to 800 MB
-// (256^3 184 mid, 188 part), 0.98 to 1.00 at 900 MB, 0.95 to 0.98 past 1 GB.  All
-// but the loads of E past the cache (far) takes 0 to 4 % longer than part past
-// 1 GB.
+// (256^3 184 mid, 188 part), 0.98 to 1.00 at 900 MB, 0.95 to 0.98 past 1 GB.  far
+// over part from 1.1 to 5.8 GB: rows of 64 and 100 cells 1.02 to 1.04, 160 to 256
+// 0.99 to 1.03, 300 to 384 0.98 to 1.01 (most below 1), 417 to 777 0.97 to 0.99.
 inline int cell_form(int nx, size_t state, size_t esz)
 {
     if (state <= 220000000) return kCellNear;
     if (esz == 2) {
         if (state <= 275000000) return kCellMid;
+        if (state > 1000000000 && nx > 256) return kCellFar;
         return nx % 64 == 0 && state > 500000000 && state <= 850000000 ? kCellMid : kCellPart;
     }
     return state <= 360000000 ? kCellMid : kCellFar;

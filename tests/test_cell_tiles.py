@@ -122,7 +122,8 @@ int main(int argc, char **argv)
 FORMS = [((100, 30, 20), 4, (0, 6, 64)), ((90, 30, 20), 4, (0, 5, 64)), ((65, 90, 420), 4, (1, 5, 64)), ((64, 90, 530), 4, (1, 6, 64)),
          ((70, 91, 620), 4, (3, 5, 64)), ((64, 64, 1300), 4, (3, 6, 256)), ((120, 65, 600), 4, (3, 6, 256)),
          ((100, 30, 20), 2, (0, 6, 64)), ((90, 30, 20), 2, (0, 5, 64)), ((64, 90, 900), 2, (1, 6, 64)), ((100, 121, 330), 2, (1, 6, 64)),
-         ((64, 128, 1300), 2, (1, 6, 64)), ((100, 121, 900), 2, (2, 6, 64)), ((64, 91, 1100), 2, (2, 6, 64))]
+         ((64, 128, 1300), 2, (1, 6, 64)), ((100, 121, 900), 2, (2, 6, 64)), ((64, 91, 1100), 2, (2, 6, 64)),
+         ((300, 121, 560), 2, (3, 6, 64))]
 
 
 def test_forms_and_lanes(tmp_path):
