@@ -1,5 +1,5 @@
 // Batches of independent grids (fdtd_amd.h, fdtd_batch_*): one device arena
-// holds every grid's state.  Grids that a context would step by cells are
+// holds every grid's state.  Grids that may step by cells (cell_batch_limit) are
 // stepped in groups, the small ones several to a group whose state fits the
 // Infinity Cache, one launch per group and step (cell_batch), many steps of a
 // group in a row.  The others take one persistent fused launch per
@@ -58,10 +58,10 @@ struct Layout {
     int jz_n;
 };
 
-// Whether a grid may step by cells: as a context's default_cell.
+// Whether a grid may step by cells.
 bool cell_size(int nx, int nz, size_t Np, size_t esz)
 {
-    return nz <= kCellMaxPlanes && 24 * Np * esz <= cell_state_limit(nx, esz);
+    return nz <= kCellMaxPlanes && 24 * Np * esz <= cell_batch_limit(nx, esz);
 }
 
 // by_cell: the batch steps grids by cells that may.

@@ -274,6 +274,20 @@ inline size_t cell_state_limit(int nx, size_t esz)
     if (half <= 4) return 850000000;
     return half == 6 || nx % 64 ? 1200000000 : 2450000000;
 }
+// The same of a batch's grids, whose tiles (fused_batch) take 0 to 10 % longer
+// than a context's.  fp32, their time over cell_batch's: two half waves 0.7 GB
+// 1.01, 1.0 to 1.1 GB 0.95 to 0.97; four 1.0 to 1.6 GB 1.00 to 1.04, 2.0 GB 0.99;
+// six 1.7 to 2.0 GB 1.02, 2.3 GB 1.00, 2.5 GB 0.98; 256 to 448 cells 2.2 to 2.6 GB
+// 1.01 to 1.09; an odd number 1.9 to 2.4 GB 1.04 to 1.06.
+inline size_t cell_batch_limit(int nx, size_t esz)
+{
+    if (esz == 2) return 6000000000;
+    const int half = (nx + 31) / 32;
+    if (half % 2) return 2000000000;
+    if (half == 2) return 850000000;
+    if (nx % 64) return 1200000000;
+    return half == 4 ? 1600000000 : half == 6 ? 2300000000 : 2600000000;
+}
 // Its form.  us of near, mid and far, or of near, mid and part, over rows of 64
 // to 320 cells, means over three or four placements, which differ by up to 2 %.
 // fp32: 220 MB 30 to 35, 30 to 35, 41 to 49; 270 MB 47 to 52, 44 to 50, 47 to 58;

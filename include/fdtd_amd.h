@@ -295,9 +295,10 @@ int fdtd_load_phantom_ids(const char *dir, int nx, int ny, int nz, int mode, int
 /* ---- batches of independent grids --------------------------------------
  *
  * A batch holds many grids of different sizes, materials, sources, storage
- * forms and step counts in one device arena.  Grids that a
- * context would step by cells (fdtd_ctx_by_cells) are stepped in groups, the
- * small ones several to a group whose state fits the Infinity Cache, one launch
+ * forms and step counts in one device arena.  Grids that are not too large
+ * (the sizes of fdtd_ctx_by_cells; four and six half waves to 1.6 and 2.3 GB,
+ * more whole waves to 2.6 GB) are stepped by cells in groups, the small ones
+ * several to a group whose state fits the Infinity Cache, one launch
  * per group and step; a step of the others is one persistent fused kernel per
  * storage form present, one Mur launch and one probe launch, replayed from captured graphs;
  * grids join (fdtd_batch_add) and leave (fdtd_batch_remove) between calls.
@@ -367,8 +368,7 @@ int fdtd_batch_probe_peak_units(fdtd_batch *b, int id, double *peak, int nprobe)
 int fdtd_batch_get_field(fdtd_batch *b, int id, int field, int level, float *host);
 /* tile_y in {2,4,8}, kchunk >= 1, graph_steps >= 1 (0 keeps a value).  With a
  * tile_y or kchunk every grid is stepped in tiles of that shape; otherwise
- * grids that a context would step by cells are stepped in groups (same
- * results).  Fix a shape before adding grids of 1 Mi cells and more: those that
+ * those that may are stepped by cells in groups (same results).  Fix a shape before adding grids of 1 Mi cells and more: those that
  * joined to step by cells keep their array stagger (128^3 in tiles 53 us a step
  * against 49). */
 int fdtd_batch_set_shape(fdtd_batch *b, int tile_y, int kchunk, int graph_steps);

@@ -81,24 +81,26 @@ int main(int argc, char **argv)
     for (int q = 1; q + 3 < argc; q += 4) {   // nx ny nz esz
         const int nx = atoi(argv[q]), ny = atoi(argv[q + 1]), nz = atoi(argv[q + 2]), esz = atoi(argv[q + 3]);
         const size_t state = 24 * (size_t)fused_pitch(nx, esz) * ny * nz * esz;
-        printf("%d ", state <= cell_state_limit(nx, esz) ? 1 : 0);
+        printf("%d%d ", state <= cell_state_limit(nx, esz) ? 1 : 0, state <= cell_batch_limit(nx, esz) ? 1 : 0);
     }
     return 0;
 }
 """
 
-# fp32 grids on either side of where the tiles are measured to be faster (times in cell_state_limit's comment)
-LIMITS = [((64, 64, 1300), 1), ((64, 450, 720), 0), ((128, 300, 230), 1), ((128, 450, 360), 0), ((100, 300, 310), 0),
-          ((192, 192, 192), 1), ((192, 270, 230), 1), ((192, 400, 345), 0), ((180, 300, 300), 0), ((256, 256, 256), 1),
-          ((320, 320, 224), 1), ((256, 256, 384), 1), ((384, 300, 225), 0), ((300, 200, 190), 1), ((300, 250, 220), 0),
-          ((160, 400, 300), 1), ((350, 330, 178), 1), ((350, 330, 260), 0), ((320, 320, 880), 0), ((24, 24, 24), 1)]
+# fp32 grids on either side of where a context's and a batch's tiles are measured to be faster (times in the comments of
+# cell_state_limit and cell_batch_limit): whether a context and a batch step them by cells
+LIMITS = [((64, 64, 1300), "11"), ((64, 450, 720), "00"), ((128, 300, 230), "11"), ((128, 300, 310), "01"), ((128, 450, 360), "00"),
+          ((100, 300, 310), "01"), ((100, 300, 360), "00"), ((192, 192, 192), "11"), ((192, 270, 230), "11"), ((192, 300, 300), "01"),
+          ((192, 400, 345), "00"), ((180, 300, 300), "00"), ((256, 256, 256), "11"), ((320, 320, 224), "11"), ((256, 256, 384), "11"),
+          ((384, 300, 225), "01"), ((300, 200, 190), "11"), ((300, 250, 220), "00"), ((160, 400, 300), "11"), ((350, 330, 178), "11"),
+          ((350, 330, 260), "00"), ((320, 320, 880), "00"), ((24, 24, 24), "11")]
 
 
 def test_state_limits(tmp_path):
     exe = _build(tmp_path, LIMIT)
     args = [str(v) for shape, _ in LIMITS for v in (*shape, 4)]
     out = subprocess.run([str(exe), *args], capture_output=True, text=True, check=True).stdout.split()
-    assert [int(v) for v in out] == [want for _, want in LIMITS]
+    assert out == [want for _, want in LIMITS]
 
 
 FORM = r"""
