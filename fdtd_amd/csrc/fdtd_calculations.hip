@@ -51,6 +51,21 @@ __device__ __forceinline__ int row_of(const LegacyParams &p, Q q)   // q / nx
     else return (int)(q / (Q)p.nx);
 }
 
+// The lane's cell of the flattened grid; false: past its end.
+template <typename Q>
+__device__ __forceinline__ bool flat_cell(const LegacyParams &p, Q &o, int &i, int &j, int &k)
+{
+    const Q nxy = (Q)p.nx * (Q)p.ny;
+    o = blockIdx.x * (Q)kBlock + threadIdx.x;
+    if (o >= nxy * (Q)p.nz) return false;
+    if constexpr (sizeof(Q) == 4) k = (int)div_by(o, p.nxy_mul, p.nxy_shift);
+    else k = (int)(o / nxy);
+    const Q r = o - (Q)k * nxy;
+    j = row_of(p, r);
+    i = (int)(r - (Q)j * (Q)p.nx);
+    return true;
+}
+
 // Plane pairs over blockIdx.y, in groups of kPairs over blockIdx.z (H and D).
 constexpr int kPairs = 32768;
 
@@ -154,6 +169,39 @@ __global__ __launch_bounds__(kBlock) void legacy_d(float *dxT, float *dyT, float
     }
 }
 
+// H and D where pairs of planes do not pay (use_pairs): one lane per cell of the
+// flattened grid, each component's loads where it is updated only.
+template <typename Q>
+__global__ __launch_bounds__(kBlock) void legacy_h_flat(float *hx, float *hy, float *hz, const float *ex, const float *ey,
+                                                        const float *ez)
+{
+    const LegacyParams &p = c_p;
+    Q o;
+    int i, j, k;
+    if (!flat_cell(p, o, i, j, k) || k >= p.nz - 1) return;
+    const Q sy = (Q)p.nx, sz = sy * (Q)p.ny;
+    const bool ip = i < p.nx - 1, jp = j < p.ny - 1;
+    if (i >= 1 && ip && jp) hx[o] = hx[o] - p.chy * (ez[o + sy] - ez[o]) + p.chy * (ey[o + sz] - ey[o]);
+    if (ip && j >= 1 && jp) hy[o] = hy[o] - p.chz * (ex[o + sz] - ex[o]) + p.chx * (ez[o + 1] - ez[o]);
+    if (ip && jp && k >= 1) hz[o] = hz[o] - p.chx * (ey[o + 1] - ey[o]) + p.chy * (ex[o + sy] - ex[o]);
+}
+
+template <typename Q>
+__global__ __launch_bounds__(kBlock) void legacy_d_flat(float *dxT, float *dyT, float *dzT, const float *dxS,
+                                                        const float *dyS, const float *dzS, const float *hx,
+                                                        const float *hy, const float *hz)
+{
+    const LegacyParams &p = c_p;
+    Q o;
+    int i, j, k;
+    if (!flat_cell(p, o, i, j, k) || k >= p.nz - 1) return;
+    const Q sy = (Q)p.nx, sz = sy * (Q)p.ny;
+    const bool ip = i < p.nx - 1, jp = j < p.ny - 1, i1 = i >= 1, j1 = j >= 1, k1 = k >= 1;
+    if (ip && j1 && jp && k1) dxT[o] = dxS[o] + p.cdy * (hz[o] - hz[o - sy]) - p.cdz * (hy[o] - hy[o - sz]);
+    if (i1 && ip && jp && k1) dyT[o] = dyS[o] + p.cdz * (hx[o] - hx[o - sz]) - p.cdx * (hz[o] - hz[o - 1]);
+    if (i1 && ip && j1 && jp) dzT[o] = dzS[o] + p.cdx * (hy[o] - hy[o - 1]) - p.cdy * (hx[o] - hx[o - sy]);
+}
+
 // fdtd_calculations.cu:187-213: one lane per listed source.
 __global__ void legacy_sources(float *dzT, const float *dzS, const float *hx, const float *hy, int it)
 {
@@ -192,13 +240,9 @@ __global__ __launch_bounds__(kBlock) void legacy_e(float *exT, float *eyT, float
     // one lane per cell of the flattened grid: every wave's 19 streams move whole lines whatever nx*ny is (14.6 us
     // at 100^3 with the lanes numbered from each plane's start, 13.6 so)
     const LegacyParams &p = c_p;
-    const Q nxy = (Q)p.nx * (Q)p.ny, o = blockIdx.x * (Q)kBlock + threadIdx.x;
-    if (o >= nxy * (Q)p.nz) return;
-    int k;
-    if constexpr (sizeof(Q) == 4) k = (int)div_by(o, p.nxy_mul, p.nxy_shift);
-    else k = (int)(o / nxy);
-    const Q r = o - (Q)k * nxy;
-    const int j = row_of(p, r), i = (int)(r - (Q)j * (Q)p.nx);
+    Q o;
+    int i, j, k;
+    if (!flat_cell(p, o, i, j, k)) return;
     const bool ux = i < p.nx - 1 && j >= 1 && j < p.ny - 1 && k >= 1 && k < p.nz - 1;
     const bool uyz = i >= 1 && k >= 1;
     if (!ux && !uyz) return;
@@ -274,6 +318,21 @@ static inline dim3 flat_grid()
     return dim3((unsigned)((n + kBlock - 1) / kBlock));
 }
 
+// H and D by pairs of planes, except in thin grids, where most cells lie beside a
+// face and the pairs' loads are for updates that are masked, and where the plane
+// and the planes' number leave many lanes of the pairs' blocks idle.  us of H, D
+// and E together, flat against pairs: 500x1000x2 15.3, 20.0; 500x500x4 22.3,
+// 25.5; 400x400x6 25.7, 26.4; 300x400x8 27.2, 27.3; 300x350x9 29.3, 29.0; 500x3x700
+// 26.0, 29.6; 400x5x500 25.7, 28.6; 400x7x350 28.8, 28.9; 2x500x1000 26.0, 28.5;
+// 3x500x700 37.5, 34.7; filled to 0.10 (5x5x20000) 16.6, 23.3; 0.39 (10x10x5000)
+// 17.3, 18.5; 0.63 (18x18x3000) 31.9, 33.1; 0.77 (14x14x5000) 31.4, 29.4; 100^3
+// 31.6, 28.4.
+static inline bool use_pairs()
+{
+    const long long n = (long long)h_p.nx * h_p.ny, blocks = (n + kBlock - 1) / kBlock, pairs = h_p.nz / 2 + h_p.nz % 2;
+    return h_p.nx >= 3 && h_p.ny >= 7 && h_p.nz >= 8 && (double)n * h_p.nz >= 0.65 * (2.0 * kBlock) * blocks * pairs;
+}
+
 static inline dim3 pair_grid()
 {
     const long long n = (long long)h_p.nx * h_p.ny;
@@ -286,8 +345,12 @@ extern "C" int updateHField(float *hx, float *hy, float *hz, float *exSource, fl
                             hipStream_t stream)
 {
     if (!h_params_set) return FDTD_ESTATE;
-    (wide() ? legacy_h<size_t, true> : streaming() ? legacy_h<uint32_t, true> : legacy_h<uint32_t, false>)
-        <<<pair_grid(), kBlock, 0, stream>>>(hx, hy, hz, exSource, eySource, ezSource);
+    if (use_pairs())
+        (wide() ? legacy_h<size_t, true> : streaming() ? legacy_h<uint32_t, true> : legacy_h<uint32_t, false>)
+            <<<pair_grid(), kBlock, 0, stream>>>(hx, hy, hz, exSource, eySource, ezSource);
+    else
+        (wide() ? legacy_h_flat<size_t> : legacy_h_flat<uint32_t>)
+            <<<flat_grid(), kBlock, 0, stream>>>(hx, hy, hz, exSource, eySource, ezSource);
     return set_err(hipGetLastError());
 }
 
@@ -295,8 +358,12 @@ extern "C" int updateDField(float *dxTarget, float *dyTarget, float *dzTarget, f
                             float *dzSource, float *hx, float *hy, float *hz, hipStream_t stream)
 {
     if (!h_params_set) return FDTD_ESTATE;
-    (wide() ? legacy_d<size_t, true> : streaming() ? legacy_d<uint32_t, true> : legacy_d<uint32_t, false>)
-        <<<pair_grid(), kBlock, 0, stream>>>(dxTarget, dyTarget, dzTarget, dxSource, dySource, dzSource, hx, hy, hz);
+    if (use_pairs())
+        (wide() ? legacy_d<size_t, true> : streaming() ? legacy_d<uint32_t, true> : legacy_d<uint32_t, false>)
+            <<<pair_grid(), kBlock, 0, stream>>>(dxTarget, dyTarget, dzTarget, dxSource, dySource, dzSource, hx, hy, hz);
+    else
+        (wide() ? legacy_d_flat<size_t> : legacy_d_flat<uint32_t>)
+            <<<flat_grid(), kBlock, 0, stream>>>(dxTarget, dyTarget, dzTarget, dxSource, dySource, dzSource, hx, hy, hz);
     return set_err(hipGetLastError());
 }
 

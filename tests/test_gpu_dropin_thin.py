@@ -1,0 +1,16 @@
+"""The drop-in H and D kernels on either side of the rule that sends thin grids
+past the pairs of planes: few planes, few rows or columns, planes that fill
+little of a block; and odd and even plane counts on both sides."""
+import pytest
+
+from tests import test_gpu_dropin_shapes as S
+
+pytestmark = pytest.mark.gpu
+
+FLAT = [(60, 40, 3), (60, 40, 7), (60, 3, 40), (60, 6, 21), (5, 5, 40), (18, 18, 31), (3, 80, 12), (300, 200, 4)]
+PAIRS = [(60, 47, 8), (60, 47, 9), (73, 7, 20), (3, 170, 9), (16, 16, 9), (257, 11, 11)]
+
+
+@pytest.mark.parametrize("shape", FLAT + PAIRS)
+def test_dropin_thin_and_pairs_bit_exact(shape):
+    S.test_dropin_shapes_bit_exact(shape, 4)
