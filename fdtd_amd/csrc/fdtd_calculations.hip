@@ -268,10 +268,12 @@ inline int set_err(hipError_t e) { return (int)e; }
 
 }  // namespace
 
-// Streaming operands where the 25 arrays of the reference's FdtdField exceed
-// the Infinity Cache (us per call, cached -> streaming): 160^3 (410 MB) E 63.7
-// -> 57.6; 256^3 H 122.9 -> 95.2, D 132 -> 99, E 276 -> 248.
-static inline bool streaming() { return 100LL * h_p.nx * h_p.ny * h_p.nz > (256LL << 20); }
+// Streaming operands where the 25 arrays of the reference's FdtdField are well
+// past the Infinity Cache.  us of H, D and E together, cached and streaming:
+// 140^3 (274 MB) 76, 80; 145^3 (305) 91, 100; 155^3 (372) 112, 120; 16x500x500 (400)
+// 114, 118; 500x16x500 (400) 108, 106; 160^3 (410) 113, 111; 400x32x400 (512) 150,
+// 136; 200^3 (800) 242, 209.  256^3 H 123, 95, D 132, 99, E 276, 248.
+static inline bool streaming() { return 100LL * h_p.nx * h_p.ny * h_p.nz > 400000000; }
 static inline bool wide() { return (long long)h_p.nx * h_p.ny * h_p.nz >= (1LL << 32); }
 
 extern "C" int fdtdSetDebyeMode(int mode)

@@ -14,3 +14,11 @@ PAIRS = [(60, 47, 8), (60, 47, 9), (73, 7, 20), (3, 170, 9), (16, 16, 9), (257, 
 @pytest.mark.parametrize("shape", FLAT + PAIRS)
 def test_dropin_thin_and_pairs_bit_exact(shape):
     S.test_dropin_shapes_bit_exact(shape, 4)
+
+
+@pytest.mark.parametrize("shape", [(159, 160, 159), (1010, 1000, 4)])
+def test_dropin_streaming_forms_bit_exact(shape):
+    """More than 400 MB in the reference's 25 arrays: streaming H, D and E, and
+    a thin grid with streaming E."""
+    assert 100 * shape[0] * shape[1] * shape[2] > 400_000_000
+    S.test_dropin_shapes_bit_exact(shape, 1)
