@@ -665,7 +665,7 @@ extern "C" int fdtd_batch_add(fdtd_batch *b, const FdtdParams *p, const FdtdExt 
     c.o0 = (uint32_t)((size_t)L.guard * L.esz);
     c.sy = (uint32_t)(L.pitch * L.esz);
     c.sz = (uint32_t)(L.plane * L.esz);
-    cell_tiles(nx, ny, cell_form(nx, 24 * L.Np * L.esz, L.esz), L.esz, c);
+    cell_tiles(nx, ny, nz, in->nprobe, cell_form(nx, 24 * L.Np * L.esz, L.esz), L.esz, c);
     for (int q = 0; q < 3; q++) { c.ch[q] = d.ch[q]; c.cd[q] = d.cd[q]; }
     c.zmask = d.zskip ? cell_zmask(lut.data(), in->nmat) : ZeroTerms{};
     c.nprobe = d.nprobe;

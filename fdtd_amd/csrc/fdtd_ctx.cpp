@@ -606,7 +606,7 @@ void fill_cell_args(fdtd_ctx *c, const StepArgs &a, CellArgs &q)
     q.hi_once = a.mur_x == 2;
     q.flip = c->n & 1;
     q.form = cell_form(c->nx, 24 * c->Np * c->esz, c->esz);
-    cell_tiles(c->nx, c->ny, q.form, c->esz, q);
+    cell_tiles(c->nx, c->ny, c->nz, c->nprobe, q.form, c->esz, q);
     const size_t nyz = (size_t)c->ny * c->nz, nxz = (size_t)c->nx * c->nz, nxy = (size_t)c->nx * c->ny;
     const float4 *m = c->mur;
     const size_t step[6] = {nyz, nyz, nxz, nxz, nxy, nxy};

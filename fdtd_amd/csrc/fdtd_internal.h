@@ -230,7 +230,7 @@ struct CellArgs {
     const MatCoef *lut;
     int nx, ny, nz;
     uint32_t o0, sy, sz;           // bytes: guard, row, plane
-    int tiles_x, tiles, run;       // tiles per row and per plane, ceil(tiles / 8)
+    int tiles_x, tiles, run;       // tiles per row and per plane; tiles in a row on one XCD, or 0 (cell_tiles)
     uint32_t tx_mul, tx_shift;     // div_consts(tiles_x)
     float ch[3], cd[3], jz;
     ZeroTerms zmask;               // materials whose cells do not load levels n-1
@@ -335,8 +335,14 @@ constexpr int cell_block_lanes(int form, size_t esz, int bxl)
 }
 // The tile geometry of a grid (CellArgs, CellInst) and the materials whose
 // cells skip levels n-1.
+// A plane takes 8 runs of blocks, one per XCD (cell_tile), the last ones part
+// empty.  Where that leaves a launch of many planes mostly of empty blocks it is
+// their dispatch, about one a nanosecond, that takes the time; such a plane takes
+// as many blocks as it has tiles, as they come (run = 0): us a step, 3x3x10000
+// fp32 77 -> 29, 10x10x10000 fp16 143 -> 76, 130x3x10000 fp32 187 -> 109 (in tiles
+// 38, 120, 122).
 template <typename A>
-inline void cell_tiles(int nx, int ny, int form, size_t esz, A &a)
+inline void cell_tiles(int nx, int ny, int nz, int nprobe, int form, size_t esz, A &a)
 {
     a.bxl = cell_lanes_log2(nx, form, esz);
     a.lanes = cell_block_lanes(form, esz, a.bxl);
@@ -346,7 +352,12 @@ inline void cell_tiles(int nx, int ny, int form, size_t esz, A &a)
     else a.tx_mul = a.tx_shift = 0;
     a.tiles = a.tiles_x * ((ny + by - 1) / by);
     a.run = (a.tiles + 7) / 8;
+    const long long rows = nz + ((long long)nprobe + a.tiles - 1) / a.tiles;   // blockIdx.y, without the runs
+    if (10LL * a.tiles < 64LL * a.run && 8LL * a.run * nz > 16384 && rows < 65536) a.run = 0;
 }
+// Blocks of a plane, and the tile of block bx of a plane.
+__host__ __device__ inline int cell_plane_blocks(int tiles, int run) { return run ? 8 * run : tiles; }
+__host__ __device__ inline int cell_tile(int bx, int run) { return run ? (bx & 7) * run + (bx >> 3) : bx; }
 // The row of tiles that tile t of a plane lies in.
 __host__ __device__ inline int cell_tile_row(int t, int tiles_x, uint32_t tx_mul, uint32_t tx_shift)
 {
@@ -598,7 +609,7 @@ struct CellGroups {
 // Blocks of a grid's step: its planes' and its probes' (one a wave).
 inline int cell_blocks(const CellInst &d)
 {
-    const int gx = 8 * d.run, w = d.lanes / 64, pb = (d.nprobe + w - 1) / w;
+    const int gx = cell_plane_blocks(d.tiles, d.run), w = d.lanes / 64, pb = (d.nprobe + w - 1) / w;
     return gx * (d.nz + (pb + gx - 1) / gx);
 }
 hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,

@@ -40,7 +40,7 @@ int main(int argc, char **argv)
     for (int q = 1; q + 3 < argc; q += 4) {   // nx ny form esz
         Tiles a;
         const int nx = atoi(argv[q]), ny = atoi(argv[q + 1]);
-        cell_tiles(nx, ny, atoi(argv[q + 2]), (size_t)atoi(argv[q + 3]), a);
+        cell_tiles(nx, ny, 3, 0, atoi(argv[q + 2]), (size_t)atoi(argv[q + 3]), a);
         long long bad = 0;
         for (int t = 0; t < a.tiles; t++) bad += cell_tile_row(t, a.tiles_x, a.tx_mul, a.tx_shift) != t / a.tiles_x;
         printf("%d %d %lld\n", a.tiles_x, a.tiles, bad);
@@ -118,6 +118,45 @@ int main(int argc, char **argv)
     return 0;
 }
 """
+
+PLANES = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "fdtd_internal.h"
+struct Tiles { int bxl, lanes, tiles_x, tiles, run; uint32_t tx_mul, tx_shift; };
+int main(int argc, char **argv)
+{
+    for (int q = 1; q + 4 < argc; q += 5) {   // nx ny nz nprobe esz
+        Tiles a;
+        const int nx = atoi(argv[q]), ny = atoi(argv[q + 1]), nz = atoi(argv[q + 2]), np = atoi(argv[q + 3]), esz = atoi(argv[q + 4]);
+        cell_tiles(nx, ny, nz, np, cell_form(nx, 24 * (size_t)fused_pitch(nx, esz) * ny * nz * esz, esz), esz, a);
+        const int gx = cell_plane_blocks(a.tiles, a.run), waves = a.lanes / 64;
+        std::vector<int> seen(a.tiles, 0);
+        for (int b = 0; b < gx; b++)
+            if (const int t = cell_tile(b, a.run); t < a.tiles) seen[t]++;
+        for (int t = 0; t < a.tiles; t++)
+            if (seen[t] != 1) return 1;
+        const int pb = (np + waves - 1) / waves;
+        if (nz + (pb + gx - 1) / gx > 65535) return 2;
+        printf("%d ", a.run == 0 ? 1 : 0);
+    }
+    return 0;
+}
+"""
+
+# (shape, probes, bytes of a value) -> whether a plane takes only as many blocks as it has tiles
+PLANE_CASES = [((3, 3, 300), 0, 4, 0), ((3, 3, 10000), 0, 4, 1), ((3, 3, 10000), 40000, 4, 1), ((3, 3, 60000), 40000, 4, 0),
+               ((64, 4, 10000), 9, 4, 1), ((130, 3, 10000), 5, 4, 1), ((16, 16, 10000), 0, 4, 0), ((10, 10, 10000), 0, 2, 1),
+               ((3, 30, 10000), 0, 4, 0), ((24, 24, 24), 0, 4, 0), ((256, 256, 256), 3, 4, 0)]
+
+
+def test_every_tile_of_a_plane_has_one_block(tmp_path):
+    exe = _build(tmp_path, PLANES)
+    args = [str(v) for shape, np_, esz, _ in PLANE_CASES for v in (*shape, np_, esz)]
+    r = subprocess.run([str(exe), *args], capture_output=True, text=True)
+    assert r.returncode == 0 and [int(v) for v in r.stdout.split()] == [want for *_, want in PLANE_CASES]
+
 
 # (shape, bytes of a value) -> form (0 near, 1 mid, 2 part, 3 far), log2 of a tile's lanes along x, lanes of a block.
 # Every combination that the dispatch has; tests/test_gpu_cell_forms.py steps these grids.

@@ -308,3 +308,33 @@ def test_batch_bytes_of_a_grid():
             assert used == x.nbytes() if fixed else used + 23 * 65000 * 4 < x.nbytes()
             b.add(x)
             b.run(3)
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+@pytest.mark.parametrize("shape,storage", [((3, 3, 4000), F.STORE_F32), ((64, 4, 5000), F.STORE_F32), ((10, 10, 5000), F.STORE_F16),
+                                           ((130, 3, 4000), F.STORE_BF16), ((130, 3, 10000), F.STORE_F32)])
+def test_many_small_planes_equal_tiles(shape, storage):
+    """Planes that take only as many blocks as they have tiles (pinned in
+    test_cell_tiles.py), with their faces and probes."""
+    from tests.test_gpu_cell import _run
+    from tests.helpers import bits_equal, first_diff
+    print(f"\nmany small planes {shape} storage {storage}", flush=True)
+    a, pa = _run(shape, storage, 4, False)
+    b, pb = _run(shape, storage, 4, True)
+    for key in a:
+        assert bits_equal(a[key], b[key]), f"{F.FIELDS[key[0]]} level {key[1]}: {first_diff(a[key], b[key])}"
+    assert np.array_equal(pa.view(np.uint64), pb.view(np.uint64))
+
+
+def test_batch_with_many_small_planes():
+    from tests.test_gpu_batch import assert_same, make_case, single
+    insts = [make_case(640, (3, 3, 5000), 4, 12), make_case(641, (30, 20, 25), 5, 12), make_case(642, (64, 4, 4000), 4, 9),
+             make_case(643, (24, 24, 24), 5, 12)]
+    refs = [single(x) for x in insts]
+    print("\nbatch with many small planes", flush=True)
+    with F.Batch(2 << 30) as b:
+        ids = [b.add(x) for x in insts]
+        assert all(b.by_cells(i) for i in ids)
+        b.run(12)
+        for q, (i, x) in enumerate(zip(ids, insts)):
+            assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
