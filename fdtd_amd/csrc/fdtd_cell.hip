@@ -166,6 +166,7 @@ struct OneStep {
     __device__ __forceinline__ int tiles_x() const { return a.tiles_x; }
     __device__ __forceinline__ int tiles() const { return a.tiles; }
     __device__ __forceinline__ int run() const { return a.run; }
+    __device__ __forceinline__ int gx() const { return a.gx; }
     __device__ __forceinline__ uint32_t tx_mul() const { return a.tx_mul; }
     __device__ __forceinline__ uint32_t tx_shift() const { return a.tx_shift; }
     __device__ __forceinline__ const uint8_t * ids() const { return a.ids; }
@@ -215,6 +216,7 @@ struct BatchStep {
     __device__ __forceinline__ int tiles_x() const { return d->tiles_x; }
     __device__ __forceinline__ int tiles() const { return d->tiles; }
     __device__ __forceinline__ int run() const { return d->run; }
+    __device__ __forceinline__ int gx() const { return d->gx; }
     __device__ __forceinline__ uint32_t tx_mul() const { return d->tx_mul; }
     __device__ __forceinline__ uint32_t tx_shift() const { return d->tx_shift; }
     __device__ __forceinline__ const uint8_t * ids() const { return d->ids; }
@@ -273,7 +275,7 @@ struct Ops {
 // cell_block_lanes are rows.  Exact form: cells whose material has a = g3 = +0 (zmask) do not
 // load E^{n-1} and D^{n-1}, as fused_tile's zero-term rows, decided per lane;
 // a grid that always loads them has an empty zmask.  C: where the step's operands
-// are (OneStep, BatchStep); block bx of the cell_plane_blocks of plane bz.
+// are (OneStep, BatchStep); block bx of the C.gx() of plane bz.
 template <typename T, bool EXACT, int BXL, int FORM, typename G>
 __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
 {
@@ -307,7 +309,7 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
         deep = jw >= 2 && jw + WY <= ny - 2 && k >= 2 && k < nz - 2 && nx > 3;
         edge = tx == 0 || (nx - 2 >= tx * BX && nx - 2 < tx * BX + BX);
     } else {
-        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * cell_plane_blocks(C.tiles(), C.run()) + bx) * (LB / 64) +
+        probe = __builtin_amdgcn_readfirstlane(((bz - nz) * C.gx() + bx) * (LB / 64) +
                                                ((int)threadIdx.x >> 6));
         if (probe >= C.nprobe()) return;
         const int *q = C.probes() + 4 * probe;
@@ -584,7 +586,7 @@ __global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), 6)) void cell_bat
     Const<CellInst> *d = (Const<CellInst> *)inst + S->idx[lo];
     const int n = step - d->start;
     if (n < 0 || n >= d->nsteps) return;
-    const int local = b - S->start[lo], gx = cell_plane_blocks(d->tiles, d->run);
+    const int local = b - S->start[lo], gx = d->gx;
     const int bz = local / gx, bx = local - bz * gx;
     const BatchStep C{d, (n + 2) % 3, (n + 1) % 3, n % 3, n & 1, n};
     if constexpr (sizeof(T) == 4 || FORM == kCellNear) {   // cell_lanes_log2
@@ -611,7 +613,7 @@ hipError_t launch_cell_t(const CellArgs &c, hipStream_t s, hipEvent_t t0, hipEve
             if (c.form == kCellFar) k = (const void *)cell_step<T, EXACT, 5, kCellFar>;
         }
     }
-    const unsigned gx = (unsigned)cell_plane_blocks(c.tiles, c.run);
+    const unsigned gx = (unsigned)c.gx;
     const unsigned waves = (unsigned)c.lanes / 64, pb = ((unsigned)c.p.nprobe + waves - 1) / waves;
     const dim3 grid(gx, (unsigned)c.nz + (pb + gx - 1) / gx);
     CellArgs arg = c;

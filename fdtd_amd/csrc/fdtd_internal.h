@@ -230,7 +230,7 @@ struct CellArgs {
     const MatCoef *lut;
     int nx, ny, nz;
     uint32_t o0, sy, sz;           // bytes: guard, row, plane
-    int tiles_x, tiles, run;       // tiles per row and per plane; tiles in a row on one XCD, or 0 (cell_tiles)
+    int tiles_x, tiles, run, gx;   // tiles per row and per plane; tiles in a row on one XCD, or 0; blocks per plane (cell_tiles)
     uint32_t tx_mul, tx_shift;     // div_consts(tiles_x)
     float ch[3], cd[3], jz;
     ZeroTerms zmask;               // materials whose cells do not load levels n-1
@@ -354,9 +354,9 @@ inline void cell_tiles(int nx, int ny, int nz, int nprobe, int form, size_t esz,
     a.run = (a.tiles + 7) / 8;
     const long long rows = nz + ((long long)nprobe + a.tiles - 1) / a.tiles;   // blockIdx.y, without the runs
     if (10LL * a.tiles < 64LL * a.run && 8LL * a.run * nz > 16384 && rows < 65536) a.run = 0;
+    a.gx = a.run ? 8 * a.run : a.tiles;
 }
-// Blocks of a plane, and the tile of block bx of a plane.
-__host__ __device__ inline int cell_plane_blocks(int tiles, int run) { return run ? 8 * run : tiles; }
+// The tile of block bx of a plane.
 __host__ __device__ inline int cell_tile(int bx, int run) { return run ? (bx & 7) * run + (bx >> 3) : bx; }
 // The row of tiles that tile t of a plane lies in.
 __host__ __device__ inline int cell_tile_row(int t, int tiles_x, uint32_t tx_mul, uint32_t tx_shift)
@@ -592,7 +592,7 @@ struct CellInst {
     double factor[9];
     int nx, ny, nz;
     uint32_t o0, sy, sz;
-    int tiles_x, tiles, run;
+    int tiles_x, tiles, run, gx;
     uint32_t tx_mul, tx_shift;
     float ch[3], cd[3];
     ZeroTerms zmask;
@@ -609,7 +609,7 @@ struct CellGroups {
 // Blocks of a grid's step: its planes' and its probes' (one a wave).
 inline int cell_blocks(const CellInst &d)
 {
-    const int gx = cell_plane_blocks(d.tiles, d.run), w = d.lanes / 64, pb = (d.nprobe + w - 1) / w;
+    const int gx = d.gx, w = d.lanes / 64, pb = (d.nprobe + w - 1) / w;
     return gx * (d.nz + (pb + gx - 1) / gx);
 }
 hipError_t launch_cell_batch(const CellInst *inst, const CellGroups *groups, int first, int count, int blocks, int step,

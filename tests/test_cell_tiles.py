@@ -34,7 +34,7 @@ PROGRAM = r"""
 #include <cstdio>
 #include <cstdlib>
 #include "fdtd_internal.h"
-struct Tiles { int bxl, lanes, tiles_x, tiles, run; uint32_t tx_mul, tx_shift; };
+struct Tiles { int bxl, lanes, tiles_x, tiles, run, gx; uint32_t tx_mul, tx_shift; };
 int main(int argc, char **argv)
 {
     for (int q = 1; q + 3 < argc; q += 4) {   // nx ny form esz
@@ -124,14 +124,14 @@ PLANES = r"""
 #include <cstdlib>
 #include <vector>
 #include "fdtd_internal.h"
-struct Tiles { int bxl, lanes, tiles_x, tiles, run; uint32_t tx_mul, tx_shift; };
+struct Tiles { int bxl, lanes, tiles_x, tiles, run, gx; uint32_t tx_mul, tx_shift; };
 int main(int argc, char **argv)
 {
     for (int q = 1; q + 4 < argc; q += 5) {   // nx ny nz nprobe esz
         Tiles a;
         const int nx = atoi(argv[q]), ny = atoi(argv[q + 1]), nz = atoi(argv[q + 2]), np = atoi(argv[q + 3]), esz = atoi(argv[q + 4]);
         cell_tiles(nx, ny, nz, np, cell_form(nx, 24 * (size_t)fused_pitch(nx, esz) * ny * nz * esz, esz), esz, a);
-        const int gx = cell_plane_blocks(a.tiles, a.run), waves = a.lanes / 64;
+        const int gx = a.gx, waves = a.lanes / 64;
         std::vector<int> seen(a.tiles, 0);
         for (int b = 0; b < gx; b++)
             if (const int t = cell_tile(b, a.run); t < a.tiles) seen[t]++;
