@@ -287,7 +287,8 @@ __device__ __forceinline__ void cell_block(const G &C, int bx, int bz)
     const int nx = C.nx(), ny = C.ny(), nz = C.nz();
 
     // Blocks (bx, k) of plane k in 8 runs of tiles, one run per XCD (workgroups
-    // go to the XCDs round-robin by id, and a plane takes a multiple of 8), so a
+    // go to the XCDs round-robin by id, and a plane takes a multiple of 8, or in
+    // grids of many small planes one block per tile: cell_tiles), so a
     // tile's neighbours in the plane and the same tiles of the planes around it
     // share its L2.  Rows past nz hold the probes.
     int i, j, k;
@@ -569,8 +570,8 @@ __global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), BXL)) void cell_s
 }
 
 // One step of a group of a batch's grids: blocks [start[q], start[q + 1]) of
-// the launch are grid q's, a multiple of 8, so that cell_block's mapping of
-// tiles to XCDs holds.  Grids outside their step window are skipped.
+// the launch are grid q's, a multiple of 8 but for grids of many small planes, so
+// that cell_block's mapping of tiles to XCDs holds.  Grids outside their step window are skipped.
 template <typename T, bool EXACT, int FORM>
 __global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), 6)) void cell_batch(const CellInst *inst, const CellGroups *groups, int first,
                                                          int count, int step)
