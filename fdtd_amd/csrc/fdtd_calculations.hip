@@ -320,19 +320,23 @@ static inline dim3 flat_grid()
     return dim3((unsigned)((n + kBlock - 1) / kBlock));
 }
 
-// H and D by pairs of planes, except in thin grids, where most cells lie beside a
-// face and the pairs' loads are for updates that are masked, and where the plane
-// and the planes' number leave many lanes of the pairs' blocks idle.  us of H, D
+// H and D by pairs of planes, except in grids whose cells all are resident at
+// once as lanes (2048 blocks on 256 CUs), where half the waves bring half the loads
+// in flight, in thin grids, where most cells lie beside a face and the pairs' loads
+// are for updates that are masked, and where the plane and the planes' number
+// leave many lanes of the pairs' blocks idle.  us of H, D
 // and E together, flat against pairs: 500x1000x2 15.3, 20.0; 500x500x4 22.3,
 // 25.5; 400x400x6 25.7, 26.4; 300x400x8 27.2, 27.3; 300x350x9 29.3, 29.0; 500x3x700
 // 26.0, 29.6; 400x5x500 25.7, 28.6; 400x7x350 28.8, 28.9; 2x500x1000 26.0, 28.5;
 // 3x500x700 37.5, 34.7; filled to 0.10 (5x5x20000) 16.6, 23.3; 0.39 (10x10x5000)
-// 17.3, 18.5; 0.63 (18x18x3000) 31.9, 33.1; 0.77 (14x14x5000) 31.4, 29.4; 100^3
-// 31.6, 28.4.
+// 17.3, 18.5; 0.63 (18x18x3000) 31.9, 33.1; 0.77 (14x14x5000) 31.4, 29.4; 66^3
+// 12.8, 14.3; 732x29x16 12.6, 14.2; 80^3 (2000 blocks) 17.3, 17.8; 82^3 (2154) 22.1,
+// 20.8; 100^3 31.6, 28.4.
 static inline bool use_pairs()
 {
     const long long n = (long long)h_p.nx * h_p.ny, blocks = (n + kBlock - 1) / kBlock, pairs = h_p.nz / 2 + h_p.nz % 2;
-    return h_p.nx >= 3 && h_p.ny >= 7 && h_p.nz >= 8 && (double)n * h_p.nz >= 0.65 * (2.0 * kBlock) * blocks * pairs;
+    return n * h_p.nz > 2048 * kBlock && h_p.nx >= 3 && h_p.ny >= 7 && h_p.nz >= 8 &&
+           (double)n * h_p.nz >= 0.65 * (2.0 * kBlock) * blocks * pairs;
 }
 
 static inline dim3 pair_grid()
