@@ -590,7 +590,7 @@ __global__ __launch_bounds__(cell_block_lanes(FORM, sizeof(T), 6)) void cell_bat
     const int local = b - S->start[lo], gx = d->gx;
     const int bz = local / gx, bx = local - bz * gx;
     const BatchStep C{d, (n + 2) % 3, (n + 1) % 3, n % 3, n & 1, n};
-    if constexpr (sizeof(T) == 4 || FORM == kCellNear) {   // cell_lanes_log2
+    if constexpr (sizeof(T) == 4 || FORM <= kCellMid) {   // cell_lanes_log2; near groups may take a step in mid
         if (d->bxl == 5) {
             cell_block<T, EXACT, 5, FORM>(C, bx, bz);
             return;

@@ -338,3 +338,22 @@ def test_batch_with_many_small_planes():
         b.run(12)
         for q, (i, x) in enumerate(zip(ids, insts)):
             assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
+
+
+@pytest.mark.filterwarnings("ignore::fdtd_amd.PrecisionWarning")
+def test_batch_a_step_at_a_time_past_the_cache():
+    """Several groups, whose state is past the Infinity Cache, a step at a time:
+    one launch for the small grids of a storage form, in the form for states
+    past the cache; with two steps at a time in groups; and a larger grid."""
+    from tests.test_gpu_batch import assert_same, make_case, single
+    insts = [make_case(650, (100, 98, 96), 4, 9), make_case(651, (96, 90, 100), 5, 6), make_case(652, (90, 100, 104), 4, 9),
+             make_case(653, (96, 110, 90), 4, 9, F.STORE_F16), make_case(654, (70, 90, 130), 4, 7, F.STORE_F16),
+             make_case(655, (130, 100, 110), 4, 8), make_case(656, (60, 100, 90), 4, 9, F.STORE_F32_FAST), make_case(657, (20, 20, 20), 4, 3, F.STORE_F16)]
+    print("\nbatch a step at a time", flush=True)
+    refs = [single(x) for x in insts]
+    with F.Batch(4 << 30) as b:
+        ids = [b.add(x) for x in insts]
+        for n in (1, 1, 2, 1, 1, 1, 2):
+            b.run(n)
+        for q, (i, x) in enumerate(zip(ids, insts)):
+            assert_same(b, i, x, refs[q], f"grid {q} {x.shape}")
